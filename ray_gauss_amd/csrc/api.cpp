@@ -49,6 +49,9 @@ struct rg_handle {
     int2* rec_id = nullptr;
     int64_t rec_cap_words = 0;
     int64_t rec_cap_rays = 0;
+    // wavefronts left to the slab stepper
+    int4* wide = nullptr;
+    int64_t wide_cap = 0;
     uint64_t tokens_issued = 0;
     struct {
         bool valid = false;
@@ -56,6 +59,7 @@ struct rg_handle {
         int gen = 0;
         int64_t num_rays = 0;
         int words = 0;
+        int rays_per_wave = 0;
     } rec_set;
     // bumped by every device (re)allocation of the handle's workspace
     int64_t alloc_epoch = 0;
@@ -242,6 +246,9 @@ rg::DevParams dev_params(const rg_handle* h) {
     p.queue = h->queue;
     p.bwd_window = h->cfg.bwd_window > 0.0f ? h->cfg.bwd_window : 0.5f;
     p.fwd_jump = h->cfg.fwd_round_per_slab ? 0 : 1;
+    p.rays_per_wave = 64;
+    p.wide = nullptr;
+    p.wide_count = nullptr;
     return p;
 }
 
@@ -321,7 +328,7 @@ int rg_destroy(rg_handle* h) {
                     h->bvh.vals[0], h->bvh.vals[1], h->bvh.hist, h->bvh.perm, h->bvh.iperm, h->bvh.nodes,
                     h->bvh.parent, h->bvh.right, h->bvh.counter, h->bvh.leaf_node, h->bvh.k_parent,
                     h->bvh.k_left, h->bvh.k_right, h->bvh.k_first, h->bvh.k_last, h->cams, h->rgb, h->drgb,
-                    h->train_rgb, h->rec, h->rec_len, h->rec_id, h->bvh.sah_prims[0], h->bvh.sah_prims[1],
+                    h->train_rgb, h->rec, h->rec_len, h->rec_id, h->wide, h->bvh.sah_prims[0], h->bvh.sah_prims[1],
                     h->bvh.sah_tasks[0], h->bvh.sah_tasks[1], h->bvh.sah_ctr, h->bvh.k_pre};
     for (void* p : ptrs)
         if (p) hipFree(p);
@@ -422,6 +429,23 @@ int rg_set_view_colors(rg_handle* h, int32_t view, const float* rgb, void* strea
     return RG_OK;
 }
 
+// Wavefronts of the job: how many rays each holds, and room for those that the tile kernels leave to
+// the slab stepper.  A whole view whose 8x8 blocks are all narrow beams leaves none.
+static int plan_waves(rg_handle* h, const rg::RayJob& j, rg::DevParams& p) {
+    if (rg::stepper_only(p)) return RG_OK;
+    p.rays_per_wave = rg::rays_per_wave(j.num_rays);
+    if (!j.ray_view && !j.pixels && rg::view_is_narrow(h->host_cams[j.view], h->n)) return RG_OK;
+    const int64_t waves = (j.num_rays + 63) / 64 * (64 / p.rays_per_wave);
+    if (waves > h->wide_cap) {
+        int rc;
+        h->wide_cap = 0;
+        if ((rc = dalloc(h, &h->wide, waves))) return rc;
+        h->wide_cap = waves;
+    }
+    p.wide = h->wide;
+    return RG_OK;
+}
+
 // Hit-list records: with cfg.replay_words > 0 a forward records, per ray, the lists it gathered
 // and returns a token for them; a backward given that token (and nothing in between: no
 // rg_prepare, rg_set_views, rg_set_config or other recording forward) replays them instead of
@@ -453,6 +477,7 @@ static uint64_t rec_forward(rg_handle* h, const rg::RayJob& j, rg::DevParams& p)
     h->rec_set.gen = h->generation;
     h->rec_set.num_rays = j.num_rays;
     h->rec_set.words = words;
+    h->rec_set.rays_per_wave = p.rays_per_wave;
     return h->rec_set.token;
 }
 
@@ -466,6 +491,7 @@ static void rec_backward(const rg_handle* h, const rg::RayJob& j, uint64_t token
     p.rec_id = h->rec_id;
     p.rec_words = r.words;
     p.rec_mode = 2;
+    p.rays_per_wave = r.rays_per_wave;  // the records' layout (never fewer wavefronts than planned)
 }
 
 int rg_forward(rg_handle* h, int32_t view, int64_t num_rays, const int32_t* pixels, float* out_rgb, float* out_depth,
@@ -482,6 +508,7 @@ int rg_forward(rg_handle* h, int32_t view, int64_t num_rays, const int32_t* pixe
     HIPCHK(h, rg::launch_reset_counters(dev_stats(h), s));
     const rg::RayJob job = single_job(h, view, num_rays, pixels);
     rg::DevParams p = dev_params(h);
+    if ((rc = plan_waves(h, job, p))) return rc;
     const uint64_t token = rec_forward(h, job, p);
     HIPCHK(h, rg::launch_forward(dev_scene(h), p, job, fwd_depth(h), out_rgb, out_depth, out_opacity, dev_stats(h), s));
     if (out_token) *out_token = token;
@@ -501,6 +528,7 @@ int rg_backward(rg_handle* h, int32_t view, int64_t num_rays, const int32_t* pix
     const rg::RayJob job = single_job(h, view, num_rays, pixels);
     const rg::DevGrad gr = dev_grad(h);
     rg::DevParams p = dev_params(h);
+    if ((rc = plan_waves(h, job, p))) return rc;
     rec_backward(h, job, replay_token, p);
     p.ray_chunk = h->cfg.bwd_ray_chunk;
     HIPCHK(h, rg::launch_backward(dev_scene(h), p, job, h->cfg.hit_depth, ray_colors, dL_dC, nullptr, 0, 1, gr,
@@ -534,6 +562,7 @@ int rg_forward_batch(rg_handle* h, const rg_ray_batch* b, float* out_rgb, float*
     hipStream_t s = static_cast<hipStream_t>(stream);
     HIPCHK(h, rg::launch_reset_counters(dev_stats(h), s));
     rg::DevParams p = dev_params(h);
+    if ((rc = plan_waves(h, j, p))) return rc;
     const uint64_t token = rec_forward(h, j, p);
     HIPCHK(h, rg::launch_forward(dev_scene(h), p, j, fwd_depth(h), out_rgb, out_depth, out_opacity, dev_stats(h), s));
     if (out_token) *out_token = token;
@@ -550,6 +579,7 @@ int rg_backward_batch(rg_handle* h, const rg_ray_batch* b, const float* ray_colo
     HIPCHK(h, rg::launch_reset_counters(dev_stats(h), s));
     const rg::DevGrad gr = dev_grad(h);
     rg::DevParams p = dev_params(h);
+    if ((rc = plan_waves(h, j, p))) return rc;
     rec_backward(h, j, replay_token, p);
     p.ray_chunk = h->cfg.bwd_ray_chunk;
     HIPCHK(h, rg::launch_backward(dev_scene(h), p, j, h->cfg.hit_depth, ray_colors, dL_dC, nullptr, 0, 1, gr,
@@ -577,15 +607,16 @@ int rg_train_batch(rg_handle* h, const rg_ray_batch* b, const float* target, int
     }
     const rg::DevScene sc = dev_scene(h);
     rg::DevParams p = dev_params(h);
+    if ((rc = plan_waves(h, j, p))) return rc;
     const uint64_t token = rec_forward(h, j, p);
     HIPCHK(h, rg::launch_forward(sc, p, j, fwd_depth(h), rgb, nullptr, nullptr, dev_stats(h), s));
     p = dev_params(h);
+    if ((rc = plan_waves(h, j, p))) return rc;
     rec_backward(h, j, token, p);
     p.ray_chunk = h->cfg.bwd_ray_chunk;
     HIPCHK(h, rg::launch_backward(sc, p, j, h->cfg.hit_depth, rgb, nullptr, target, loss_kind, 0, dev_grad(h),
                                   dev_stats(h), s));
-    if (out_loss)
-        HIPCHK(h, hipMemcpyAsync(out_loss, h->counters + 6, sizeof(float), hipMemcpyDeviceToDevice, s));
+    if (out_loss) HIPCHK(h, rg::launch_loss_out(dev_stats(h), out_loss, s));
     return RG_OK;
 }
 

@@ -244,7 +244,7 @@ __global__ void k_preorder(int n, const int* __restrict__ kl, const int* __restr
     const int size = 2 * (last - first + 1) - 1;
     const int miss = pre + size;  // == total when nothing follows
     nodes[2 * pre].w = __int_as_float(miss);
-    nodes[2 * pre + 1].w = __int_as_float(leafk);
+    if (!internal) nodes[2 * pre + 1].w = __int_as_float(leafk);
     const int p = kpar[x];
     if (p < 0) {
         parent[pre] = -1;
@@ -254,6 +254,7 @@ __global__ void k_preorder(int n, const int* __restrict__ kl, const int* __restr
         const int ppre = 2 * kf[p] + lt;  // right edge adds no left turn
         parent[pre] = ppre;
         right[ppre] = pre;
+        nodes[2 * ppre + 1].w = __int_as_float(~pre);
     }
     if (!internal) leaf_node[leafk] = pre;
     else kpre[x] = pre;
@@ -276,7 +277,7 @@ __device__ __forceinline__ void refit_internal(int q, float4* nodes, const int* 
     const float4 blo = nodes[2 * b], bhi = nodes[2 * b + 1];
     const float qmiss = nodes[2 * q].w;
     nodes[2 * q] = make_float4(fminf(alo.x, blo.x), fminf(alo.y, blo.y), fminf(alo.z, blo.z), qmiss);
-    nodes[2 * q + 1] = make_float4(fmaxf(ahi.x, bhi.x), fmaxf(ahi.y, bhi.y), fmaxf(ahi.z, bhi.z), __int_as_float(-1));
+    nodes[2 * q + 1] = make_float4(fmaxf(ahi.x, bhi.x), fmaxf(ahi.y, bhi.y), fmaxf(ahi.z, bhi.z), __int_as_float(~b));
 }
 
 __device__ __forceinline__ bool same_bits(float a, float b) { return __float_as_int(a) == __float_as_int(b); }

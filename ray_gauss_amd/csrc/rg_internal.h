@@ -10,7 +10,8 @@
 //   leafbox[2*slot+0..1] = padded AABB (lo.xyz, -), (hi.xyz, -)
 //   rgb[v*n + slot] = (r, g, b, 0) per-view colour                           float4
 //   nodes[2*p+0] = (lo.xyz, miss), nodes[2*p+1] = (hi.xyz, leaf)  p = DFS preorder index
-//     internal node: left child p+1, right child right[p]; leaf: leaf = slot, -1 otherwise;
+//     internal node: left child p+1, right child right[p], leaf = ~right[p] (negative); leaf node:
+//     leaf = slot;
 //     miss = index of the first node after p's subtree (= total when none): a threaded tree,
 //     traversed with no stack.
 //   acc[16*slot + ...] gradient accumulators: 0-2 d mu, 3 d sigma, 4-6 d s, 8-11 d q(w,x,y,z)
@@ -51,11 +52,12 @@ struct DevParams {
     int jitter;      // sub-pixel jitter of the rays
     int rnd_sample;  // sample offsets: 0 none, 1 random, 2 half a sample
     unsigned int iteration;  // seeds each ray's generator: tea4(iteration, pixel)
-    // hit-list records (rg_train_batch): ray r owns words rec[r * rec_words ...]; rec_len[r] = words
-    // written (bit 31: the records stop early).  rec_mode 0 off, 1 forward writes, 2 backward reads.
+    // hit-list records: rec_words words per ray; rec_len[item] = words written (bit 31: the records stop
+    // early; bit 30: the wavefront's tile record, in cells).  rec_mode 0 off, 1 forward writes, 2
+    // backward reads.
     unsigned int* rec;
     int* rec_len;
-    int2* rec_id;  // (view, pixel) of the ray whose records row r holds
+    int2* rec_id;  // (view, pixel) of the ray that the item's records were made for
     int rec_words;
     int rec_mode;
     // launch structure of the ray kernels: ray_chunk 0 = one 8x8 tile per wavefront, grid-launched,
@@ -70,6 +72,12 @@ struct DevParams {
     float bwd_window;
     // forward: step over slabs empty for every lane of a wavefront together (jump_empty)
     int fwd_jump;
+    // rays a wavefront holds (64, 32, 16, 8 or 4; fewer than 64 only in grid launches)
+    int rays_per_wave;
+    // wavefronts whose rays do not make up narrow beams, left by the tile kernel to the slab stepper:
+    // (wavefront, lanes: low, high word, 0), and their number (nullptr: none)
+    int4* wide;
+    unsigned long long* wide_count;
 };
 
 // Gradient accumulators (device-scope atomic adds; the finish kernel reads and clears them).
@@ -81,7 +89,8 @@ struct DevGrad {
 
 // Counters (device, 16): 0 K, 1 P, 2 overflow slabs, 3 fallback slabs, 4 gathers, 6 loss (float),
 // 7 debug scratch, 8 record words, 9 truncated records, 10 dropped by bounds checks, 11 rays with
-// an out-of-range view or pixel, 12..15 unused
+// an out-of-range view or pixel, 12 / 13 wavefronts left to the stepper by the forward / backward,
+// 14 loss of narrow wavefronts (double), 15 unused
 struct DevStats {
     unsigned long long* c;
 };
@@ -211,14 +220,30 @@ struct RayJob {
     const rg_camera* cams;     // device array
     int num_views;
 };
+constexpr int kWideBlocks = 4096;  // blocks of a stepper launch over the tile kernel's leftovers
+hipError_t launch_forward_steps(const DevScene& sc, const DevParams& p, const RayJob& job, int hit_depth, float* out_rgb,
+                                float* out_depth, float* out_opacity, DevStats st, hipStream_t s);
+hipError_t launch_backward_steps(const DevScene& sc, const DevParams& p, const RayJob& job, int hit_depth,
+                                 const float* ray_colors, const float* dLdC, const float* target, int loss_kind,
+                                 int count_stats, DevGrad gr, DevStats st, hipStream_t s);
+hipError_t launch_reset_counters(DevStats st, hipStream_t s);
+hipError_t launch_loss_out(DevStats st, float* out, hipStream_t s);
+hipError_t launch_debug_hits(const DevScene& sc, const DevParams& p, const RayJob& job, int max_slabs, int max_pairs,
+                             int32_t* pairs, int64_t* counts, float* ro, float* rd, float* te, float* tx,
+                             hipStream_t s);
+
+// ---- launchers (tile.hip) ---------------------------------------------------------------------
+// Whether these settings leave every ray to the slab stepper (in wavefronts of 64).
+bool stepper_only(const DevParams& p);
+// Rays per wavefront for a job of num_items work items.
+int rays_per_wave(int64_t num_items);
+// Whether every 8x8 pixel block of the view (jittered or not) is a beam that the tile kernels take.
+bool view_is_narrow(const rg_camera& cam, int64_t n);
+// Forward and backward of a job: tiles, then (p.wide) what they leave to the slab stepper.
 hipError_t launch_forward(const DevScene& sc, const DevParams& p, const RayJob& job, int hit_depth, float* out_rgb,
                           float* out_depth, float* out_opacity, DevStats st, hipStream_t s);
 hipError_t launch_backward(const DevScene& sc, const DevParams& p, const RayJob& job, int hit_depth,
                            const float* ray_colors, const float* dLdC, const float* target, int loss_kind,
                            int count_stats, DevGrad gr, DevStats st, hipStream_t s);
-hipError_t launch_reset_counters(DevStats st, hipStream_t s);
-hipError_t launch_debug_hits(const DevScene& sc, const DevParams& p, const RayJob& job, int max_slabs, int max_pairs,
-                             int32_t* pairs, int64_t* counts, float* ro, float* rd, float* te, float* tx,
-                             hipStream_t s);
 
 }  // namespace rg

@@ -14,7 +14,7 @@ constexpr int kWave = 64;
 constexpr int kGradVals = 14;
 
 enum CounterIdx { C_K = 0, C_P = 1, C_OVF = 2, C_FALLBACK = 3, C_GATHER = 4, C_LOSS = 6, C_REC_WORDS = 8,
-                  C_REC_FULL = 9, C_DROP = 10, C_BAD = 11 };
+                  C_REC_FULL = 9, C_DROP = 10, C_BAD = 11, C_LOSS64 = 14 };
 
 struct RayOut {
     float C[3];
@@ -353,21 +353,23 @@ __device__ __forceinline__ void trav(const DevParams& p, const DevScene& sc, con
     else traverse(sc.nodes, sc.total_nodes, ray, ta, tb, on_leaf);
 }
 
-// Layout: the rays of a group of 64 (ray index / 64) share one region; sector c of ray r sits at
-// ((group * C + c) * 64 + r % 64) * 8 words, C = words per ray / 8.  The 64 rays of a wavefront
-// thus write neighbouring sectors (no stride that would send every lane to one memory channel).
+// Layout: the R rays of a wavefront (DevParams::rays_per_wave) share one region of R * words per ray;
+// sector c of the ray in lane l sits at (c * R + l) * 8 words.  The rays of a wavefront thus write
+// neighbouring sectors (no stride that would send every lane to one memory channel).
 struct Rec {
     unsigned int* w = nullptr;  // sector 0 of this ray; nullptr: off
+    int stride = 8 * kWave;     // words from one of its sectors to the next
     int pos = 0;                // next word (a multiple of 8)
     int end = 0;                // capacity (recording) or words recorded (replay)
     bool full = false;          // recording ran out of space
 };
 
-__device__ __forceinline__ unsigned int* rec_base(unsigned int* rec, int64_t ray, int words) {
-    return rec + (((ray >> 6) * (int64_t)(words >> 3)) * 64 + (ray & 63)) * 8;
+// Region of wavefront `wave` (groups of 64 items cut into 64 / rays_per_wave wavefronts each).
+__device__ __forceinline__ unsigned int* rec_region(const DevParams& p, int64_t wave) {
+    return p.rec + wave * ((int64_t)p.rays_per_wave * p.rec_words);
 }
 
-__device__ __forceinline__ unsigned int* rec_at(const Rec& rc, int w) { return rc.w + ((w >> 3) << 9) + (w & 7); }
+__device__ __forceinline__ unsigned int* rec_at(const Rec& rc, int w) { return rc.w + (w >> 3) * rc.stride + (w & 7); }
 
 __device__ __forceinline__ int rec_len(int cnt) { return (2 + cnt + 7) & ~7; }
 
@@ -409,6 +411,30 @@ __device__ __forceinline__ void flush_counters(const Counters& c, DevStats st) {
     }
 }
 
+// Item of lane `lane` of wavefront `wave`, -1 for a lane without one.  With 64 rays per wavefront the
+// items are consecutive (8x8 tiles of a view); with fewer, each group of 64 items is cut along the
+// Z-curve of its 8x8 tile, so that 16 rays are a 4x4 block and 4 rays a 2x2 block.
+__device__ __forceinline__ int64_t wave_item(const DevParams& p, int64_t wave, int lane) {
+    if (p.rays_per_wave == kWave) return wave * kWave + lane;
+    if (lane >= p.rays_per_wave) return -1;
+    const int64_t i = wave * p.rays_per_wave + lane;
+    const int z = (int)(i & 63);
+    const int x = (z & 1) | ((z >> 1) & 2) | ((z >> 2) & 4), y = ((z >> 1) & 1) | ((z >> 2) & 2) | ((z >> 3) & 4);
+    return (i & ~(int64_t)63) + 8 * y + x;
+}
+
+// rec_len of a ray in a wavefront's tile record: its 16-byte cells, the ray's beam in it, kTileRecord.
+constexpr int kTileRecord = 0x40000000, kTileGroupShift = 28;
+
+// Starts a ray: clears its output; false when the ray has no slab to process (it misses the scene
+// box, or its first slab is below half an ulp of t).
+__device__ __forceinline__ bool forward_begin(const DevParams& p, const Ray& ray, RayOut& o) {
+    o.C[0] = o.C[1] = o.C[2] = 0.0f;
+    o.depth = 0.0f;
+    o.T = 1.0f;
+    return ray.tenter < ray.texit && add_exact(ray.tenter, p.dt * (float)p.spb) > ray.tenter;
+}
+
 enum RayStatus { RAY_NONE = 0, RAY_OK = 1, RAY_BAD = 2 };
 
 // Work item -> (view, pixel, output row).  RAY_NONE: past the end of the job, or a padding item
@@ -447,13 +473,12 @@ __device__ __forceinline__ int resolve(const RayJob& job, int64_t w, RayRef& q) 
 // Writes a finished ray's colour (with the background behind its remaining transmittance),
 // depth and opacity, and closes its hit-list records.
 template <int RM>
-__device__ __forceinline__ void forward_finish(const DevParams& p, const RayRef& q, const RayOut& o, const Rec& rc,
+__device__ __forceinline__ void forward_finish(const DevParams& p, const RayRef& q, int64_t item, const RayOut& o, const Rec& rc,
                                                Counters& ctr, float* __restrict__ out_rgb, float* __restrict__ out_depth,
                                                float* __restrict__ out_opac) {
     if constexpr (RM == 1) {
-        p.rec_len[q.out] = rc.pos | (rc.full ? (int)0x80000000u : 0);
-        p.rec_id[q.out] = make_int2(q.view, q.pixel);  // the backward replays only the same ray
-        ctr.rec_words += rc.pos;
+        p.rec_len[item] = rc.pos | (rc.full ? (int)0x80000000u : 0);
+        p.rec_id[item] = make_int2(q.view, q.pixel);  // the backward replays only the same ray
         ctr.rec_full += rc.full ? 1u : 0u;
     }
     out_rgb[3 * q.out + 0] = o.C[0] + o.T * p.bg;
@@ -465,7 +490,7 @@ __device__ __forceinline__ void forward_finish(const DevParams& p, const RayRef&
 
 // A ray whose view or pixel index is out of range: NaN outputs, no records, counted.
 template <int RM>
-__device__ __forceinline__ void forward_bad(const DevParams& p, const RayRef& q, DevStats st,
+__device__ __forceinline__ void forward_bad(const DevParams& p, const RayRef& q, int64_t item, DevStats st,
                                             float* __restrict__ out_rgb, float* __restrict__ out_depth,
                                             float* __restrict__ out_opac) {
     atomicAdd(&st.c[C_BAD], 1ull);
@@ -476,8 +501,8 @@ __device__ __forceinline__ void forward_bad(const DevParams& p, const RayRef& q,
     if (out_depth) out_depth[q.out] = nan;
     if (out_opac) out_opac[q.out] = nan;
     if constexpr (RM == 1) {
-        p.rec_len[q.out] = 0;
-        p.rec_id[q.out] = make_int2(-1, -1);
+        p.rec_len[item] = 0;
+        p.rec_id[item] = make_int2(-1, -1);
     }
 }
 
@@ -496,6 +521,8 @@ struct BwdRay {
     float dL[3] = {0.0f, 0.0f, 0.0f};
     float Cf[3] = {0.0f, 0.0f, 0.0f};
     int view = 0;
+    int tile = -1;       // the ray's beam in its wavefront's tile record (-1: none)
+    bool trunc = false;  // the record holds its hits up to some depth only
     Rec rc;
 };
 
@@ -503,10 +530,10 @@ struct BwdRay {
 // per-pixel loss against target, whose value is added to loss), its hit-list records when they
 // were written for this same ray, and the ray itself.  A ray with zero dL/dC stays inactive.
 template <bool RNG, int RM>
-__device__ __forceinline__ void backward_setup(const DevScene& sc, const DevParams& p, const RayJob& job, int64_t item,
-                                               const float* __restrict__ ray_colors, const float* __restrict__ dLdC,
-                                               const float* __restrict__ target, int loss_kind, DevStats st,
-                                               BwdRay& b, float& loss) {
+__device__ __forceinline__ void backward_setup(const DevScene& sc, const DevParams& p, const RayJob& job, int64_t wave,
+                                               int lane, int64_t item, const float* __restrict__ ray_colors,
+                                               const float* __restrict__ dLdC, const float* __restrict__ target,
+                                               int loss_kind, DevStats st, BwdRay& b, float& loss) {
     RayRef q;
     const int rs = resolve(job, item, q);
     if (rs == RAY_BAD) atomicAdd(&st.c[C_BAD], 1ull);
@@ -535,17 +562,34 @@ __device__ __forceinline__ void backward_setup(const DevScene& sc, const DevPara
     b.active = true;
     b.view = q.view;
     if constexpr (RM == 2) {
-        // records of this output row are replayed only when the forward wrote them for the same
+        // records of this item are replayed only when the forward wrote them for the same
         // (view, pixel); otherwise the ray walks the tree
-        const int2 id = p.rec_id[q.out];
+        const int2 id = p.rec_id[item];
         if (id.x == q.view && id.y == q.pixel) {
-            b.rc.w = rec_base(p.rec, q.out, p.rec_words);
-            b.rc.end = min(p.rec_len[q.out] & 0x7fffffff, p.rec_words);
+            const int len = p.rec_len[item];
+            if (len & kTileRecord) {
+                b.tile = (len >> kTileGroupShift) & 3;
+                b.trunc = len < 0;
+                b.rc.end = min(len & ((1 << kTileGroupShift) - 1), (p.rays_per_wave * p.rec_words) >> 2);
+            } else {
+                b.rc.w = rec_region(p, wave) + 8 * lane;
+                b.rc.stride = 8 * p.rays_per_wave;
+                b.rc.end = min(len & 0x7fffffff, p.rec_words);
+            }
         }
     }
     const rg_camera cam = job.cams[q.view];
     b.seed = RNG ? tea4(p.iteration, (unsigned int)q.pixel) : 0u;
     b.ray = make_ray(cam, q.pixel, sc.box, p.t_near, p.t_far, RNG ? p.jitter : 0, &b.seed);
+}
+
+// Adds the wavefront's loss to the loss counters: whole wavefronts in 32 bits, the many small terms
+// of narrow ones in 64, where the order of their additions does not show (k_loss_out adds the two).
+__device__ __forceinline__ void add_loss(const DevParams& p, float loss, int lane, DevStats st) {
+    const float ls = wave_sum64(loss);
+    if (lane != 0 || ls == 0.0f) return;
+    if (p.rays_per_wave == kWave) atomicAdd(reinterpret_cast<float*>(&st.c[C_LOSS]), ls);
+    else atomicAdd(reinterpret_cast<double*>(&st.c[C_LOSS64]), (double)ls);
 }
 
 // ------------------------------------------------------------------ persistent kernels --------
@@ -594,6 +638,11 @@ __device__ __forceinline__ bool take_chunk(const DevParams& p, int64_t num_items
 // Lanes of mask below this lane.
 __device__ __forceinline__ int lanes_below(unsigned long long mask) {
     return __builtin_amdgcn_mbcnt_hi((unsigned int)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)mask, 0u));
+}
+
+// Wavefronts of a job (groups of 64 items, each cut into 64 / rays_per_wave).
+inline int64_t num_waves(const DevParams& p, int64_t items) {
+    return (items + kWave - 1) / kWave * (kWave / p.rays_per_wave);
 }
 
 }  // namespace rg

@@ -1,0 +1,638 @@
+// Tile kernels: the forward and backward of wavefronts whose rays form narrow beams.
+//
+// A wavefront whose rays form a narrow beam (8x8 tiles of a view, subsets of them) marches as one:
+// in each round the lanes near the laggard (tile_window) process one slab each, and the
+// candidates whose depth range meets the round's come from one list for all lanes (beam_gather),
+// taken in slot order.  A candidate's record is read once for the wavefront, through scalar loads,
+// and every lane applies the exact predicate to it; the slabs a ray processes, the hits it sums in
+// each and their order are those of the per-ray slab stepper (trace.hip).
+
+#include <hip/hip_runtime.h>
+
+#include <climits>
+
+#include "rg_device.h"
+#include "rg_internal.h"
+#include "rg_tile.h"
+#include "rg_trace.h"
+
+namespace rg {
+namespace {
+
+constexpr int kMaxSeg = 4096;
+
+constexpr float kTileSync = 0.75f;  // lanes within this many slabs of the laggard step together
+// A wavefront's rays make up at most kTileGroups beams, each of one view and within the spread
+// (per direction component, from its first ray; 8x8 pixels of a 1000-pixel, 40-degree view are 0.006)
+// kTileSpread and sqrt(kTileDensity / n); other wavefronts go to the slab stepper.  A beam's
+// candidates grow with the Gaussians and with the square of its width, its rays' own hits do not.
+// Measured on 64 random rays of a block of S pixels out of 1024 (stepper / tile, train step): 1M
+// Gaussians S = 32 103 / 54 ms, 64 175 / 152, 128 (spread 0.09) 274 / 377; 300k Gaussians S = 128
+// 109 / 88, 256 125 / 97; 20k 256 10.1 / 8.9.  Several beams: a list of 8x8 tiles with ragged edges
+// has wavefronts that hold the end of one row of tiles and the start of the next (one beam each; in
+// the stepper the 1 % of such wavefronts took 10 of 290 ms at 1M Gaussians).
+constexpr float kTileSpread = 0.2f, kTileDensity = 3000.0f;
+constexpr int kTileGroups = 4;
+
+// Assigns the lanes with act to beams (group 0 .. kTileGroups - 1); false when they make up more.
+__device__ __forceinline__ bool tile_groups(const DevScene& sc, bool act, int view, const Ray& r, int& group) {
+    const float limit = fminf(kTileSpread, __builtin_sqrtf(kTileDensity / (float)sc.n));
+    group = -1;
+    unsigned long long rem = __ballot(act);
+    for (int k = 0; k < kTileGroups && rem != 0ULL; ++k) {
+        const int f = __ffsll((long long)rem) - 1;
+        const float x = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(r.dx), f));
+        const float y = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(r.dy), f));
+        const float z = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(r.dz), f));
+        const bool near = fabsf(r.dx - x) <= limit && fabsf(r.dy - y) <= limit && fabsf(r.dz - z) <= limit;
+        const bool mine = ((rem >> threadIdx.x) & 1ULL) != 0ULL && view == __builtin_amdgcn_readlane(view, f) && near;
+        if (mine) group = k;
+        const unsigned long long m = __ballot(mine);
+        if (m == 0ULL) return false;  // a NaN direction
+        rem &= ~m;
+    }
+    return rem == 0ULL;
+}
+
+// The gathered depth range of a marching tile (wave-uniform).
+struct TileWalk {
+    float s1 = 0.0f;      // end of the range
+    int m = 1;            // its length in slabs
+    int cnt = 0;          // candidates in the list
+    bool valid = false;
+    bool direct = false;  // the round's candidates do not fit: it walks the tree itself
+};
+
+// Makes the list cover the round [tlag, whi].  The range's length doubles while the list is mostly
+// empty and halves while it is nearly full; a round whose own candidates do not fit is walked.
+__device__ __forceinline__ void tile_list(TileWalk& w, const DevScene& sc, const Beam& b, float tlag, float whi,
+                                          float slab, TileLds& W, int lane, bool alive, Counters& ctr) {
+    if (w.valid && !(whi > w.s1)) return;
+    if (w.valid && 4 * w.cnt < kTileCand) w.m = min(w.m * 2, kMaxSeg);
+    else if (w.valid && 4 * w.cnt > 3 * kTileCand) w.m = max(w.m >> 1, 1);
+    w.valid = true;
+    w.direct = false;
+    while (true) {
+        w.s1 = w.m > 1 ? fmaxf(tlag + (float)(w.m + 1) * slab, whi) : whi;
+        w.cnt = beam_gather(sc.nodes, sc.geo, sc.total_nodes, b, tlag, w.s1, W, lane);
+        if (alive) ctr.gathers++;
+        if (w.cnt >= 0) return;
+        if (w.m == 1) break;
+        w.m >>= 1;
+    }
+    w.cnt = 0;
+    w.direct = true;
+}
+
+// The lanes of the next round: its depths [tlag, whi] and whether this lane takes part.
+__device__ __forceinline__ bool tile_window(bool alive, float tb, float slab, float& tlag, float& whi) {
+    tlag = uniform_f(wave_min64f(alive ? tb : INFINITY));
+    const bool part = alive && tb < tlag + kTileSync * slab;
+    whi = add_exact(uniform_f(wave_max64f(part ? tb : -INFINITY)), slab);
+    return part;
+}
+
+// Chunk j of the list: this lane's candidate and the lanes whose candidate meets [wlo, whi].
+__device__ __forceinline__ unsigned long long tile_chunk(const TileLds& W, int cnt, int j, int lane, float wlo, float whi,
+                                                         int& slot) {
+    const int i = 64 * j + lane;
+    const bool in = i < cnt;
+    slot = in ? W.slot[i] : 0;
+    return __ballot(in && !(W.z0[i] > whi) && !(W.z1[i] < wlo));
+}
+
+// After a round without candidates: every lane steps over the slabs that end before the next
+// candidate's depths (or the end of the list).
+__device__ __forceinline__ void tile_jump(const TileWalk& w, const TileLds& W, int lane, float whi, float slab, bool alive,
+                                          const Ray& ray, float& tb) {
+    float next = w.s1;
+    for (int i = lane; i < w.cnt; i += kWave)
+        if (W.z0[i] > whi) next = fminf(next, W.z0[i]);
+    next = uniform_f(wave_min64f(next));
+    while (alive) {
+        const float nt = add_exact(tb, slab);
+        if (!(tb < ray.texit) || !(fminf(ray.texit, nt) < next) || !(nt > tb)) break;
+        tb = nt;
+    }
+}
+
+// Record of a tile: 16-byte cells in the space of its rays' hit-list records.  Per round with hits a
+// header (depth of the laggard, number of events, view, beam) followed by its events (slot, lanes that
+// hit it: low word, high word, 0).  A lane's slab of a round is the first at or beyond the header's
+// depth.  One lane stores each cell: eight share a cache line, which leaves L2 once.
+struct TileRec {
+    u32x4* cells = nullptr;
+    int pos = 0, cap = 0;  // cells of whole rounds written, cells there are
+    bool full = false;     // a round did not fit: nothing is recorded from it on
+    int n = 0;             // events of the current round
+};
+
+__device__ __forceinline__ void tile_rec_event(TileRec& r, int slot, unsigned long long hits, int lane) {
+    ++r.n;
+    if (r.pos + r.n >= r.cap) r.full = true;
+    if (lane == 0 && !r.full)
+        r.cells[r.pos + r.n] = u32x4{(unsigned int)slot, (unsigned int)hits, (unsigned int)(hits >> 32), 0u};
+}
+
+__device__ __forceinline__ void tile_rec_round(TileRec& r, float tlag, int view, int group, int lane) {
+    if (r.n > 0 && !r.full) {
+        if (lane == 0) 
+            r.cells[r.pos] = u32x4{__float_as_uint(tlag), (unsigned int)r.n, (unsigned int)view, (unsigned int)group};
+        r.pos += 1 + r.n;
+    }
+    r.n = 0;
+}
+
+// Forward of the lanes with act, which share their view, as one beam.  Called by all 64 lanes.
+template <int SPB, bool RNG, int RM>
+__device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams& p, bool act, const Ray& ray,
+                                             unsigned int& seed, int view, int group, int hit_depth, TileLds& W, int lane,
+                                             Counters& ctr, RayOut& o, TileRec& rc) {
+    const float slab = p.dt * (float)p.spb;
+    const float4* __restrict__ rgbv = sc.rgb + (size_t)view * sc.n;
+    const Beam beam = make_beam(act, ray);
+    TileWalk w;
+    w.m = p.seg_slabs;
+    bool alive = act && o.T > p.t_eps;
+    float tb = ray.tenter;
+    while (__ballot(alive) != 0ULL) {
+        float tlag, whi;
+        const bool part = tile_window(alive, tb, slab, tlag, whi);
+        tile_list(w, sc, beam, tlag, whi, slab, W, lane, alive, ctr);
+        const float tmin = fmaxf(ray.tenter, tb), tmax = fminf(ray.texit, add_exact(tb, slab));
+        float sig[SPB], cr[SPB], cg[SPB], cb[SPB];
+#pragma unroll
+        for (int i = 0; i < SPB; ++i) sig[i] = cr[i] = cg[i] = cb[i] = 0.0f;
+        int nh = 0;
+        auto eval = [&](int slot, bool cond) {
+            const float4 g0 = ld_uniform(sc.geo, 4 * (int64_t)slot), g1 = ld_uniform(sc.geo, 4 * (int64_t)slot + 1),
+                         g2 = ld_uniform(sc.geo, 4 * (int64_t)slot + 2), g3 = ld_uniform(sc.geo, 4 * (int64_t)slot + 3);
+            Isect I;
+            const bool hit = cond && intersect(g0, g1, g2, g3, ray, I) && overlaps(tmin, tmax, I.r1, I.r2);
+            const unsigned long long hits = __ballot(hit);
+            if (hits == 0ULL) return;
+            if constexpr (RM == 1) {
+                if (!rc.full) tile_rec_event(rc, slot, hits, lane);
+            }
+            if (hit) {
+                refine_sampling(g0, g1, g2, g3, ray, I);
+                accum_hit<SPB, RNG>(I, g0.w, ld_uniform(rgbv, slot), tb, seed, p, sig, cr, cg, cb);
+                if (tb == ray.tenter || I.r1 > tmin) ctr.P++;
+                ++nh;
+            }
+        };
+        bool any = w.direct;
+        for (int j = 0; kWave * j < w.cnt; ++j) {
+            int sl;
+            unsigned long long m = tile_chunk(W, w.cnt, j, lane, tlag, whi, sl);
+            any |= m != 0ULL;
+            while (m != 0ULL) {
+                const int slot = __builtin_amdgcn_readlane(sl, __builtin_ctzll(m));
+                m &= m - 1ULL;
+                eval(slot, part);
+            }
+        }
+        if (w.direct) {
+            const float ix = 1.0f / ray.dx, iy = 1.0f / ray.dy, iz = 1.0f / ray.dz;
+            for (int idx = 0; idx < sc.total_nodes;) {
+                idx = __builtin_amdgcn_readfirstlane(idx);
+                const float4 lo = ld_node(sc.nodes, 2 * idx), hi = ld_node(sc.nodes, 2 * idx + 1);
+                const int miss = __float_as_int(lo.w), leaf = __float_as_int(hi.w);
+                if (miss <= idx || leaf >= sc.n) break;  // malformed link: never loop
+                const bool h = part && box_hit(lo, hi, ray, ix, iy, iz, tmin, tmax);
+                const bool met = __ballot(h) != 0ULL;
+                if (met && leaf >= 0) eval(leaf, h);
+                idx = met && leaf < 0 ? idx + 1 : miss;
+            }
+            w.valid = false;
+        }
+        if constexpr (RM == 1) {
+            if (!rc.full) tile_rec_round(rc, tlag, view, group, lane);
+        }
+        if (part) {
+            if (nh > 0) {
+                ctr.K += nh;
+                if (p.max_hits > 0 && nh > p.max_hits) ctr.ovf++;
+                if (nh > hit_depth) ctr.fallback++;
+                composite<SPB, RNG>(sig, cr, cg, cb, tb, seed, p, o);
+                if (RNG && p.rnd_sample == 1) seed = skip_draws(seed, p.spb);  // the slab's draws are spent
+            }
+            const float nt = add_exact(tb, slab);
+            alive = nt > tb && nt < ray.texit && o.T > p.t_eps;
+            tb = nt;
+        }
+        if (!any && p.fwd_jump) {
+            tile_jump(w, W, lane, whi, slab, alive, ray, tb);
+            alive = alive && tb < ray.texit;
+        }
+    }
+}
+
+// Backward of the lanes with act, called by all 64 lanes.  In each round the wavefront has a list
+// of events -- a Gaussian and the lanes that hit it in their slab of the round -- which it goes
+// through twice: to recompute the slabs' sample buffers and from them the per-sample coefficients,
+// and to sum each Gaussian's gradient moments over its lanes.  The events come from the forward's
+// record of the tile (cells; lanes take part with their beam in it, tile, -1: none), and for the lanes with walk, once it ends, from the
+// tile's own gathers.
+template <int SPB, bool RNG>
+__device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParams& p, bool act, const Ray& ray,
+                                              unsigned int seed, int view, const float* Cfwd, const float* dL,
+                                              const u32x4* __restrict__ cells, int num_cells, int tile, bool walk,
+                                              TileLds& W, GradStage& G, int lane, const DevGrad& gr, Counters& ctr,
+                                              unsigned long long* drops) {
+    const float slab = p.dt * (float)p.spb;
+    int nst = 0;
+    bool alive = act && (ray.tenter < ray.texit) && (add_exact(ray.tenter, slab) > ray.tenter) && 1.0f > p.t_eps;
+    float T = 1.0f;
+    float Dr = dL[0] * Cfwd[0] + dL[1] * Cfwd[1] + dL[2] * Cfwd[2];  // dLdC . (colour not yet composited)
+    float tb = ray.tenter;
+    // events of the current batch, one per lane (in the record's case a window of its cells)
+    int ev_slot = 0, ev_lo = 0, ev_hi = 0, ev_beam = 0;
+    int wbase = -kWave;  // first cell of the window
+    auto window = [&](int first) {
+        wbase = first;
+        const int i = first + lane;
+        u32x4 c = {0u, 0u, 0u, 0u};
+        if (i < num_cells) c = __builtin_nontemporal_load(cells + i);
+        ev_slot = (int)c.x;
+        ev_lo = (int)c.y;
+        ev_hi = (int)c.z;
+        ev_beam = (int)c.w;
+    };
+    int pos = 0;
+    unsigned long long todo = 0ULL;  // lanes of the beam being walked
+    int gview = 0, group = -1;
+    Beam beam = {};
+    TileWalk w;
+    while (true) {
+        const bool replay = pos < num_cells;
+        float tlag = 0.0f, whi = 0.0f;
+        int total = 0, first = 0;  // events of the round (replay), lane of the first one
+        bool part;
+        if (replay) {
+            if (pos - wbase >= kWave) window(pos);
+            first = pos - wbase;
+            total = __builtin_amdgcn_readlane(ev_lo, first);
+            if (first + 1 + total > kWave && first > 0) {
+                window(pos);
+                first = 0;
+            }
+            tlag = __uint_as_float((unsigned int)__builtin_amdgcn_readlane(ev_slot, first));
+            gview = __builtin_amdgcn_readlane(ev_hi, first);
+            const bool mine = tile == __builtin_amdgcn_readlane(ev_beam, first);
+            ++first;
+            if (total <= 0 || total >= num_cells - pos) {  // never expected: end of the record
+                pos = num_cells;
+                continue;
+            }
+            while (alive && mine && tb < tlag) {
+                const float nt = add_exact(tb, slab);
+                if (!(nt > tb) || !(nt < ray.texit)) alive = false;
+                else tb = nt;
+            }
+            part = alive && mine && tb < tlag + kTileSync * slab;
+        } else {
+            if ((__ballot(alive && walk) & todo) == 0ULL) {  // the next beam
+                if (group < 0) {
+                    int g = 0;
+                    if (!tile_groups(sc, alive && walk, view, ray, g)) g = view;  // (left to this kernel: one view)
+                    group = alive && walk ? g : INT_MAX;
+                }
+                const unsigned long long rem = __ballot(alive && walk);
+                if (rem == 0ULL) break;
+                const int f = __ffsll((long long)rem) - 1;
+                gview = __builtin_amdgcn_readlane(view, f);
+                todo = __ballot(alive && walk && group == __builtin_amdgcn_readlane(group, f));
+                beam = make_beam(((todo >> lane) & 1ULL) != 0ULL, ray);
+                w = TileWalk();
+                w.m = p.seg_slabs;
+            }
+            const bool mine = alive && ((todo >> lane) & 1ULL) != 0ULL;
+            part = tile_window(mine, tb, slab, tlag, whi);
+            tile_list(w, sc, beam, tlag, whi, slab, W, lane, mine, ctr);
+        }
+        const float4* __restrict__ rgbv = sc.rgb + (size_t)gview * sc.n;
+        const int key_base = gview * sc.n;
+        const float tmin = fmaxf(ray.tenter, tb), tmax = fminf(ray.texit, add_exact(tb, slab));
+        const unsigned int cur_seed = seed;
+        float sig[SPB], cr[SPB], cg[SPB], cb[SPB];
+#pragma unroll
+        for (int i = 0; i < SPB; ++i) sig[i] = cr[i] = cg[i] = cb[i] = 0.0f;
+        int nh = 0;
+        bool any = false, one = false;  // the round has candidates; its events fit one batch
+        int ne = 0;
+        for (int pass = 0; pass < 2; ++pass) {
+            // the enumeration of a walked round, resumed batch by batch
+            int j = -1, sl = 0, idx = 0;
+            unsigned long long m = 0ULL;
+            for (int done = 0;;) {
+                bool last;
+                if (replay) {
+                    if (done > 0 || (pass == 1 && total >= kWave)) {  // a long round's later batches
+                        window(pos + 1 + done);
+                        first = 0;
+                    }
+                    ne = min(total - done, kWave - first);
+                    last = done + ne >= total;
+                } else if (pass == 1 && one) {
+                    last = true;
+                } else {
+                    ne = 0;
+                    last = false;
+                    while (ne < kWave) {
+                        int slot;
+                        bool cond = part;
+                        if (w.direct) {
+                            if (idx >= sc.total_nodes) {
+                                last = true;
+                                break;
+                            }
+                            idx = __builtin_amdgcn_readfirstlane(idx);
+                            const float4 lo = ld_node(sc.nodes, 2 * idx), hi = ld_node(sc.nodes, 2 * idx + 1);
+                            const int miss = __float_as_int(lo.w);
+                            slot = __float_as_int(hi.w);
+                            if (miss <= idx || slot >= sc.n) {  // malformed link: never loop
+                                last = true;
+                                break;
+                            }
+                            cond = part && box_hit(lo, hi, ray, 1.0f / ray.dx, 1.0f / ray.dy, 1.0f / ray.dz, tmin, tmax);
+                            const bool met = __ballot(cond) != 0ULL;
+                            idx = met && slot < 0 ? idx + 1 : miss;
+                            if (!met || slot < 0) continue;
+                            any = true;
+                        } else {
+                            if (m == 0ULL) {
+                                if (kWave * (++j) >= w.cnt) {
+                                    last = true;
+                                    break;
+                                }
+                                m = tile_chunk(W, w.cnt, j, lane, tlag, whi, sl);
+                                any |= m != 0ULL;
+                                continue;
+                            }
+                            slot = __builtin_amdgcn_readlane(sl, __builtin_ctzll(m));
+                            m &= m - 1ULL;
+                        }
+                        const float4 g0 = ld_uniform(sc.geo, 4 * (int64_t)slot), g1 = ld_uniform(sc.geo, 4 * (int64_t)slot + 1),
+                                     g2 = ld_uniform(sc.geo, 4 * (int64_t)slot + 2),
+                                     g3 = ld_uniform(sc.geo, 4 * (int64_t)slot + 3);
+                        Isect I;
+                        const bool hit = cond && intersect(g0, g1, g2, g3, ray, I) && overlaps(tmin, tmax, I.r1, I.r2);
+                        const unsigned long long hits = __ballot(hit);
+                        if (hits == 0ULL) continue;
+                        const bool at = lane == ne;
+                        ev_slot = at ? slot : ev_slot;
+                        ev_lo = at ? (int)(unsigned int)hits : ev_lo;
+                        ev_hi = at ? (int)(unsigned int)(hits >> 32) : ev_hi;
+                        ++ne;
+                    }
+                    first = 0;
+                    if (pass == 0 && done == 0) one = last;
+                }
+                for (int e = first; e < first + ne; ++e) {
+                    const int slot = __builtin_amdgcn_readlane(ev_slot, e);
+                    const unsigned long long hits =
+                        (unsigned long long)(unsigned int)__builtin_amdgcn_readlane(ev_lo, e) |
+                        (unsigned long long)(unsigned int)__builtin_amdgcn_readlane(ev_hi, e) << 32;
+                    const bool in = part && ((hits >> lane) & 1ULL) != 0ULL;
+                    if (__ballot(in) == 0ULL) continue;
+                    if ((unsigned)slot >= (unsigned)sc.n) {
+                        if (lane == 0) count_drop(drops);
+                        continue;
+                    }
+                    const float4 g0 = ld_uniform(sc.geo, 4 * (int64_t)slot), g1 = ld_uniform(sc.geo, 4 * (int64_t)slot + 1),
+                                 g2 = ld_uniform(sc.geo, 4 * (int64_t)slot + 2), g3 = ld_uniform(sc.geo, 4 * (int64_t)slot + 3);
+                    const float4 col = ld_uniform(rgbv, slot);
+                    float v[kMoments];
+#pragma unroll
+                    for (int k = 0; k < kMoments; ++k) v[k] = 0.0f;
+                    if (in) {
+                        // the hit passed the exact test: only its sampling terms are computed
+                        Isect I;
+                        float bq, cq;
+                        isect_terms(g0, g1, g2, g3, ray, I, bq, cq);
+                        refine_sampling(g0, g1, g2, g3, ray, I);
+                        if (pass == 0) {
+                            accum_hit<SPB, RNG>(I, g0.w, col, tb, cur_seed, p, sig, cr, cg, cb);
+                            ++nh;
+                        } else {
+                            grad_moments<SPB, RNG>(I, g0.w, col, tb, cur_seed, p, sig, cr, dL, v);
+                        }
+                    }
+                    if (pass == 1) grad_scatter_wave(v, key_base + slot, sc, gr, lane, G, nst, drops);
+                }
+                done += ne;
+                if (last) break;
+            }
+            if (pass == 0) {
+                if (nh > 0) {
+                    slab_coeffs<SPB>(sig, cr, cg, cb, p, dL, T, Dr);
+                    if (RNG && p.rnd_sample == 1) seed = skip_draws(seed, p.spb);  // the slab's draws are spent
+                }
+                if (__ballot(nh > 0) == 0ULL) break;
+            }
+        }
+        if (replay) pos += 1 + total;
+        if (part) {
+            const float nt = add_exact(tb, slab);
+            alive = nt > tb && nt < ray.texit && T > p.t_eps;
+            tb = nt;
+        }
+        if (!replay) {
+            if (w.direct) w.valid = false;
+            else if (!any) {
+                const bool mine = alive && ((todo >> lane) & 1ULL) != 0ULL;
+                tile_jump(w, W, lane, whi, slab, mine, ray, tb);
+                alive = alive && tb < ray.texit;
+            }
+        }
+    }
+    stage_flush(G, nst, sc, gr, lane, drops);
+}
+
+// ------------------------------------------------------------------ kernels ------------------
+
+// Wavefront of a block: runs of `chunk` consecutive wavefronts go to one XCD (blocks are dispatched
+// round-robin over the eight), so that its L2 serves a compact part of the scene, and the runs in
+// turn to all of them, so that no XCD is left with the cheaper views of a batch.
+__device__ __forceinline__ int64_t tile_wave(int64_t b, int chunk) {
+    const int64_t k = b >> 3;
+    return ((k / chunk) * 8 + (b & 7)) * chunk + k % chunk;
+}
+
+// Leaves the lanes with mine to the slab stepper.
+__device__ __forceinline__ void tile_leave(const DevParams& p, int64_t wave, bool mine, int lane) {
+    const unsigned long long m = __ballot(mine);
+    if (lane == 0)
+        p.wide[atomicAdd(p.wide_count, 1ull)] = make_int4((int)wave, (int)(unsigned int)m, (int)(unsigned int)(m >> 32), 0);
+}
+
+template <int SPB, bool RNG, int RM>
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(SPB == 8 ? 4 : 3)))
+k_tile_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int chunk, int hit_depth,
+               float* __restrict__ out_rgb, float* __restrict__ out_depth, float* __restrict__ out_opac, DevStats st) {
+    __shared__ TileLds W;
+    const int lane = threadIdx.x;
+    const int64_t wave = tile_wave(blockIdx.x, chunk);
+    const int64_t item = wave_item(p, wave, lane);
+    const bool in = item >= 0 && item < num_items;
+    if (__ballot(in) == 0ULL) return;
+    Counters ctr;
+    RayRef q;
+    q.view = -1;
+    const int rs = in ? resolve(job, item, q) : (int)RAY_NONE;
+    Ray ray = {};
+    unsigned int seed = 0u;
+    RayOut o;
+    bool alive = false;
+    if (rs == RAY_OK) {
+        const rg_camera cam = job.cams[q.view];
+        seed = RNG ? tea4(p.iteration, (unsigned int)q.pixel) : 0u;
+        ray = make_ray(cam, q.pixel, sc.box, p.t_near, p.t_far, RNG ? p.jitter : 0, &seed);
+        alive = forward_begin(p, ray, o);
+    }
+    int group = 0;  // one view, all of it narrow
+    if (p.wide && !tile_groups(sc, alive, q.view, ray, group)) {
+        tile_leave(p, wave, in, lane);
+        return;
+    }
+    Rec rc;
+    TileRec tr;
+    if constexpr (RM == 1) {
+        tr.cells = reinterpret_cast<u32x4*>(rec_region(p, wave));
+        tr.cap = (p.rays_per_wave * p.rec_words) >> 2;
+    }
+    for (int g = 0; g < kTileGroups; ++g) {
+        const bool mine = alive && group == g;
+        const unsigned long long m = __ballot(mine);
+        if (m == 0ULL) break;
+        const int view = __builtin_amdgcn_readlane(q.view, __ffsll((long long)m) - 1);
+        forward_tile<SPB, RNG, RM>(sc, p, mine, ray, seed, view, g, hit_depth, W, lane, ctr, o, tr);
+        if (mine) rc.full = tr.full;
+    }
+    if constexpr (RM == 1) {
+        rc.pos = tr.pos | (max(group, 0) << kTileGroupShift) | kTileRecord;
+        if (lane == 0) ctr.rec_words += 4 * tr.pos;
+        if (rs == RAY_NONE && in) p.rec_id[item] = make_int2(-1, -1);  // padding: no records
+    }
+    if (rs == RAY_OK) forward_finish<RM>(p, q, item, o, rc, ctr, out_rgb, out_depth, out_opac);
+    if (rs == RAY_BAD) forward_bad<RM>(p, q, item, st, out_rgb, out_depth, out_opac);
+    flush_counters(ctr, st);
+}
+
+template <int SPB, bool RNG, int RM>
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(3)))
+k_tile_backward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int chunk, const float* __restrict__ ray_colors,
+                const float* __restrict__ dLdC, const float* __restrict__ target, int loss_kind, int count_stats,
+                DevGrad gr, DevStats st) {
+    __shared__ TileLds W;
+    __shared__ GradStage G;
+    const int lane = threadIdx.x;
+    const int64_t wave = tile_wave(blockIdx.x, chunk);
+    const int64_t item = wave_item(p, wave, lane);
+    const bool in = item >= 0 && item < num_items;
+    if (__ballot(in) == 0ULL) return;
+    Counters ctr;
+    float loss = 0.0f;
+    BwdRay b;
+    if (in) backward_setup<RNG, RM>(sc, p, job, wave, lane, item, ray_colors, dLdC, target, loss_kind, st, b, loss);
+    if (target) add_loss(p, loss, lane, st);
+    // the rays whose tile the forward recorded, and the others if they can go as a tile too
+    const unsigned long long recorded = RM == 2 ? __ballot(b.active && b.tile >= 0) : 0ULL;
+    const bool rest = b.active && b.tile < 0;
+    int group;
+    const bool leave = p.wide && __ballot(rest) != 0ULL &&
+                       (__ballot(rest && b.rc.w) != 0ULL || !tile_groups(sc, rest, b.view, b.ray, group));
+    if (leave) tile_leave(p, wave, rest, lane);
+    int num_cells = 0;
+    if (recorded != 0ULL) num_cells = __builtin_amdgcn_readlane(b.rc.end, __ffsll((long long)recorded) - 1);
+    const u32x4* cells = RM == 2 ? reinterpret_cast<const u32x4*>(rec_region(p, wave)) : nullptr;
+    backward_tile<SPB, RNG>(sc, p, b.active && !(leave && rest), b.ray, b.seed, b.view, b.Cf, b.dL, cells, num_cells,
+                            b.tile, rest || b.trunc, W, G, lane, gr, ctr, st.c + C_DROP);
+    if (count_stats) flush_counters(ctr, st);
+}
+
+// Launch of a tile kernel over all wavefronts of a job.
+template <typename K, typename... A>
+void launch_tiles(K kernel, const DevScene& sc, const DevParams& p, const RayJob& job, hipStream_t s, A... args) {
+    const int64_t waves = num_waves(p, job.num_rays);
+    const int chunk = (int)(waves < 8 * 8 * 64 ? (waves + 63) / 64 : 64);  // at least 8 runs for each XCD
+    const int64_t nb = (waves + 8 * chunk - 1) / (8 * chunk) * (8 * chunk);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(kWave), 0, s, sc, p, job, job.num_rays, chunk, args...);
+}
+
+// Specialised on SPB (8 or 16 samples per slab), on whether the random generator is used and on the
+// record mode.
+#define RG_TILE_DISPATCH(RMV, RMON, KERNEL, ...)                                                       \
+    do {                                                                                               \
+        const bool rng = p.jitter || p.rnd_sample;                                                     \
+        if (p.spb <= 8) {                                                                              \
+            if (rng) launch_tiles(RMV ? KERNEL<8, true, RMON> : KERNEL<8, true, 0>, __VA_ARGS__);      \
+            else launch_tiles(RMV ? KERNEL<8, false, RMON> : KERNEL<8, false, 0>, __VA_ARGS__);        \
+        } else {                                                                                       \
+            if (rng) launch_tiles(RMV ? KERNEL<16, true, RMON> : KERNEL<16, true, 0>, __VA_ARGS__);    \
+            else launch_tiles(RMV ? KERNEL<16, false, RMON> : KERNEL<16, false, 0>, __VA_ARGS__);      \
+        }                                                                                              \
+    } while (0)
+
+}  // namespace
+
+// The stepper takes all rays where its own options are asked for (per-lane walks, refilled lanes) and
+// below depth zero, where a beam's bounds do not hold.
+bool stepper_only(const DevParams& p) {
+    return !p.packet || !(p.t_near >= 0.0f) || (p.ray_chunk > 0 && p.refill_lanes > 0);
+}
+
+// Small jobs spread their rays over more wavefronts: with fewer than the GPU holds (4 on each of its
+// 1024 SIMDs) the slowest wavefront is the launch, and a narrower beam has fewer candidates.  Beyond
+// that narrow wavefronts only repeat work.  Drop-in training step with 64 / 32 / 16 / 8 / 4 rays (ms):
+// 64 tiles 2.57 / 1.95 / 1.24 / 0.92 / 0.75, 475 tiles 4.17 / 2.72 / 1.67 / 1.31 / 1.20, 2555 tiles
+// 3.32 / 2.25 / 2.13 / 2.34 / 3.37, 3750 tiles 9.9 / 11.3 / 13.2 / 18.8 / 29.3.
+int rays_per_wave(int64_t num_items) {
+    const int64_t tiles = (num_items + kWave - 1) / kWave;
+    return tiles <= 256 ? 4 : tiles <= 512 ? 8 : tiles <= 1024 ? 16 : tiles <= 3072 ? 32 : 64;
+}
+
+// A block's rays differ by at most eight pixel steps of the image plane along each axis; their unit
+// directions differ by no more, the plane's nearest point being w at a right angle.
+bool view_is_narrow(const rg_camera& cam, int64_t n) {
+    auto dot = [](const float* a, const float* b) { return (double)a[0] * b[0] + (double)a[1] * b[1] + (double)a[2] * b[2]; };
+    const double uw = dot(cam.u, cam.w), vw = dot(cam.v, cam.w), ww = dot(cam.w, cam.w);
+    const double uu = dot(cam.u, cam.u), vv = dot(cam.v, cam.v);
+    if (!(ww > 0.0) || !(uw * uw <= 1e-8 * uu * ww) || !(vw * vw <= 1e-8 * vv * ww)) return false;
+    const double dx = 16.0 * fabs((double)cam.tanx) / cam.width, dy = 16.0 * fabs((double)cam.tany) / cam.height;
+    const double spread = 1.01 * sqrt((dx * dx * uu + dy * dy * vv) / ww);
+    return spread < kTileSpread && (double)n * spread * spread < kTileDensity;
+}
+
+hipError_t launch_forward(const DevScene& sc, const DevParams& p0, const RayJob& job, int hit_depth, float* out_rgb,
+                          float* out_depth, float* out_opacity, DevStats st, hipStream_t s) {
+    if (job.num_rays <= 0) return hipSuccess;
+    DevParams p = p0;
+    p.wide_count = st.c + 12;
+    if (!stepper_only(p)) {
+        RG_TILE_DISPATCH(p.rec_mode == 1, 1, k_tile_forward, sc, p, job, s, hit_depth, out_rgb, out_depth, out_opacity, st);
+        if (!p.wide) return hipGetLastError();
+    } else {
+        p.wide = nullptr;
+    }
+    return launch_forward_steps(sc, p, job, hit_depth, out_rgb, out_depth, out_opacity, st, s);
+}
+
+hipError_t launch_backward(const DevScene& sc, const DevParams& p0, const RayJob& job, int hit_depth,
+                           const float* ray_colors, const float* dLdC, const float* target, int loss_kind,
+                           int count_stats, DevGrad gr, DevStats st, hipStream_t s) {
+    if (job.num_rays <= 0) return hipSuccess;
+    DevParams p = p0;
+    p.wide_count = st.c + 13;
+    if (!stepper_only(p)) {
+        RG_TILE_DISPATCH(p.rec_mode == 2, 2, k_tile_backward, sc, p, job, s, ray_colors, dLdC, target, loss_kind, count_stats,
+                         gr, st);
+        if (!p.wide) return hipGetLastError();
+    } else {
+        p.wide = nullptr;
+    }
+    return launch_backward_steps(sc, p, job, hit_depth, ray_colors, dLdC, target, loss_kind, count_stats, gr, st, s);
+}
+
+}  // namespace rg

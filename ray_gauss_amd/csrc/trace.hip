@@ -383,8 +383,6 @@ __device__ __forceinline__ bool advance_slab(SegState& s, const DevParams& p) {
 
 // ------------------------------------------------------------------ per-ray bodies -----------
 
-// Starts a ray: clears its output and sets up its slab stepper; false when the ray has no slab
-// to process (it misses the scene box, or its first slab is below half an ulp of t).
 // Wavefront-wide step over slabs without hits, after a round in which no lane had one: the lanes
 // stepping through a list (step) advance together over the slabs empty for them, up to the
 // wavefront's earliest possible next hit -- the smallest start (or the segment end) among the list
@@ -411,16 +409,6 @@ __device__ __forceinline__ void jump_empty(SegState& s, const Ray& ray, const De
             ++s.k;
         }
     }
-}
-
-__device__ __forceinline__ bool forward_begin(const DevParams& p, const Ray& ray, RayOut& o, SegState& s) {
-    o.C[0] = o.C[1] = o.C[2] = 0.0f;
-    o.depth = 0.0f;
-    o.T = 1.0f;
-    if (!(ray.tenter < ray.texit)) return false;
-    if (!(add_exact(ray.tenter, p.dt * (float)p.spb) > ray.tenter)) return false;
-    seg_init(s, ray, p);
-    return true;
 }
 
 // One slab of the forward (the reference's raygen loop body, forward/gaussians_aabb.cu:546-606):
@@ -487,7 +475,8 @@ __device__ void forward_ray(const DevScene& sc, const DevParams& p, const Ray& r
                             const float4* __restrict__ rgbv, IList<CAP>& L, int lane, Counters& ctr, RayOut& o,
                             Rec& rc) {
     SegState s;
-    bool alive = forward_begin(p, ray, o, s);
+    bool alive = forward_begin(p, ray, o);
+    seg_init(s, ray, p);
     bool jump = false;
     while (__ballot(alive) != 0ULL) {
         if (jump) jump_empty<CAP>(s, ray, p, L, lane, alive && s.valid && !s.direct, alive, INT_MAX);
@@ -739,19 +728,18 @@ __device__ void backward_wave(const DevScene& sc, const DevParams& p, bool activ
     stage_flush(G, nst, sc, gr, lane, drops);
 }
 
+// Renders the work items below `end` of wavefront `wave`, one per lane.
 template <int SPB, int CAP, bool RNG, int RM>
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(SPB == 8 ? 4 : 3))) k_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items,
-                                                   float* __restrict__ out_rgb, float* __restrict__ out_depth,
-                                                   float* __restrict__ out_opac, DevStats st) {
-    __shared__ IList<CAP> L;
-    const int lane = threadIdx.x;
-    const int64_t nb = gridDim.x;
-    const int64_t item = block_item(blockIdx.x, nb) * kWave + lane;
+__device__ __forceinline__ void forward_items(const DevScene& sc, const DevParams& p, const RayJob& job, int64_t wave,
+                                              int64_t end, IList<CAP>& L, int lane, float* __restrict__ out_rgb,
+                                              float* __restrict__ out_depth, float* __restrict__ out_opac, DevStats st) {
     Counters ctr;
     RayRef q;
-    const int rs = item < num_items ? resolve(job, item, q) : (int)RAY_NONE;
+    const int64_t item = wave_item(p, wave, lane);
+    const bool in = item >= 0 && item < end;
+    const int rs = in ? resolve(job, item, q) : (int)RAY_NONE;
     if (rs == RAY_BAD) {
-        forward_bad<RM>(p, q, st, out_rgb, out_depth, out_opac);
+        forward_bad<RM>(p, q, item, st, out_rgb, out_depth, out_opac);
     } else if (rs == RAY_OK) {
         const rg_camera cam = job.cams[q.view];
         unsigned int seed = RNG ? tea4(p.iteration, (unsigned int)q.pixel) : 0u;
@@ -759,13 +747,50 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(SPB 
         RayOut o;
         Rec rc;
         if constexpr (RM == 1) {
-            rc.w = rec_base(p.rec, q.out, p.rec_words);
+            rc.w = rec_region(p, wave) + 8 * lane;
+            rc.stride = 8 * p.rays_per_wave;
             rc.end = p.rec_words;
         }
         forward_ray<SPB, CAP, RNG, RM>(sc, p, ray, seed, sc.rgb + (size_t)q.view * sc.n, L, lane, ctr, o, rc);
-        forward_finish<RM>(p, q, o, rc, ctr, out_rgb, out_depth, out_opac);
+        if constexpr (RM == 1) ctr.rec_words += rc.pos;
+        forward_finish<RM>(p, q, item, o, rc, ctr, out_rgb, out_depth, out_opac);
+    } else if (RM == 1 && in) {
+        p.rec_id[item] = make_int2(-1, -1);  // padding: no records
     }
     flush_counters(ctr, st);
+}
+
+// The wavefront of each block, or (p.wide) the wavefronts that the tile kernel left to the stepper.
+template <int SPB, int CAP, bool RNG, int RM>
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(SPB == 8 ? 4 : 3))) k_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items,
+                                                   float* __restrict__ out_rgb, float* __restrict__ out_depth,
+                                                   float* __restrict__ out_opac, DevStats st) {
+    __shared__ IList<CAP> L;
+    const int lane = threadIdx.x;
+    const int64_t nb = p.wide ? (int64_t)*p.wide_count : 1;
+    for (int64_t i = p.wide ? blockIdx.x : 0; i < nb; i += gridDim.x)
+        forward_items<SPB, CAP, RNG, RM>(sc, p, job, p.wide ? p.wide[i].x : block_item(blockIdx.x, gridDim.x), num_items, L,
+                                         lane, out_rgb, out_depth, out_opac, st);
+}
+
+// Backward of the work items below `end` of wavefront `wave`, one per lane; lanes: those that take part
+// (the rest were done by the tile kernel, with the loss and the bad rays of all of them).
+template <int SPB, int CAP, bool RNG, int RM>
+__device__ __forceinline__ void backward_items(const DevScene& sc, const DevParams& p, const RayJob& job, int64_t wave,
+                                               int64_t end, unsigned long long lanes, IList<CAP>& L, GradStage& G, int lane,
+                                               const float* __restrict__ ray_colors, const float* __restrict__ dLdC,
+                                               const float* __restrict__ target, int loss_kind, int count_stats,
+                                               const DevGrad& gr, DevStats st) {
+    Counters ctr;
+    float loss = 0.0f;
+    BwdRay b;
+    const int64_t item = wave_item(p, wave, lane);
+    if (item >= 0 && item < end && ((lanes >> lane) & 1ULL))
+        backward_setup<RNG, RM>(sc, p, job, wave, lane, item, ray_colors, dLdC, target, loss_kind, st, b, loss);
+    backward_wave<SPB, CAP, RNG, RM>(sc, p, b.active, b.ray, b.seed, sc.rgb + (size_t)b.view * sc.n, b.Cf, b.dL, L, G,
+                                     lane, gr, b.view, ctr, b.rc, st.c + C_DROP);
+    if (count_stats) flush_counters(ctr, st);
+    if (target && !p.wide) add_loss(p, loss, lane, st);
 }
 
 // Backward over a batch.  dL/dC comes from dLdC, or -- with target != nullptr -- from the
@@ -780,18 +805,17 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(3)))
     __shared__ IList<CAP> L;
     __shared__ GradStage G;
     const int lane = threadIdx.x;
-    const int64_t nb = gridDim.x;
-    const int64_t item = block_item(blockIdx.x, nb) * kWave + lane;
-    Counters ctr;
-    BwdRay b;
-    float loss = 0.0f;
-    if (item < num_items) backward_setup<RNG, RM>(sc, p, job, item, ray_colors, dLdC, target, loss_kind, st, b, loss);
-    backward_wave<SPB, CAP, RNG, RM>(sc, p, b.active, b.ray, b.seed, sc.rgb + (size_t)b.view * sc.n, b.Cf, b.dL, L, G,
-                                     lane, gr, b.view, ctr, b.rc, st.c + C_DROP);
-    if (count_stats) flush_counters(ctr, st);
-    if (target) {
-        const float ls = wave_sum64(loss);
-        if (lane == 0 && ls != 0.0f) atomicAdd(reinterpret_cast<float*>(&st.c[C_LOSS]), ls);
+    const int64_t nb = p.wide ? (int64_t)*p.wide_count : 1;
+    for (int64_t i = p.wide ? blockIdx.x : 0; i < nb; i += gridDim.x) {
+        int64_t wave = block_item(blockIdx.x, gridDim.x);
+        unsigned long long lanes = ~0ULL;
+        if (p.wide) {
+            const int4 w = p.wide[i];
+            wave = w.x;
+            lanes = (unsigned long long)(unsigned int)w.y | (unsigned long long)(unsigned int)w.z << 32;
+        }
+        backward_items<SPB, CAP, RNG, RM>(sc, p, job, wave, num_items, lanes, L, G, lane, ray_colors, dLdC, target,
+                                          loss_kind, count_stats, gr, st);
     }
 }
 
@@ -805,30 +829,9 @@ k_forward_pq(DevScene sc, DevParams p, RayJob job, int64_t num_items, float* __r
     const int lane = threadIdx.x;
     int64_t lo = 0, hi = 0;
     unsigned int spent = 0u;
-    while (take_chunk(p, num_items, blockIdx.x & 7, lo, hi, spent)) {
-        for (int64_t base = lo; base < hi; base += kWave) {
-            const int64_t item = base + lane;
-            Counters ctr;  // flushed per tile: no per-lane state lives across tiles
-            RayRef q;
-            const int rs = item < hi ? resolve(job, item, q) : (int)RAY_NONE;
-            if (rs == RAY_BAD) {
-                forward_bad<RM>(p, q, st, out_rgb, out_depth, out_opac);
-            } else if (rs == RAY_OK) {
-                const rg_camera cam = job.cams[q.view];
-                unsigned int seed = RNG ? tea4(p.iteration, (unsigned int)q.pixel) : 0u;
-                const Ray ray = make_ray(cam, q.pixel, sc.box, p.t_near, p.t_far, RNG ? p.jitter : 0, &seed);
-                RayOut o;
-                Rec rc;
-                if constexpr (RM == 1) {
-                    rc.w = rec_base(p.rec, q.out, p.rec_words);
-                    rc.end = p.rec_words;
-                }
-                forward_ray<SPB, CAP, RNG, RM>(sc, p, ray, seed, sc.rgb + (size_t)q.view * sc.n, L, lane, ctr, o, rc);
-                forward_finish<RM>(p, q, o, rc, ctr, out_rgb, out_depth, out_opac);
-            }
-            flush_counters(ctr, st);
-        }
-    }
+    while (take_chunk(p, num_items, blockIdx.x & 7, lo, hi, spent))
+        for (int64_t base = lo; base < hi; base += kWave)  // counters are flushed per tile
+            forward_items<SPB, CAP, RNG, RM>(sc, p, job, base / kWave, hi, L, lane, out_rgb, out_depth, out_opac, st);
 }
 
 // Persistent forward that refills idle lanes (refill_lanes = k, 0 < k < 64): as soon as k lanes
@@ -864,6 +867,7 @@ k_forward_refill(DevScene sc, DevParams p, RayJob job, int64_t num_items, float*
     o.depth = 0.0f;
     o.T = 1.0f;
     Rec rc;
+    int64_t item = 0;
     while (true) {
         if (more && __popcll(__ballot(!alive)) >= refill) {
             // hand the next items to the idle lanes, taking chunks from the queues as needed
@@ -879,21 +883,23 @@ k_forward_refill(DevScene sc, DevParams p, RayJob job, int64_t num_items, float*
                 const int rank = lanes_below(nm);
                 if (need && rank < avail) {
                     need = false;
-                    const int rs = resolve(job, clo + rank, q);
+                    item = clo + rank;
+                    const int rs = resolve(job, item, q);
                     if (rs == RAY_OK) {
                         const rg_camera cam = job.cams[q.view];
                         seed = RNG ? tea4(p.iteration, (unsigned int)q.pixel) : 0u;
                         ray = make_ray(cam, q.pixel, sc.box, p.t_near, p.t_far, RNG ? p.jitter : 0, &seed);
                         if constexpr (RM == 1) {
-                            rc.w = rec_base(p.rec, q.out, p.rec_words);
+                            rc.w = rec_region(p, item / kWave) + 8 * (item % kWave);
                             rc.pos = 0;
                             rc.end = p.rec_words;
                             rc.full = false;
                         }
-                        alive = forward_begin(p, ray, o, s);
-                        if (!alive) forward_finish<RM>(p, q, o, rc, ctr, out_rgb, out_depth, out_opac);
+                        alive = forward_begin(p, ray, o);
+                        seg_init(s, ray, p);
+                        if (!alive) forward_finish<RM>(p, q, item, o, rc, ctr, out_rgb, out_depth, out_opac);
                     } else if (rs == RAY_BAD) {
-                        forward_bad<RM>(p, q, st, out_rgb, out_depth, out_opac);
+                        forward_bad<RM>(p, q, item, st, out_rgb, out_depth, out_opac);
                     }
                 }
                 clo += min((int64_t)__popcll(nm), avail);
@@ -905,7 +911,8 @@ k_forward_refill(DevScene sc, DevParams p, RayJob job, int64_t num_items, float*
         }
         if (alive && !forward_step<SPB, CAP, RNG, RM>(sc, p, ray, seed, sc.rgb + (size_t)q.view * sc.n, L, lane, ctr, o,
                                                       rc, s)) {
-            forward_finish<RM>(p, q, o, rc, ctr, out_rgb, out_depth, out_opac);
+            if constexpr (RM == 1) ctr.rec_words += rc.pos;
+            forward_finish<RM>(p, q, item, o, rc, ctr, out_rgb, out_depth, out_opac);
             alive = false;
         }
     }
@@ -925,22 +932,10 @@ k_backward_pq(DevScene sc, DevParams p, RayJob job, int64_t num_items, const flo
     const int xcd = blockIdx.x & 7;
     int64_t lo = 0, hi = 0;
     unsigned int spent = 0u;
-    while (take_chunk(p, num_items, xcd, lo, hi, spent)) {
-        for (int64_t base = lo; base < hi; base += kWave) {
-            const int64_t item = base + lane;
-            Counters ctr;  // flushed per tile: no per-lane state lives across tiles
-            float loss = 0.0f;
-            BwdRay b;
-            if (item < hi) backward_setup<RNG, RM>(sc, p, job, item, ray_colors, dLdC, target, loss_kind, st, b, loss);
-            backward_wave<SPB, CAP, RNG, RM>(sc, p, b.active, b.ray, b.seed, sc.rgb + (size_t)b.view * sc.n, b.Cf, b.dL,
-                                             L, G, lane, gr, b.view, ctr, b.rc, st.c + C_DROP);
-            if (count_stats) flush_counters(ctr, st);
-            if (target) {
-                const float ls = wave_sum64(loss);
-                if (lane == 0 && ls != 0.0f) atomicAdd(reinterpret_cast<float*>(&st.c[C_LOSS]), ls);
-            }
-        }
-    }
+    while (take_chunk(p, num_items, xcd, lo, hi, spent))
+        for (int64_t base = lo; base < hi; base += kWave)  // counters are flushed per tile
+            backward_items<SPB, CAP, RNG, RM>(sc, p, job, base / kWave, hi, ~0ULL, L, G, lane, ray_colors, dLdC, target,
+                                              loss_kind, count_stats, gr, st);
 }
 
 __global__ void k_reset_queue(unsigned long long* q) {
@@ -1008,6 +1003,11 @@ __global__ void k_reset_counters(unsigned long long* c) {
     if (threadIdx.x < 16) c[threadIdx.x] = 0;
 }
 
+__global__ void k_loss_out(const unsigned long long* c, float* out) {
+    if (threadIdx.x == 0)
+        *out = (float)((double)*reinterpret_cast<const float*>(&c[C_LOSS]) + *reinterpret_cast<const double*>(&c[C_LOSS64]));
+}
+
 }  // namespace
 
 // In the implicit single-view mode RayJob.num_rays carries the padded 8x8-tile item count.
@@ -1051,6 +1051,11 @@ __global__ void k_reset_counters(unsigned long long* c) {
 #define RG_DISPATCH(SPBV, CAPV, RNGV, RMV, ...) RG_DISPATCH_ANY(RG_DISPATCH_CAP, SPBV, CAPV, RNGV, RMV, 2, __VA_ARGS__)
 #define RG_DISPATCH_FWD(SPBV, CAPV, RNGV, RMV, ...) \
     RG_DISPATCH_ANY(RG_DISPATCH_CAP6, SPBV, CAPV, RNGV, RMV, 1, __VA_ARGS__)
+
+hipError_t launch_loss_out(DevStats st, float* out, hipStream_t s) {
+    hipLaunchKernelGGL(k_loss_out, dim3(1), dim3(64), 0, s, st.c, out);
+    return hipGetLastError();
+}
 
 hipError_t launch_reset_counters(DevStats st, hipStream_t s) {
     hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, st.c);
@@ -1097,43 +1102,46 @@ static void launch_persistent(K kernel, int64_t items, const DevParams& p, hipSt
         else launch_persistent(KERNEL<SPBC, 32, RNGC, RMC>, __VA_ARGS__);                                           \
     } while (0)
 
-hipError_t launch_forward(const DevScene& sc, const DevParams& p, const RayJob& job, int hit_depth, float* out_rgb,
-                          float* out_depth, float* out_opacity, DevStats st, hipStream_t s) {
+// Blocks of a stepper launch: one per wavefront, or as many as take the tile kernel's leftovers in
+// turn (their number is known on the device alone; none is the common case).
+static unsigned int step_blocks(const DevParams& p, int64_t items) {
+    const int64_t nb = num_waves(p, items);
+    return (unsigned int)(p.wide ? (nb < kWideBlocks ? nb : kWideBlocks) : ((nb + 7) / 8) * 8);
+}
+
+hipError_t launch_forward_steps(const DevScene& sc, const DevParams& p, const RayJob& job, int hit_depth, float* out_rgb,
+                                float* out_depth, float* out_opacity, DevStats st, hipStream_t s) {
     const int64_t items = job.num_rays;  // already the padded item count in implicit mode
     if (items <= 0) return hipSuccess;
     const bool rng = p.jitter || p.rnd_sample;
-    if (p.ray_chunk > 0 && p.refill_lanes > 0 && p.refill_lanes < kWave) {
+    if (p.ray_chunk > 0 && !p.wide && p.refill_lanes > 0 && p.refill_lanes < kWave) {
         RG_DISPATCH_ANY(RG_PQ_CAP6, p.spb <= 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 1, 1, k_forward_refill, items, p,
                         s, sc, p, job, items, out_rgb, out_depth, out_opacity, st);
         return hipGetLastError();
     }
-    if (p.ray_chunk > 0) {
+    if (p.ray_chunk > 0 && !p.wide) {
         RG_DISPATCH_ANY(RG_PQ_CAP6, p.spb <= 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 1, 1, k_forward_pq, items, p, s,
                         sc, p, job, items, out_rgb, out_depth, out_opacity, st);
         return hipGetLastError();
     }
-    const int64_t nb = (items + kWave - 1) / kWave;
-    const int64_t nbp = ((nb + 7) / 8) * 8;
-    RG_DISPATCH_FWD(p.spb <= 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 1, k_forward, dim3((unsigned)nbp), dim3(kWave), 0, s, sc, p, job,
-                items, out_rgb, out_depth, out_opacity, st);
+    RG_DISPATCH_FWD(p.spb <= 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 1, k_forward, dim3(step_blocks(p, items)), dim3(kWave),
+                    0, s, sc, p, job, items, out_rgb, out_depth, out_opacity, st);
     return hipGetLastError();
 }
 
-hipError_t launch_backward(const DevScene& sc, const DevParams& p, const RayJob& job, int hit_depth,
-                           const float* ray_colors, const float* dLdC, const float* target, int loss_kind,
-                           int count_stats, DevGrad gr, DevStats st, hipStream_t s) {
+hipError_t launch_backward_steps(const DevScene& sc, const DevParams& p, const RayJob& job, int hit_depth,
+                                 const float* ray_colors, const float* dLdC, const float* target, int loss_kind,
+                                 int count_stats, DevGrad gr, DevStats st, hipStream_t s) {
     const int64_t items = job.num_rays;
     if (items <= 0) return hipSuccess;
     const bool rng = p.jitter || p.rnd_sample;
-    if (p.ray_chunk > 0) {
+    if (p.ray_chunk > 0 && !p.wide) {
         RG_DISPATCH_ANY(RG_PQ_CAP, p.spb <= 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 2, 2, k_backward_pq, items, p, s,
                         sc, p, job, items, ray_colors, dLdC, target, loss_kind, count_stats, gr, st);
         return hipGetLastError();
     }
-    const int64_t nb = (items + kWave - 1) / kWave;
-    const int64_t nbp = ((nb + 7) / 8) * 8;
-    RG_DISPATCH(p.spb <= 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 2, k_backward, dim3((unsigned)nbp), dim3(kWave), 0, s, sc, p, job,
-                items, ray_colors, dLdC, target, loss_kind, count_stats, gr, st);
+    RG_DISPATCH(p.spb <= 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 2, k_backward, dim3(step_blocks(p, items)), dim3(kWave), 0, s,
+                sc, p, job, items, ray_colors, dLdC, target, loss_kind, count_stats, gr, st);
     return hipGetLastError();
 }
 

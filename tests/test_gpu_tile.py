@@ -1,0 +1,101 @@
+"""Tiles (wavefronts of rays marching as one beam) against the per-ray slab stepper, which
+``packet=False`` selects: the images are bit-identical (the same hits in the same order) and the
+gradients equal up to the order of atomic sums, with replayed records, records that end early and
+none, over the shapes where the two could part: ragged tiles, several views in a wavefront, beams
+too wide for a tile, rounds with more candidates than the list holds, a camera inside the scene."""
+
+import numpy as np
+import pytest
+import torch
+
+from ray_gauss_amd import scenes
+from ray_gauss_amd.batch import tile_order_pixels
+from ray_gauss_amd.cameras import look_at_camera, orbit_eye
+from ray_gauss_amd.caster import TuneConfig
+
+from gpu_helpers import max_rel, prepared_caster
+
+pytestmark = pytest.mark.gpu
+
+
+def _compare(scene, params, cams, dev, rv, rp, words):
+    rv = torch.as_tensor(np.asarray(rv, np.int32)).to(dev)
+    rp = torch.as_tensor(np.asarray(rp, np.int32)).to(dev)
+    gen = torch.Generator(device=dev).manual_seed(3)
+    dL = torch.randn((rv.shape[0], 3), generator=gen, device=dev)
+    out = {}
+    for packet in (False, True):
+        rc, _ = prepared_caster(scene, params, cams, dev, TuneConfig(packet=packet, replay_words=words))
+        rgb, depth, opac = rc.forward_batch(rv, rp, depth=True, opacity=True)
+        st = rc.stats()
+        rc.backward_batch(rv, rp, rgb, dL, rc.last_token)
+        assert rc.stats()["dropped"] == 0
+        g = {k: v.cpu().numpy() for k, v in rc.finish_grads().items() if v is not None}
+        out[packet] = (rgb, depth, opac, st, g)
+    a, b = out[False], out[True]
+    for i in range(3):
+        assert torch.equal(a[i], b[i]), i
+    assert a[3]["slab_hits"] == b[3]["slab_hits"] and a[3]["pairs"] == b[3]["pairs"]
+    for k, v in a[4].items():
+        assert max_rel(b[4][k], v) <= 1e-5, k
+    return b[3]
+
+
+def _view(w, h, radius=3.0, fov=40.0, az=30.0):
+    return look_at_camera(orbit_eye(radius, az, 20.0), width=w, height=h, fovx_deg=fov).launch_record()
+
+
+@pytest.mark.parametrize("words", [0, 8, 1536])
+@pytest.mark.parametrize("w,h", [(1, 1), (7, 9), (64, 1), (65, 17)])
+def test_ragged_tiles(gpu_device, w, h, words):
+    sc = scenes.scene_uniform(3000, seed=w + h)
+    prm = scenes.RenderParams(dt=0.01, t_eps=1e-4, white_background=True)
+    cam = _view(w, h)
+    st = _compare(sc, prm, [cam], gpu_device, np.zeros(w * h), np.arange(w * h), words)
+    assert st["slab_hits"] > 0
+
+
+@pytest.mark.parametrize("views,fov", [(3, 2.0), (6, 2.0), (2, 120.0)])
+def test_wavefronts_of_several_views_and_wide_beams(gpu_device, views, fov):
+    """Rays of three narrow views in turn march as three beams of one wavefront; six views, or views
+    whose 64 rays spread over 120 degrees, go to the slab stepper."""
+    sc = scenes.scene_uniform(3000, seed=views)
+    prm = scenes.RenderParams(dt=0.01, t_eps=1e-4)
+    cams = [_view(16, 16, fov=fov, az=50.0 * v) for v in range(views)]
+    i = np.arange(16 * 16 * views)
+    st = _compare(sc, prm, cams, gpu_device, i % views, np.random.default_rng(0).permutation(256)[i // views], 64)
+    assert st["slab_hits"] > 0
+
+
+@pytest.mark.parametrize("words", [0, 16, 1536])
+def test_wavefronts_across_rows_of_tiles(gpu_device, words):
+    """A large list of 8x8 tiles of a view whose width is no multiple of eight: wavefronts of 64 rays
+    that hold the end of a row of tiles and the start of the next march as two beams of one view."""
+    sc = scenes.scene_uniform(2000, seed=4)
+    prm = scenes.RenderParams(dt=0.02, t_eps=1e-4)
+    cam = _view(611, 401)
+    rp = tile_order_pixels(611, 401)
+    st = _compare(sc, prm, [cam], gpu_device, np.zeros(len(rp)), rp, words)
+    assert st["slab_hits"] > 0
+
+
+@pytest.mark.parametrize("words", [0, 64, 4096])
+def test_rounds_with_more_candidates_than_the_list(gpu_device, words):
+    """Large overlapping Gaussians: single slabs hold more candidates than a tile's list, so their
+    rounds walk the tree and have more events than one batch."""
+    sc = scenes.scene_uniform(1200, seed=5, log_scale_mean=-1.2)
+    sc.densities[:] = 0.11 + 0.002 * np.arange(1200, dtype=np.float32) / 1200
+    sc.scales[:] *= 4.0
+    prm = scenes.RenderParams(dt=0.02, t_eps=1e-4)
+    st = _compare(sc, prm, [_view(9, 9)], gpu_device, np.zeros(81), np.arange(81), words)
+    assert st["fallback_slabs"] > 0 and st["slab_hits"] > 300 * 64
+
+
+@pytest.mark.parametrize("t_near", [0.0, 0.7, -0.5])
+def test_camera_inside_the_scene(gpu_device, t_near):
+    """Rays that start inside the scene (and inside ellipsoids); depths below zero are left to the
+    slab stepper."""
+    sc = scenes.scene_uniform(3000, seed=11, log_scale_mean=-2.5)
+    prm = scenes.RenderParams(dt=0.01, t_eps=1e-4, t_near=t_near, t_far=2.5)
+    st = _compare(sc, prm, [_view(24, 16, radius=0.3)], gpu_device, np.zeros(384), np.arange(384), 512)
+    assert st["slab_hits"] > 0
