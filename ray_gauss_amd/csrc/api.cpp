@@ -52,6 +52,12 @@ struct rg_handle {
     // wavefronts left to the slab stepper
     int4* wide = nullptr;
     int64_t wide_cap = 0;
+    // order of a job's wavefronts, their weight buckets, the grid of counts behind them
+    int* order = nullptr;
+    unsigned char* order_bucket = nullptr;
+    int64_t order_cap = 0;
+    unsigned int* order_grid = nullptr;
+    int64_t order_views = 0;
     uint64_t tokens_issued = 0;
     struct {
         bool valid = false;
@@ -249,6 +255,9 @@ rg::DevParams dev_params(const rg_handle* h) {
     p.rays_per_wave = 64;
     p.wide = nullptr;
     p.wide_count = nullptr;
+    p.order = nullptr;
+    p.order_bucket = nullptr;
+    p.order_grid = nullptr;
     return p;
 }
 
@@ -308,13 +317,13 @@ int rg_create(rg_handle** out, const rg_config* cfg) {
         return rc;
     }
     h->cfg = *cfg;
-    if ((rc = dalloc(h, &h->box, 8)) || (rc = dalloc(h, &h->counters, 16)) || (rc = dalloc(h, &h->queue, 16))) {
+    if ((rc = dalloc(h, &h->box, 8)) || (rc = dalloc(h, &h->counters, rg::kCounters)) || (rc = dalloc(h, &h->queue, 16))) {
         if (h->box) hipFree(h->box);
         if (h->counters) hipFree(h->counters);
         delete h;
         return rc;
     }
-    if (hipMemset(h->counters, 0, 16 * sizeof(unsigned long long)) != hipSuccess) {
+    if (hipMemset(h->counters, 0, rg::kCounters * sizeof(unsigned long long)) != hipSuccess) {
         delete h;
         return RG_ERR_HIP;
     }
@@ -328,7 +337,7 @@ int rg_destroy(rg_handle* h) {
                     h->bvh.vals[0], h->bvh.vals[1], h->bvh.hist, h->bvh.perm, h->bvh.iperm, h->bvh.nodes,
                     h->bvh.parent, h->bvh.right, h->bvh.counter, h->bvh.leaf_node, h->bvh.k_parent,
                     h->bvh.k_left, h->bvh.k_right, h->bvh.k_first, h->bvh.k_last, h->cams, h->rgb, h->drgb,
-                    h->train_rgb, h->rec, h->rec_len, h->rec_id, h->wide, h->bvh.sah_prims[0], h->bvh.sah_prims[1],
+                    h->train_rgb, h->rec, h->rec_len, h->rec_id, h->wide, h->order, h->order_bucket, h->order_grid, h->bvh.sah_prims[0], h->bvh.sah_prims[1],
                     h->bvh.sah_tasks[0], h->bvh.sah_tasks[1], h->bvh.sah_ctr, h->bvh.k_pre};
     for (void* p : ptrs)
         if (p) hipFree(p);
@@ -429,15 +438,33 @@ int rg_set_view_colors(rg_handle* h, int32_t view, const float* rgb, void* strea
     return RG_OK;
 }
 
-// Wavefronts of the job: how many rays each holds, and room for those that the tile kernels leave to
-// the slab stepper.  A whole view whose 8x8 blocks are all narrow beams leaves none.
-static int plan_waves(rg_handle* h, const rg::RayJob& j, rg::DevParams& p) {
+// Wavefronts of the job: how many rays each holds, the order they are taken in, and room for those
+// that the tile kernels leave to the slab stepper.  A whole view whose 8x8 blocks are all narrow
+// beams leaves none.
+static int plan_waves(rg_handle* h, const rg::RayJob& j, rg::DevParams& p, hipStream_t s) {
     if (rg::stepper_only(p)) return RG_OK;
     p.rays_per_wave = rg::rays_per_wave(j.num_rays);
-    if (!j.ray_view && !j.pixels && rg::view_is_narrow(h->host_cams[j.view], h->n)) return RG_OK;
     const int64_t waves = (j.num_rays + 63) / 64 * (64 / p.rays_per_wave);
+    const int views = j.ray_view ? j.num_views : 1;
+    int rc;
+    if (waves >= rg::kOrderMin && views <= 4096) {
+        if (waves > h->order_cap) {
+            h->order_cap = 0;
+            if ((rc = dalloc(h, &h->order, waves)) || (rc = dalloc(h, &h->order_bucket, waves))) return rc;
+            h->order_cap = waves;
+        }
+        if (views > h->order_views) {
+            h->order_views = 0;
+            if ((rc = dalloc(h, &h->order_grid, rg::order_grid_cells(views)))) return rc;
+            HIPCHK(h, rg::launch_zero(reinterpret_cast<float*>(h->order_grid), rg::order_grid_cells(views), s));
+            h->order_views = views;
+        }
+        p.order = h->order;
+        p.order_bucket = h->order_bucket;
+        p.order_grid = h->order_grid;
+    }
+    if (!j.ray_view && !j.pixels && rg::view_is_narrow(h->host_cams[j.view], h->n)) return RG_OK;
     if (waves > h->wide_cap) {
-        int rc;
         h->wide_cap = 0;
         if ((rc = dalloc(h, &h->wide, waves))) return rc;
         h->wide_cap = waves;
@@ -508,7 +535,7 @@ int rg_forward(rg_handle* h, int32_t view, int64_t num_rays, const int32_t* pixe
     HIPCHK(h, rg::launch_reset_counters(dev_stats(h), s));
     const rg::RayJob job = single_job(h, view, num_rays, pixels);
     rg::DevParams p = dev_params(h);
-    if ((rc = plan_waves(h, job, p))) return rc;
+    if ((rc = plan_waves(h, job, p, s))) return rc;
     const uint64_t token = rec_forward(h, job, p);
     HIPCHK(h, rg::launch_forward(dev_scene(h), p, job, fwd_depth(h), out_rgb, out_depth, out_opacity, dev_stats(h), s));
     if (out_token) *out_token = token;
@@ -528,7 +555,7 @@ int rg_backward(rg_handle* h, int32_t view, int64_t num_rays, const int32_t* pix
     const rg::RayJob job = single_job(h, view, num_rays, pixels);
     const rg::DevGrad gr = dev_grad(h);
     rg::DevParams p = dev_params(h);
-    if ((rc = plan_waves(h, job, p))) return rc;
+    if ((rc = plan_waves(h, job, p, s))) return rc;
     rec_backward(h, job, replay_token, p);
     p.ray_chunk = h->cfg.bwd_ray_chunk;
     HIPCHK(h, rg::launch_backward(dev_scene(h), p, job, h->cfg.hit_depth, ray_colors, dL_dC, nullptr, 0, 1, gr,
@@ -562,7 +589,7 @@ int rg_forward_batch(rg_handle* h, const rg_ray_batch* b, float* out_rgb, float*
     hipStream_t s = static_cast<hipStream_t>(stream);
     HIPCHK(h, rg::launch_reset_counters(dev_stats(h), s));
     rg::DevParams p = dev_params(h);
-    if ((rc = plan_waves(h, j, p))) return rc;
+    if ((rc = plan_waves(h, j, p, s))) return rc;
     const uint64_t token = rec_forward(h, j, p);
     HIPCHK(h, rg::launch_forward(dev_scene(h), p, j, fwd_depth(h), out_rgb, out_depth, out_opacity, dev_stats(h), s));
     if (out_token) *out_token = token;
@@ -579,7 +606,7 @@ int rg_backward_batch(rg_handle* h, const rg_ray_batch* b, const float* ray_colo
     HIPCHK(h, rg::launch_reset_counters(dev_stats(h), s));
     const rg::DevGrad gr = dev_grad(h);
     rg::DevParams p = dev_params(h);
-    if ((rc = plan_waves(h, j, p))) return rc;
+    if ((rc = plan_waves(h, j, p, s))) return rc;
     rec_backward(h, j, replay_token, p);
     p.ray_chunk = h->cfg.bwd_ray_chunk;
     HIPCHK(h, rg::launch_backward(dev_scene(h), p, j, h->cfg.hit_depth, ray_colors, dL_dC, nullptr, 0, 1, gr,
@@ -607,11 +634,11 @@ int rg_train_batch(rg_handle* h, const rg_ray_batch* b, const float* target, int
     }
     const rg::DevScene sc = dev_scene(h);
     rg::DevParams p = dev_params(h);
-    if ((rc = plan_waves(h, j, p))) return rc;
+    if ((rc = plan_waves(h, j, p, s))) return rc;
     const uint64_t token = rec_forward(h, j, p);
     HIPCHK(h, rg::launch_forward(sc, p, j, fwd_depth(h), rgb, nullptr, nullptr, dev_stats(h), s));
     p = dev_params(h);
-    if ((rc = plan_waves(h, j, p))) return rc;
+    if ((rc = plan_waves(h, j, p, s))) return rc;
     rec_backward(h, j, token, p);
     p.ray_chunk = h->cfg.bwd_ray_chunk;
     HIPCHK(h, rg::launch_backward(sc, p, j, h->cfg.hit_depth, rgb, nullptr, target, loss_kind, 0, dev_grad(h),

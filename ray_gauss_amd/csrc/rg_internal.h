@@ -78,6 +78,11 @@ struct DevParams {
     // (wavefront, lanes: low, high word, 0), and their number (nullptr: none)
     int4* wide;
     unsigned long long* wide_count;
+    // order in which the tile kernels' blocks take the wavefronts (nullptr: their own), with the weight
+    // bucket of each and the grid of counts they come from (zero between jobs)
+    int* order;
+    unsigned char* order_bucket;
+    unsigned int* order_grid;
 };
 
 // Gradient accumulators (device-scope atomic adds; the finish kernel reads and clears them).
@@ -87,10 +92,12 @@ struct DevGrad {
     int num_views;  // rows of drgb
 };
 
-// Counters (device, 16): 0 K, 1 P, 2 overflow slabs, 3 fallback slabs, 4 gathers, 6 loss (float),
+// Counters (device, kCounters): 0 K, 1 P, 2 overflow slabs, 3 fallback slabs, 4 gathers, 6 loss (float),
 // 7 debug scratch, 8 record words, 9 truncated records, 10 dropped by bounds checks, 11 rays with
 // an out-of-range view or pixel, 12 / 13 wavefronts left to the stepper by the forward / backward,
-// 14 loss of narrow wavefronts (double), 15 unused
+// 14 loss of narrow wavefronts (double), 15 unused, 16..47 / 48..79 sizes and cursors of the order's
+// buckets in the forward / backward
+constexpr int kCounters = 80;
 struct DevStats {
     unsigned long long* c;
 };
@@ -237,6 +244,10 @@ hipError_t launch_debug_hits(const DevScene& sc, const DevParams& p, const RayJo
 bool stepper_only(const DevParams& p);
 // Rays per wavefront for a job of num_items work items.
 int rays_per_wave(int64_t num_items);
+// Jobs of fewer wavefronts than this keep their own order (all of them start at once).
+constexpr int64_t kOrderMin = 2048;
+// Cells of DevParams::order_grid for jobs over `views` views.
+int64_t order_grid_cells(int views);
 // Whether every 8x8 pixel block of the view (jittered or not) is a beam that the tile kernels take.
 bool view_is_narrow(const rg_camera& cam, int64_t n);
 // Forward and backward of a job: tiles, then (p.wide) what they leave to the slab stepper.

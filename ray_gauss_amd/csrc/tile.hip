@@ -450,14 +450,111 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
     stage_flush(G, nst, sc, gr, lane, drops);
 }
 
+// ------------------------------------------------------------------ order --------------------
+//
+// The wavefronts of a job cost from a few to hundreds of times their mean (a blob's core against its
+// rim), and a launch lasts as long as its dearest ones, which sit next to each other in the image:
+// on one view of 100k Gaussians the 10000 wavefronts of a forward took 530 us on average and the
+// last of them 6 ms, 5.65 ms for what 4096 resident wavefronts could do in 1.3.  So the dear ones
+// start first.  What a wavefront costs is estimated in the forward from the Gaussians' means around
+// its pixels, counted on a coarse grid of each view, and known in the backward from its record.
+constexpr int kGrid = 128;              // cells of a view along each axis
+constexpr int kSplats = 1 << 20;        // Gaussians counted at most (every k-th of more)
+constexpr int kOrderBuckets = 32;       // half octaves of the weight
+constexpr int kOrderBlock = 1024;
+
+__global__ void __launch_bounds__(256) k_tile_splat(int n, int stride, const float4* __restrict__ geo,
+                                                    const rg_camera* __restrict__ cams, int first_view,
+                                                    unsigned int* __restrict__ grid) {
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * stride;
+    if (i >= n) return;
+    const rg_camera& c = cams[first_view + blockIdx.y];
+    const float4 g = geo[4 * i];
+    const float dx = g.x - c.eye[0], dy = g.y - c.eye[1], dz = g.z - c.eye[2];
+    const float z = dx * c.w[0] + dy * c.w[1] + dz * c.w[2];
+    const float x = (dx * c.u[0] + dy * c.u[1] + dz * c.u[2]) / (c.tanx * z);
+    const float y = (dx * c.v[0] + dy * c.v[1] + dz * c.v[2]) / (c.tany * z);
+    if (!(z > 0.0f) || !(fabsf(x) < 1.0f) || !(fabsf(y) < 1.0f)) return;
+    const int cx = min((int)((x + 1.0f) * (0.5f * kGrid)), kGrid - 1), cy = min((int)((y + 1.0f) * (0.5f * kGrid)), kGrid - 1);
+    atomicAdd(&grid[((int)blockIdx.y * kGrid + cy) * kGrid + cx], 1u);
+}
+
+// Bucket of each wavefront's weight: the count of the 3x3 cells around its first ray, or (grid ==
+// nullptr) the cells of its record.
+__global__ void __launch_bounds__(256) k_tile_weight(DevParams p, RayJob job, int64_t num_items, int first_view, int waves,
+                                                     const unsigned int* __restrict__ grid,
+                                                     unsigned char* __restrict__ bucket, int* __restrict__ hist) {
+    __shared__ int cnt[kOrderBuckets];
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (threadIdx.x < kOrderBuckets) cnt[threadIdx.x] = 0;
+    __syncthreads();
+    unsigned int w = 0u;
+    RayRef q;
+    const int64_t item = i < waves ? wave_item(p, i, 0) : num_items;
+    if (item < num_items && resolve(job, item, q) == RAY_OK) {
+        if (grid) {
+            const rg_camera& c = job.cams[q.view];
+            const int cx = (int)((int64_t)(q.pixel % c.width) * kGrid / c.width);
+            const int cy = (int)((int64_t)(q.pixel / c.width) * kGrid / c.height);
+            const unsigned int* g = grid + (int64_t)(q.view - first_view) * kGrid * kGrid;
+            for (int y = max(cy - 1, 0); y <= min(cy + 1, kGrid - 1); ++y)
+                for (int x = max(cx - 1, 0); x <= min(cx + 1, kGrid - 1); ++x) w += g[y * kGrid + x];
+        } else {
+            const int len = p.rec_len[item];
+            if (len & kTileRecord) w = (unsigned int)len & ((1u << kTileGroupShift) - 1u);
+        }
+    }
+    // twice the exponent plus the leading bit of the mantissa; bucket 0 the heaviest
+    const int b = kOrderBuckets - 1 - min((__float_as_int((float)(w + 1u)) >> 22) - 2 * 127, kOrderBuckets - 1);
+    if (i < waves) {
+        bucket[i] = (unsigned char)b;
+        atomicAdd(&cnt[b], 1);
+    }
+    __syncthreads();
+    if (threadIdx.x < kOrderBuckets && cnt[threadIdx.x] > 0) atomicAdd(&hist[threadIdx.x], cnt[threadIdx.x]);
+}
+
+// The wavefronts by falling weight, near their own order within a bucket (hist: the buckets' sizes, then
+// their cursors); clears the grid for the next job.
+__global__ void __launch_bounds__(kOrderBlock) k_tile_order(int waves, const unsigned char* __restrict__ bucket,
+                                                            int* __restrict__ hist, int* __restrict__ order,
+                                                            unsigned int* grid, int cells) {
+    __shared__ int cnt[kOrderBuckets], at[kOrderBuckets];
+    const int t = threadIdx.x, i = blockIdx.x * kOrderBlock + t;
+    if (t < kOrderBuckets) cnt[t] = 0;
+    for (int k = i; k < cells; k += gridDim.x * kOrderBlock) grid[k] = 0u;
+    __syncthreads();
+    const int b = i < waves ? bucket[i] : -1;
+    int rank = 0;
+    for (unsigned long long rem = __ballot(b >= 0); rem != 0ULL;) {
+        const int v = __builtin_amdgcn_readlane(b, __ffsll((long long)rem) - 1);
+        const unsigned long long m = __ballot(b == v);
+        int first = 0;
+        if ((t & 63) == 0) first = atomicAdd(&cnt[v], __popcll(m));
+        first = __builtin_amdgcn_readfirstlane(first);
+        if (b == v) rank = first + mask_rank(m);
+        rem &= ~m;
+    }
+    __syncthreads();
+    if (t < kOrderBuckets && cnt[t] > 0) {
+        int start = 0;
+        for (int k = 0; k < t; ++k) start += hist[k];
+        at[t] = start + atomicAdd(&hist[kOrderBuckets + t], cnt[t]);
+    }
+    __syncthreads();
+    if (b >= 0) order[at[b] + rank] = i;
+}
+
 // ------------------------------------------------------------------ kernels ------------------
 
-// Wavefront of a block: runs of `chunk` consecutive wavefronts go to one XCD (blocks are dispatched
+// Wavefront of a block, -1 past the last: runs of `chunk` go to one XCD (blocks are dispatched
 // round-robin over the eight), so that its L2 serves a compact part of the scene, and the runs in
-// turn to all of them, so that no XCD is left with the cheaper views of a batch.
-__device__ __forceinline__ int64_t tile_wave(int64_t b, int chunk) {
+// turn to all of them, so that no XCD is left with the cheaper ones.
+__device__ __forceinline__ int64_t tile_wave(const DevParams& p, int64_t b, int chunk, int waves) {
     const int64_t k = b >> 3;
-    return ((k / chunk) * 8 + (b & 7)) * chunk + k % chunk;
+    const int64_t i = ((k / chunk) * 8 + (b & 7)) * chunk + k % chunk;
+    if (i >= waves) return -1;
+    return p.order ? p.order[i] : i;
 }
 
 // Leaves the lanes with mine to the slab stepper.
@@ -469,14 +566,14 @@ __device__ __forceinline__ void tile_leave(const DevParams& p, int64_t wave, boo
 
 template <int SPB, bool RNG, int RM>
 __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(SPB == 8 ? 4 : 3)))
-k_tile_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int chunk, int hit_depth,
+k_tile_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int waves, int chunk, int hit_depth,
                float* __restrict__ out_rgb, float* __restrict__ out_depth, float* __restrict__ out_opac, DevStats st) {
     __shared__ TileLds W;
     const int lane = threadIdx.x;
-    const int64_t wave = tile_wave(blockIdx.x, chunk);
+    const int64_t wave = tile_wave(p, blockIdx.x, chunk, waves);
+    if (wave < 0) return;
     const int64_t item = wave_item(p, wave, lane);
     const bool in = item >= 0 && item < num_items;
-    if (__ballot(in) == 0ULL) return;
     Counters ctr;
     RayRef q;
     q.view = -1;
@@ -513,7 +610,10 @@ k_tile_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int chun
     if constexpr (RM == 1) {
         rc.pos = tr.pos | (max(group, 0) << kTileGroupShift) | kTileRecord;
         if (lane == 0) ctr.rec_words += 4 * tr.pos;
-        if (rs == RAY_NONE && in) p.rec_id[item] = make_int2(-1, -1);  // padding: no records
+        if (rs == RAY_NONE && in) {  // padding: no records
+            p.rec_len[item] = 0;
+            p.rec_id[item] = make_int2(-1, -1);
+        }
     }
     if (rs == RAY_OK) forward_finish<RM>(p, q, item, o, rc, ctr, out_rgb, out_depth, out_opac);
     if (rs == RAY_BAD) forward_bad<RM>(p, q, item, st, out_rgb, out_depth, out_opac);
@@ -522,16 +622,16 @@ k_tile_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int chun
 
 template <int SPB, bool RNG, int RM>
 __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(3)))
-k_tile_backward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int chunk, const float* __restrict__ ray_colors,
+k_tile_backward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int waves, int chunk, const float* __restrict__ ray_colors,
                 const float* __restrict__ dLdC, const float* __restrict__ target, int loss_kind, int count_stats,
                 DevGrad gr, DevStats st) {
     __shared__ TileLds W;
     __shared__ GradStage G;
     const int lane = threadIdx.x;
-    const int64_t wave = tile_wave(blockIdx.x, chunk);
+    const int64_t wave = tile_wave(p, blockIdx.x, chunk, waves);
+    if (wave < 0) return;
     const int64_t item = wave_item(p, wave, lane);
     const bool in = item >= 0 && item < num_items;
-    if (__ballot(in) == 0ULL) return;
     Counters ctr;
     float loss = 0.0f;
     BwdRay b;
@@ -556,9 +656,27 @@ k_tile_backward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int chu
 template <typename K, typename... A>
 void launch_tiles(K kernel, const DevScene& sc, const DevParams& p, const RayJob& job, hipStream_t s, A... args) {
     const int64_t waves = num_waves(p, job.num_rays);
-    const int chunk = (int)(waves < 8 * 8 * 64 ? (waves + 63) / 64 : 64);  // at least 8 runs for each XCD
+    // 64 wavefronts of the image's own order, at least 8 runs for each XCD; 8 of the ordered ones
+    const int chunk = p.order ? 8 : (int)(waves < 8 * 8 * 64 ? (waves + 63) / 64 : 64);
     const int64_t nb = (waves + 8 * chunk - 1) / (8 * chunk) * (8 * chunk);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(kWave), 0, s, sc, p, job, job.num_rays, chunk, args...);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(kWave), 0, s, sc, p, job, job.num_rays, (int)waves, chunk, args...);
+}
+
+// Fills p.order (dear wavefronts first): from the Gaussians' means (forward), or the records.
+void launch_order(const DevScene& sc, const DevParams& p, const RayJob& job, bool records, unsigned long long* counters,
+                  hipStream_t s) {
+    int* hist = reinterpret_cast<int*>(counters);
+    const int waves = (int)num_waves(p, job.num_rays);
+    const int first = job.ray_view ? 0 : job.view, views = job.ray_view ? job.num_views : 1;
+    const int64_t stride = ((int64_t)sc.n * views + kSplats) / kSplats;
+    const int64_t count = (sc.n + stride - 1) / stride;
+    if (!records && count > 0)
+        hipLaunchKernelGGL(k_tile_splat, dim3((unsigned)((count + 255) / 256), views), dim3(256), 0, s, sc.n, (int)stride,
+                           sc.geo, job.cams, first, p.order_grid);
+    hipLaunchKernelGGL(k_tile_weight, dim3((waves + 255) / 256), dim3(256), 0, s, p, job, job.num_rays, first, waves,
+                       records ? nullptr : p.order_grid, p.order_bucket, hist);
+    hipLaunchKernelGGL(k_tile_order, dim3((waves + kOrderBlock - 1) / kOrderBlock), dim3(kOrderBlock), 0, s, waves,
+                       p.order_bucket, hist, p.order, p.order_grid, records ? 0 : views * kGrid * kGrid);
 }
 
 // Specialised on SPB (8 or 16 samples per slab), on whether the random generator is used and on the
@@ -593,6 +711,8 @@ int rays_per_wave(int64_t num_items) {
     return tiles <= 256 ? 4 : tiles <= 512 ? 8 : tiles <= 1024 ? 16 : tiles <= 3072 ? 32 : 64;
 }
 
+int64_t order_grid_cells(int views) { return (int64_t)views * kGrid * kGrid; }
+
 // A block's rays differ by at most eight pixel steps of the image plane along each axis; their unit
 // directions differ by no more, the plane's nearest point being w at a right angle.
 bool view_is_narrow(const rg_camera& cam, int64_t n) {
@@ -611,6 +731,7 @@ hipError_t launch_forward(const DevScene& sc, const DevParams& p0, const RayJob&
     DevParams p = p0;
     p.wide_count = st.c + 12;
     if (!stepper_only(p)) {
+        if (p.order) launch_order(sc, p, job, false, st.c + 16, s);
         RG_TILE_DISPATCH(p.rec_mode == 1, 1, k_tile_forward, sc, p, job, s, hit_depth, out_rgb, out_depth, out_opacity, st);
         if (!p.wide) return hipGetLastError();
     } else {
@@ -626,6 +747,7 @@ hipError_t launch_backward(const DevScene& sc, const DevParams& p0, const RayJob
     DevParams p = p0;
     p.wide_count = st.c + 13;
     if (!stepper_only(p)) {
+        if (p.order) launch_order(sc, p, job, p.rec_mode == 2, st.c + 48, s);
         RG_TILE_DISPATCH(p.rec_mode == 2, 2, k_tile_backward, sc, p, job, s, ray_colors, dLdC, target, loss_kind, count_stats,
                          gr, st);
         if (!p.wide) return hipGetLastError();

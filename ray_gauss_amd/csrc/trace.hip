@@ -1000,7 +1000,7 @@ __global__ void __launch_bounds__(kWave) k_debug_hits(DevScene sc, DevParams p, 
 }
 
 __global__ void k_reset_counters(unsigned long long* c) {
-    if (threadIdx.x < 16) c[threadIdx.x] = 0;
+    if (threadIdx.x < kCounters) c[threadIdx.x] = 0;
 }
 
 __global__ void k_loss_out(const unsigned long long* c, float* out) {
@@ -1058,7 +1058,7 @@ hipError_t launch_loss_out(DevStats st, float* out, hipStream_t s) {
 }
 
 hipError_t launch_reset_counters(DevStats st, hipStream_t s) {
-    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, st.c);
+    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(128), 0, s, st.c);
     return hipGetLastError();
 }
 
