@@ -9,7 +9,8 @@
 //              a node's preorder index is 2*first_leaf + (left turns on its root path), and its
 //              subtree occupies the next 2*leaves-1 indices.
 //   refit : bottom-up, one thread per leaf; the second thread to reach an internal node (atomic
-//           flag) writes the union of its children's boxes.
+//           flag, in LDS where the node spans one block of leaves) writes the union of its
+//           children's boxes.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -66,6 +67,12 @@ __global__ void k_morton(int n, const float4* __restrict__ leafbox_orig, const f
 
 // ---------------------------------------------------------------- radix sort ----------------
 
+// Up to this many tiles of 2048 keys each scatter block adds up the histogram rows of the tiles before
+// it by itself (tiles KB from L2, coalesced); beyond, one block scans the whole histogram first.  That
+// scan is a launch of 13.5 us per pass at 100k keys (8 passes), and at 3M keys a rebuild took 8.2 ms
+// with it and 2.3 ms without.
+constexpr int kSelfTiles = 4096;
+
 __global__ void __launch_bounds__(kSortBlock) k_hist(int n, int shift, const unsigned long long* __restrict__ keys,
                                                      unsigned int* __restrict__ hist, int tiles) {
     __shared__ unsigned int cnt[256];
@@ -77,10 +84,11 @@ __global__ void __launch_bounds__(kSortBlock) k_hist(int n, int shift, const uns
         if (i < n) atomicAdd(&cnt[(keys[i] >> shift) & 0xff], 1u);
     }
     __syncthreads();
-    hist[threadIdx.x * tiles + blockIdx.x] = cnt[threadIdx.x];
+    if (tiles <= kSelfTiles) hist[blockIdx.x * 256 + threadIdx.x] = cnt[threadIdx.x];
+    else hist[threadIdx.x * tiles + blockIdx.x] = cnt[threadIdx.x];
 }
 
-// Exclusive scan of hist[0..m) in place, one block of 1024 threads.
+// Exclusive scan of hist[0..m) in place, one block of 1024 threads (more than kSelfTiles tiles).
 __global__ void __launch_bounds__(1024) k_scan(unsigned int* hist, int m) {
     __shared__ unsigned int part[1024];
     const int t = threadIdx.x;
@@ -104,55 +112,85 @@ __global__ void __launch_bounds__(1024) k_scan(unsigned int* hist, int m) {
     }
 }
 
-// Stable scatter: keys of a tile are ranked round by round (256 keys per round, in order);
-// within a wavefront equal digits are matched with 8 ballots.
+// Stable scatter: each wavefront ranks its eighth-of-a-tile runs of 64 keys in order (equal digits of a
+// run matched with 8 ballots) against counters of its own, so the workgroup meets only to add them
+// up: 10.2 us at 100k keys against 12.7 with 256 keys ranked per workgroup round, five barriers each.
 __global__ void __launch_bounds__(kSortBlock) k_scatter(int n, int shift, const unsigned long long* __restrict__ kin,
                                                         const int* __restrict__ vin, unsigned long long* __restrict__ kout,
                                                         int* __restrict__ vout, const unsigned int* __restrict__ hist,
                                                         int tiles) {
-    __shared__ unsigned int base[256];
-    __shared__ unsigned int wcnt[kSortBlock / 64][256];
+    constexpr int kWaves = kSortBlock / 64;
+    __shared__ unsigned int wcnt[kWaves][256];
+    __shared__ unsigned int part[kWaves];
     const int t = threadIdx.x;
     const int lane = t & 63, w = t >> 6;
-    base[t] = hist[t * tiles + blockIdx.x];
     const unsigned long long lt = (lane == 0) ? 0ULL : (~0ULL >> (64 - lane));
-    const int tile0 = blockIdx.x * kTile;
+    const int first = blockIdx.x * kTile + w * (kTile / kWaves) + lane;
+    unsigned long long key[kSortItems];
+    int val[kSortItems];
+    unsigned int rank[kSortItems];
+#pragma unroll
     for (int r = 0; r < kSortItems; ++r) {
-        for (int d = lane; d < 256; d += 64) wcnt[w][d] = 0;
-        const int i = tile0 + r * kSortBlock + t;
-        const bool valid = i < n;
-        unsigned long long key = 0;
-        int val = 0;
-        unsigned int dg = 0;
-        if (valid) {
-            key = kin[i];
-            val = vin[i];
-            dg = (unsigned int)((key >> shift) & 0xff);
+        const int i = first + r * 64;
+        key[r] = i < n ? kin[i] : 0;
+        val[r] = i < n ? vin[i] : 0;
+    }
+    // base of digit t in this tile
+    unsigned int base;
+    if (tiles <= kSelfTiles) {
+        unsigned int before = 0, total = 0;
+#pragma unroll 8
+        for (int k = 0; k < tiles; ++k) {
+            const unsigned int v = hist[k * 256 + t];
+            before += k < (int)blockIdx.x ? v : 0u;
+            total += v;
         }
+        // exclusive scan of the digits' totals: within the wavefront, then over the four
+        unsigned int x = total;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned int y = __shfl_up(x, o, 64);
+            x += lane >= o ? y : 0u;
+        }
+        if (lane == 63) part[w] = x;
+        __syncthreads();
+        for (int k = 0; k < w; ++k) x += part[k];
+        base = x - total + before;
+    } else {
+        base = hist[t * tiles + blockIdx.x];
+    }
+    volatile unsigned int* cnt = wcnt[w];  // a wavefront's LDS accesses complete in order
+    for (int d = lane; d < 256; d += 64) cnt[d] = 0;
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r) {
+        const bool valid = first + r * 64 < n;
+        const unsigned int dg = (unsigned int)((key[r] >> shift) & 0xff);
         unsigned long long mask = __ballot(valid);
+#pragma unroll
         for (int bit = 0; bit < 8; ++bit) {
             const unsigned long long bb = __ballot(valid && ((dg >> bit) & 1));
             mask &= ((dg >> bit) & 1) ? bb : ~bb;
         }
-        const unsigned int rank = (unsigned int)__popcll(mask & lt);
-        const unsigned int cnt = (unsigned int)__popcll(mask);
-        __syncthreads();
-        if (valid && rank == 0) wcnt[w][dg] = cnt;
-        __syncthreads();
-        if (valid) {
-            unsigned int pre = 0;
-            for (int ww = 0; ww < w; ++ww) pre += wcnt[ww][dg];
-            const unsigned int pos = base[dg] + pre + rank;
-            kout[pos] = key;
-            vout[pos] = val;
-        }
-        __syncthreads();
-        {
-            unsigned int add = 0;
-            for (int ww = 0; ww < kSortBlock / 64; ++ww) add += wcnt[ww][t];
-            base[t] += add;
-        }
-        __syncthreads();
+        const unsigned int before = (unsigned int)__popcll(mask & lt);
+        const unsigned int seen = cnt[dg];
+        rank[r] = seen + before;
+        __builtin_amdgcn_wave_barrier();
+        if (valid && before == 0) cnt[dg] = seen + (unsigned int)__popcll(mask);
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    for (int k = 0; k < kWaves; ++k) {
+        const unsigned int c = wcnt[k][t];
+        wcnt[k][t] = base;
+        base += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r) {
+        if (first + r * 64 >= n) continue;
+        const unsigned int pos = wcnt[w][(unsigned int)((key[r] >> shift) & 0xff)] + rank[r];
+        kout[pos] = key[r];
+        vout[pos] = val[r];
     }
 }
 
@@ -282,23 +320,133 @@ __device__ __forceinline__ void refit_internal(int q, float4* nodes, const int* 
 
 __device__ __forceinline__ bool same_bits(float a, float b) { return __float_as_int(a) == __float_as_int(b); }
 
-// Refit of any tree in one launch: each leaf climbs towards the root; the second of two siblings
-// to arrive at a parent (a flag per node) computes it and continues.
-__global__ void k_refit(int n, const float4* __restrict__ leafbox, float4* nodes, const int* __restrict__ parent,
-                        const int* __restrict__ right, int* counter, const int* __restrict__ leaf_node) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    int p = leaf_node[k];
-    refit_leaf(k, p, leafbox, nodes);
-    for (int guard = 0; guard < 192; ++guard) {  // tree depth <= 96 (augmented 96-bit keys)
-        const int q = parent[p];
-        if (q < 0) break;
-        __threadfence();
-        if (atomicAdd(&counter[q], 1) == 0) return;  // sibling not finished: it continues
-        __threadfence();
-        refit_internal(q, nodes, right);
-        p = q;
+// Refit of an LBVH, bottom-up: the second of two siblings to arrive at a parent (a flag per node) unites
+// their boxes and climbs on.  Slots are in Morton order, so nearly all internal nodes span leaves of
+// one block of 256, which k_refit_block climbs in LDS; it lists the subtrees where it stops, and
+// k_refit_climb takes the lists of 16 blocks in one workgroup through the nodes that span leaves of
+// these, then those of 16 such groups, to the root.  No step leaves its workgroup, and what bounds it
+// is a climb's chain of about three memory latencies a level.  Climbing with flags between all
+// workgroups, each step fenced between the XCDs' L2 caches, took 650 us at 100k Gaussians (the refit
+// with its preprocessing 664 us, 6.4 ms at 1M; now 107 and 283 us).
+constexpr int kRefitBlock = 256;
+constexpr int kClimbLists = 16;  // lists of one workgroup, 16 threads to each
+
+__device__ __forceinline__ bool within(int first, int last, int span) { return first / span == last / span; }
+
+struct Box6 {
+    float4 lo, hi;
+};
+
+__device__ __forceinline__ Box6 unite(const Box6& a, const Box6& b) {
+    return Box6{make_float4(fminf(a.lo.x, b.lo.x), fminf(a.lo.y, b.lo.y), fminf(a.lo.z, b.lo.z), 0.0f),
+                make_float4(fmaxf(a.hi.x, b.hi.x), fmaxf(a.hi.y, b.hi.y), fmaxf(a.hi.z, b.hi.z), 0.0f)};
+}
+
+// stops / num_stops: per block, the Karras codes (leaf k: ~k) of its largest subtrees.
+__global__ void __launch_bounds__(kRefitBlock) k_refit_block(int n, const float4* __restrict__ leafbox, BvhBuffers b,
+                                                             int* __restrict__ stops, int* __restrict__ num_stops) {
+    __shared__ float box[6][2][kRefitBlock];  // of a node's left and right child, by Karras id
+    __shared__ int arrived[kRefitBlock];
+    __shared__ int count;
+    const int s0 = blockIdx.x * kRefitBlock, t = threadIdx.x, k = s0 + t;
+    arrived[t] = 0;
+    if (t == 0) count = 0;
+    if (k < n - 1 && !within(b.k_first[k], b.k_last[k], kRefitBlock)) b.counter[k] = 0;  // for the climb
+    __syncthreads();
+    if (k < n) {
+        Box6 x = {leafbox[2 * k], leafbox[2 * k + 1]};
+        refit_leaf(k, b.leaf_node[k], leafbox, b.nodes);
+        int code = ~k, p = b.k_parent[n - 1 + k];
+        bool stop = true;
+        for (int guard = 0; p >= 0 && guard < kRefitBlock; ++guard) {
+            if (!within(b.k_first[p], b.k_last[p], kRefitBlock)) break;
+            const int li = p - s0, side = b.k_left[p] == code ? 0 : 1;
+            const float v[6] = {x.lo.x, x.lo.y, x.lo.z, x.hi.x, x.hi.y, x.hi.z};
+#pragma unroll
+            for (int c = 0; c < 6; ++c) box[c][side][li] = v[c];
+            __threadfence_block();
+            if (atomicAdd(&arrived[li], 1) == 0) {  // the sibling's climb continues
+                stop = false;
+                break;
+            }
+            __threadfence_block();
+            const int o = side ^ 1;
+            const Box6 y = {make_float4(box[0][o][li], box[1][o][li], box[2][o][li], 0.0f),
+                            make_float4(box[3][o][li], box[4][o][li], box[5][o][li], 0.0f)};
+            x = side == 0 ? unite(x, y) : unite(y, x);
+            const int q = b.k_pre[p];
+            b.nodes[2 * q] = make_float4(x.lo.x, x.lo.y, x.lo.z, b.nodes[2 * q].w);
+            b.nodes[2 * q + 1] = make_float4(x.hi.x, x.hi.y, x.hi.z, __int_as_float(~b.right[q]));
+            code = p;
+            p = b.k_parent[p];
+        }
+        if (stop && p >= 0) stops[s0 + atomicAdd(&count, 1)] = code;
     }
+    __syncthreads();
+    if (t == 0) num_stops[blockIdx.x] = count;
+}
+
+// What a climb needs of a node, loaded a level ahead (p: Karras id, -1 above the root).
+struct ClimbNode {
+    int p, first, last, pre, right, left, parent;
+};
+
+__device__ __forceinline__ ClimbNode climb_node(const BvhBuffers& b, int p) {
+    ClimbNode c{};
+    c.p = p;
+    if (p >= 0) {
+        c.first = b.k_first[p];
+        c.last = b.k_last[p];
+        c.pre = b.k_pre[p];
+        c.left = b.k_left[p];
+        c.parent = b.k_parent[p];
+        c.right = b.right[c.pre];
+    }
+    return c;
+}
+
+// One workgroup per kClimbLists consecutive lists (list i: num_in[i] codes from in[i * stride]): climbs
+// from each through the nodes that span leaves of one group of `span` (0: all), listing where it
+// stops.  Each thread's stores are complete before its flag is set, and nobody outside the workgroup
+// reads them in this launch.
+__global__ void __launch_bounds__(kRefitBlock) k_refit_climb(int n, BvhBuffers b, const int* __restrict__ in,
+                                                             const int* __restrict__ num_in, int num_lists, int stride,
+                                                             int span, int* __restrict__ out, int* __restrict__ num_out) {
+    __shared__ int count;
+    const int t = threadIdx.x, l = blockIdx.x * kClimbLists + t / 16;
+    int* dst = out + (int64_t)blockIdx.x * kClimbLists * stride;
+    if (t == 0) count = 0;
+    __syncthreads();
+    const int m = l < num_lists ? num_in[l] : 0;
+    for (int e = t % 16; e < m; e += 16) {
+        int code = in[(int64_t)l * stride + e];
+        const int at = code >= 0 ? b.k_pre[code] : b.leaf_node[~code];
+        Box6 x = {b.nodes[2 * at], b.nodes[2 * at + 1]};
+        ClimbNode c = climb_node(b, b.k_parent[code >= 0 ? code : n - 1 + ~code]);
+        bool stop = true;
+        for (int guard = 0; c.p >= 0 && guard < 192; ++guard) {  // tree depth <= 96 (augmented 96-bit keys)
+            if (span > 0 && !within(c.first, c.last, span)) break;
+            const ClimbNode up = climb_node(b, c.parent);
+            __threadfence_block();
+            if (__hip_atomic_fetch_add(&b.counter[c.p], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0) {
+                stop = false;  // the sibling's climb continues
+                break;
+            }
+            __threadfence_block();
+            const bool is_left = c.left == code;
+            const int o = is_left ? c.right : c.pre + 1;
+            const Box6 y = {b.nodes[2 * o], b.nodes[2 * o + 1]};
+            x = is_left ? unite(x, y) : unite(y, x);
+            const int miss = c.pre + 2 * (c.last - c.first + 1) - 1;
+            b.nodes[2 * c.pre] = make_float4(x.lo.x, x.lo.y, x.lo.z, __int_as_float(miss));
+            b.nodes[2 * c.pre + 1] = make_float4(x.hi.x, x.hi.y, x.hi.z, __int_as_float(~c.right));
+            code = c.p;
+            c = up;
+        }
+        if (stop && c.p >= 0) dst[atomicAdd(&count, 1)] = code;
+    }
+    __syncthreads();
+    if (t == 0) num_out[blockIdx.x] = count;
 }
 
 // Level-synchronous refit of a binned-SAH tree: the leaves, then one launch per level of internal
@@ -384,7 +532,7 @@ int launch_radix_sort(int n, int passes, unsigned long long* keys[2], int* vals[
     for (int pass = 0; pass < passes; ++pass) {
         const int shift = pass * 8;
         hipLaunchKernelGGL(k_hist, dim3(tiles), dim3(kSortBlock), 0, s, n, shift, keys[cur], hist, tiles);
-        hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, hist, 256 * tiles);
+        if (tiles > kSelfTiles) hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, hist, 256 * tiles);
         hipLaunchKernelGGL(k_scatter, dim3(tiles), dim3(kSortBlock), 0, s, n, shift, keys[cur], vals[cur],
                            keys[cur ^ 1], vals[cur ^ 1], hist, tiles);
         cur ^= 1;
@@ -434,10 +582,18 @@ hipError_t launch_lbvh_refit(int n, const float4* leafbox_sorted, BvhBuffers& b,
         }
         return hipGetLastError();
     }
-    const int total = 2 * n - 1;
-    hipLaunchKernelGGL(k_fill, dim3(blocks(total, 256)), dim3(256), 0, s, b.counter, total, 0);
-    hipLaunchKernelGGL(k_refit, dim3(blocks(n, 256)), dim3(256), 0, s, n, leafbox_sorted, b.nodes, b.parent, b.right,
-                       b.counter, b.leaf_node);
+    // the lists live in the build's sort buffers, free between builds
+    int* list[2] = {b.vals[0], b.vals[1]};
+    int* num[2] = {reinterpret_cast<int*>(b.keys[0]), reinterpret_cast<int*>(b.keys[1])};
+    int lists = blocks(n, kRefitBlock), cur = 0;
+    hipLaunchKernelGGL(k_refit_block, dim3(lists), dim3(kRefitBlock), 0, s, n, leafbox_sorted, b, list[0], num[0]);
+    for (int64_t stride = kRefitBlock; lists > 1; stride *= kClimbLists) {
+        const int groups = blocks(lists, kClimbLists);
+        hipLaunchKernelGGL(k_refit_climb, dim3(groups), dim3(kRefitBlock), 0, s, n, b, list[cur], num[cur], lists, (int)stride,
+                           groups > 1 ? (int)stride * kClimbLists : 0, list[cur ^ 1], num[cur ^ 1]);
+        lists = groups;
+        cur ^= 1;
+    }
     return hipGetLastError();
 }
 
