@@ -119,7 +119,38 @@ __device__ __forceinline__ void composite(const float* sig, const float* cr, con
     }
 }
 
-// Per-sample backward coefficients of one slab, from its buffers: overwrites (sig, cr) with
+// Thresholded densities of one hit at the slab's samples (accum_hit's m).
+template <int SPB, bool RNG>
+__device__ __forceinline__ void sample_densities(const Isect& I, float sigma, float tb, unsigned int seed,
+                                                 const DevParams& p, float* m) {
+    unsigned int st = seed;
+    const WExp k = wexp(I);
+#pragma unroll
+    for (int i = 0; i < SPB; ++i) {
+        if (SPB > 8 && i >= p.spb) break;
+        const float t = sample_t(tb, i, p.dt, RNG ? p.rnd_sample : 0, st);
+        const float sw = sigma * weight(k, t - I.tc);
+        m[i] = sw > p.sigma_thr ? sw : 0.0f;
+    }
+}
+
+// Adds a hit's densities and their colour's projection F = dLdC . c on dL/dC to the slab's sums: of the
+// colour the backward needs no more.
+template <int SPB>
+__device__ __forceinline__ void accum_densities(const float* m, float F, const DevParams& p, float* sig, float* ep) {
+#pragma unroll
+    for (int i = 0; i < SPB; ++i) {
+        if (SPB > 8 && i >= p.spb) break;
+        sig[i] += m[i];
+        ep[i] += m[i] * F;
+    }
+}
+
+__device__ __forceinline__ float project_color(const float* dL, float4 c) {
+    return dL[0] * c.x + dL[1] * c.y + dL[2] * c.z;
+}
+
+// Per-sample backward coefficients of one slab, from its sums: overwrites (sig, ep) with
 // (G_i, Bq_i) and advances T and the projected colour remainder Dr = dLdC . Crem past the
 // slab (Crem_i: the ray's colour not yet composited before sample i; only its projection on
 // dLdC enters the coefficients, so one scalar is carried instead of three).
@@ -128,8 +159,7 @@ __device__ __forceinline__ void composite(const float* sig, const float* cr, con
 //   E_i  = dLdC . c^_i = (dLdC . sums_i) / sigma_i
 //   G_i  = A_i - Bq_i E_i, so that a hit of colour c weighs sample i by phi_i = G_i + Bq_i (dLdC . c)
 template <int SPB>
-__device__ __forceinline__ void slab_coeffs(float* sig, float* cr, float* cg, float* cb, const DevParams& p,
-                                            const float* dL, float& T, float& Dr) {
+__device__ __forceinline__ void slab_coeffs(float* sig, float* ep, const DevParams& p, float& T, float& Dr) {
 #pragma unroll
     for (int i = 0; i < SPB; ++i) {
         if (SPB > 8 && i >= p.spb) break;
@@ -137,73 +167,68 @@ __device__ __forceinline__ void slab_coeffs(float* sig, float* cr, float* cg, fl
         const float alpha = sample_alpha(s, p.dt);
         // the forward's colour is sums / sigma (composite); only its projection E on dLdC enters
         const float inv = s > 0.0f ? __builtin_amdgcn_rcpf(s) : 0.0f;
-        const float E = (dL[0] * cr[i] + dL[1] * cg[i] + dL[2] * cb[i]) * inv;
+        const float E = ep[i] * inv;
         const float A = p.dt * (T * E - Dr);
         const float ta = T * alpha;
         const float Bq = ta * inv;
         Dr -= ta * E;
         T *= 1.0f - alpha;
         sig[i] = A - Bq * E;
-        cr[i] = Bq;
+        ep[i] = Bq;
     }
 }
 
+// D' = M' d, as the predicate forms it (exact FP32).
+__device__ __forceinline__ void ray_in_ellipsoid(const float4 g1, const float4 g2, const float4 g3, const Ray& r, float* D) {
+#pragma clang fp contract(off)
+    D[0] = (g1.x * r.dx + g1.y * r.dy) + g1.z * r.dz;
+    D[1] = (g2.x * r.dx + g2.y * r.dy) + g2.z * r.dz;
+    D[2] = (g3.x * r.dx + g3.y * r.dy) + g3.z * r.dz;
+}
+
 // Gradient moments of one (slab, hit) for one ray.  Over the slab's samples the hit contributes
-// four sums (Ss = sum w phi, S1 = sum w phi tau, S2 = sum w phi tau^2, Sc = sum w Bq; tau = t - t_c,
-// phi = G + Bq F with F = dLdC . colour; G, Bq from slab_coeffs).
+// four sums of its densities m = sigma w (S0 = sum m phi, T1 = sum m phi tau, T2 = sum m phi tau^2,
+// Sc = sum m Bq; tau = t - t_c, phi = G + Bq F with F = dLdC . colour; G, Bq from slab_coeffs).
 // Every gradient of the Gaussian is linear in the ray-dependent moments
 //   Gy'   = P S0 + D T1                                     (3)
 //   Y'    = P P^T S0 + (P D^T + D P^T) T1 + D D^T T2         (6, symmetric)
-//   Ss, and dL_c sigma Sc                                   (1 + 3)
-// (S0, T1, T2 = sigma Ss, sigma S1, sigma S2; P, D the ray's ellipsoid-space offset and direction)
+//   S0 / sigma, and dL_c Sc                                 (1 + 3)
+// (P, D the ray's ellipsoid-space offset at t_c and direction, the ones that the densities come from:
+// another evaluation of P, as good by itself, costs the gradients 1.2 to 1.5 times their error)
 // with coefficients that depend on the Gaussian alone, so the wave sums these 13 moments over its
 // lanes and expand the sum once per Gaussian (expand_grad) instead of once per lane.
 constexpr int kMoments = 13;
 
 template <int SPB, bool RNG>
-__device__ __forceinline__ void grad_moments(const Isect& I, float sigma, float4 col, float tb, unsigned int seed,
-                                             const DevParams& p, const float* Gq, const float* Bq, const float* dL,
-                                             float* v) {
-    const float F = dL[0] * col.x + dL[1] * col.y + dL[2] * col.z;
-    float Ss = 0.0f, S1 = 0.0f, S2 = 0.0f, Sc = 0.0f;
+__device__ __forceinline__ void grad_moments(const float* P, const float* D, float sigma, const float* m, float tc, float F,
+                                             float tb, unsigned int seed, const DevParams& p, const float* Gq,
+                                             const float* Bq, const float* dL, float* v) {
+    float S0 = 0.0f, T1 = 0.0f, T2 = 0.0f, Sc = 0.0f;
     unsigned int st = seed;
-    const WExp k = wexp(I);
 #pragma unroll
     for (int i = 0; i < SPB; ++i) {
         if (SPB > 8 && i >= p.spb) break;
-        const float t = sample_t(tb, i, p.dt, RNG ? p.rnd_sample : 0, st);
-        const float tau = t - I.tc;
-        const float w0 = weight(k, tau);
-        const float w = sigma * w0 > p.sigma_thr ? w0 : 0.0f;  // below the threshold: exact zeros
-        const float phi = Gq[i] + Bq[i] * F;
-        const float wp = w * phi;
-        Ss += wp;
-        S1 += wp * tau;
-        S2 += wp * (tau * tau);
-        Sc += w * Bq[i];
+        const float tau = sample_t(tb, i, p.dt, RNG ? p.rnd_sample : 0, st) - tc;
+        const float wp = m[i] * (Gq[i] + Bq[i] * F);
+        S0 += wp;
+        T1 += wp * tau;
+        T2 += wp * (tau * tau);
+        Sc += m[i] * Bq[i];
     }
-    const float S0 = sigma * Ss, T1 = sigma * S1, T2 = sigma * S2;
-    const float P[3] = {I.Px, I.Py, I.Pz};
-    const float D[3] = {I.Dx, I.Dy, I.Dz};
-    // Gy' = U = P S0 + D T1; with W = P T1 + D T2, Y'_ab = P_a U_b + D_a W_b (symmetric)
     float W[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         v[a] = P[a] * S0 + D[a] * T1;
         W[a] = P[a] * T1 + D[a] * T2;
     }
-    // Y' entries (0,0) (1,1) (2,2) (0,1) (0,2) (1,2)
+    // with U = Gy' and W = P T1 + D T2: Y'_ab = P_a U_b + D_a W_b; (0,0) (1,1) (2,2) (0,1) (0,2) (1,2)
     const int ya[6] = {0, 1, 2, 0, 0, 1}, yb[6] = {0, 1, 2, 1, 2, 2};
 #pragma unroll
-    for (int e = 0; e < 6; ++e) {
-        const int a = ya[e], b = yb[e];
-        v[3 + e] = P[a] * v[b] + D[a] * W[b];
-    }
-    v[9] = Ss;
-    const float sc_ = sigma * Sc;
-    v[10] = dL[0] * sc_;
-    v[11] = dL[1] * sc_;
-    v[12] = dL[2] * sc_;
+    for (int k = 0; k < 6; ++k) v[3 + k] = P[ya[k]] * v[yb[k]] + D[ya[k]] * W[yb[k]];
+    v[9] = S0 * __builtin_amdgcn_rcpf(sigma);
+    v[10] = dL[0] * Sc;
+    v[11] = dL[1] * Sc;
+    v[12] = dL[2] * Sc;
 }
 
 // The 14 gradient values of one Gaussian from its summed moments m (grad_moments):

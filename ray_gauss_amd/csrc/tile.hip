@@ -228,6 +228,25 @@ __device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams
     }
 }
 
+// The events of a round whose sample densities the first pass leaves in LDS for the second, which then
+// needs neither the predicate's terms nor the weights again: the arithmetic of an event is what
+// bounds the backward (about 250 vector instructions in the first pass and 340 in the second, 1220
+// events per tile at 1M Gaussians).  Four of them with the staging area are the LDS that three
+// wavefronts per SIMD leave to each (160 KB / 12); most rounds have no more.  Measured on a training
+// pass: 165 -> 146 ms at 1M Gaussians (8 views of 1237x822), 23.2 -> 21.5 ms at 300k, 231 -> 191 us at
+// 4096 with one 64x64 view.
+constexpr int kKept = 4;
+struct KeptEvents {
+    float4 m[kKept][2][kWave];  // thresholded density sigma w of the 8 samples
+    float4 ptc[kKept][kWave];   // the offset P and t_c
+};
+
+// A walked tile holds its candidates, a replayed one its round's kept events.
+union BwdLds {
+    TileLds W;
+    KeptEvents K;
+};
+
 // Backward of the lanes with act, called by all 64 lanes.  In each round the wavefront has a list
 // of events -- a Gaussian and the lanes that hit it in their slab of the round -- which it goes
 // through twice: to recompute the slabs' sample buffers and from them the per-sample coefficients,
@@ -238,9 +257,10 @@ template <int SPB, bool RNG>
 __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParams& p, bool act, const Ray& ray,
                                               unsigned int seed, int view, const float* Cfwd, const float* dL,
                                               const u32x4* __restrict__ cells, int num_cells, int tile, bool walk,
-                                              TileLds& W, GradStage& G, int lane, const DevGrad& gr, Counters& ctr,
+                                              BwdLds& S, GradStage& G, int lane, const DevGrad& gr, Counters& ctr,
                                               unsigned long long* drops) {
     const float slab = p.dt * (float)p.spb;
+    TileLds& W = S.W;
     int nst = 0;
     bool alive = act && (ray.tenter < ray.texit) && (add_exact(ray.tenter, slab) > ray.tenter) && 1.0f > p.t_eps;
     float T = 1.0f;
@@ -315,26 +335,28 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
         const int key_base = gview * sc.n;
         const float tmin = fmaxf(ray.tenter, tb), tmax = fminf(ray.texit, add_exact(tb, slab));
         const unsigned int cur_seed = seed;
-        float sig[SPB], cr[SPB], cg[SPB], cb[SPB];
+        // the density sums and the projected colour sums, then the coefficients G_i, Bq_i
+        float sig[SPB], ep[SPB];
 #pragma unroll
-        for (int i = 0; i < SPB; ++i) sig[i] = cr[i] = cg[i] = cb[i] = 0.0f;
+        for (int i = 0; i < SPB; ++i) sig[i] = ep[i] = 0.0f;
         int nh = 0;
         bool any = false, one = false;  // the round has candidates; its events fit one batch
         int ne = 0;
-        for (int pass = 0; pass < 2; ++pass) {
+        // goes through the round's events in order: fn(number in the round, slot, lane hit it)
+        auto each_event = [&](bool again, auto&& fn) {
             // the enumeration of a walked round, resumed batch by batch
             int j = -1, sl = 0, idx = 0;
             unsigned long long m = 0ULL;
             for (int done = 0;;) {
                 bool last;
                 if (replay) {
-                    if (done > 0 || (pass == 1 && total >= kWave)) {  // a long round's later batches
+                    if (done > 0 || (again && total >= kWave)) {  // a long round's later batches
                         window(pos + 1 + done);
                         first = 0;
                     }
                     ne = min(total - done, kWave - first);
                     last = done + ne >= total;
-                } else if (pass == 1 && one) {
+                } else if (again && one) {
                     last = true;
                 } else {
                     ne = 0;
@@ -387,7 +409,7 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
                         ++ne;
                     }
                     first = 0;
-                    if (pass == 0 && done == 0) one = last;
+                    if (!again && done == 0) one = last;
                 }
                 for (int e = first; e < first + ne; ++e) {
                     const int slot = __builtin_amdgcn_readlane(ev_slot, e);
@@ -395,42 +417,75 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
                         (unsigned long long)(unsigned int)__builtin_amdgcn_readlane(ev_lo, e) |
                         (unsigned long long)(unsigned int)__builtin_amdgcn_readlane(ev_hi, e) << 32;
                     const bool in = part && ((hits >> lane) & 1ULL) != 0ULL;
-                    if (__ballot(in) == 0ULL) continue;
+                    if (__builtin_amdgcn_ballot_w64(in) == 0ULL) continue;
                     if ((unsigned)slot >= (unsigned)sc.n) {
-                        if (lane == 0) count_drop(drops);
+                        if (lane == 0 && !again) count_drop(drops);
                         continue;
                     }
-                    const float4 g0 = ld_uniform(sc.geo, 4 * (int64_t)slot), g1 = ld_uniform(sc.geo, 4 * (int64_t)slot + 1),
-                                 g2 = ld_uniform(sc.geo, 4 * (int64_t)slot + 2), g3 = ld_uniform(sc.geo, 4 * (int64_t)slot + 3);
-                    const float4 col = ld_uniform(rgbv, slot);
-                    float v[kMoments];
-#pragma unroll
-                    for (int k = 0; k < kMoments; ++k) v[k] = 0.0f;
-                    if (in) {
-                        // the hit passed the exact test: only its sampling terms are computed
-                        Isect I;
-                        float bq, cq;
-                        isect_terms(g0, g1, g2, g3, ray, I, bq, cq);
-                        refine_sampling(g0, g1, g2, g3, ray, I);
-                        if (pass == 0) {
-                            accum_hit<SPB, RNG>(I, g0.w, col, tb, cur_seed, p, sig, cr, cg, cb);
-                            ++nh;
-                        } else {
-                            grad_moments<SPB, RNG>(I, g0.w, col, tb, cur_seed, p, sig, cr, dL, v);
-                        }
-                    }
-                    if (pass == 1) grad_scatter_wave(v, key_base + slot, sc, gr, lane, G, nst, drops);
+                    fn(done + e - first, slot, in);
                 }
                 done += ne;
                 if (last) break;
             }
-            if (pass == 0) {
-                if (nh > 0) {
-                    slab_coeffs<SPB>(sig, cr, cg, cb, p, dL, T, Dr);
-                    if (RNG && p.rnd_sample == 1) seed = skip_draws(seed, p.spb);  // the slab's draws are spent
+        };
+        // densities of a hit: it passed the exact test, so only its sampling terms are computed
+        auto densities = [&](const float4 g0, const float4 g1, const float4 g2, const float4 g3, float* md) -> float4 {
+            Isect I;
+            float bq, cq;
+            isect_terms(g0, g1, g2, g3, ray, I, bq, cq);
+            refine_sampling(g0, g1, g2, g3, ray, I);
+            sample_densities<SPB, RNG>(I, g0.w, tb, cur_seed, p, md);
+            return make_float4(I.Px, I.Py, I.Pz, I.tc);
+        };
+        each_event(false, [&](int number, int slot, bool in) {
+            const float4 g0 = ld_uniform(sc.geo, 4 * (int64_t)slot), g1 = ld_uniform(sc.geo, 4 * (int64_t)slot + 1),
+                         g2 = ld_uniform(sc.geo, 4 * (int64_t)slot + 2), g3 = ld_uniform(sc.geo, 4 * (int64_t)slot + 3);
+            const float4 col = ld_uniform(rgbv, slot);
+            if (!in) return;
+            float md[SPB];
+            const float4 ptc = densities(g0, g1, g2, g3, md);
+            accum_densities<SPB>(md, project_color(dL, col), p, sig, ep);
+            if constexpr (SPB == 8) {
+                if (replay && number < kKept) {
+                    S.K.m[number][0][lane] = make_float4(md[0], md[1], md[2], md[3]);
+                    S.K.m[number][1][lane] = make_float4(md[4], md[5], md[6], md[7]);
+                    S.K.ptc[number][lane] = ptc;
                 }
-                if (__ballot(nh > 0) == 0ULL) break;
             }
+            ++nh;
+        });
+        if (nh > 0) {
+            slab_coeffs<SPB>(sig, ep, p, T, Dr);
+            if (RNG && p.rnd_sample == 1) seed = skip_draws(seed, p.spb);  // the slab's draws are spent
+        }
+        if (__builtin_amdgcn_ballot_w64(nh > 0) != 0ULL) {
+            each_event(true, [&](int number, int slot, bool in) {
+                const float4 g0 = ld_uniform(sc.geo, 4 * (int64_t)slot), g1 = ld_uniform(sc.geo, 4 * (int64_t)slot + 1),
+                             g2 = ld_uniform(sc.geo, 4 * (int64_t)slot + 2), g3 = ld_uniform(sc.geo, 4 * (int64_t)slot + 3);
+                const float4 col = ld_uniform(rgbv, slot);
+                float v[kMoments];
+#pragma unroll
+                for (int k = 0; k < kMoments; ++k) v[k] = 0.0f;
+                if (in) {
+                    float md[SPB];
+                    float4 ptc;
+                    if (SPB == 8 && replay && number < kKept) {
+                        if constexpr (SPB == 8) {
+                            const float4 a = S.K.m[number][0][lane], b = S.K.m[number][1][lane];
+                            md[0] = a.x, md[1] = a.y, md[2] = a.z, md[3] = a.w;
+                            md[4] = b.x, md[5] = b.y, md[6] = b.z, md[7] = b.w;
+                            ptc = S.K.ptc[number][lane];
+                        }
+                    } else {
+                        ptc = densities(g0, g1, g2, g3, md);
+                    }
+                    const float P[3] = {ptc.x, ptc.y, ptc.z};
+                    float D[3];
+                    ray_in_ellipsoid(g1, g2, g3, ray, D);
+                    grad_moments<SPB, RNG>(P, D, g0.w, md, ptc.w, project_color(dL, col), tb, cur_seed, p, sig, ep, dL, v);
+                }
+                grad_scatter_wave(v, key_base + slot, sc, gr, lane, G, nst, drops);
+            });
         }
         if (replay) pos += 1 + total;
         if (part) {
@@ -625,7 +680,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(3)))
 k_tile_backward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int waves, int chunk, const float* __restrict__ ray_colors,
                 const float* __restrict__ dLdC, const float* __restrict__ target, int loss_kind, int count_stats,
                 DevGrad gr, DevStats st) {
-    __shared__ TileLds W;
+    __shared__ BwdLds S;
     __shared__ GradStage G;
     const int lane = threadIdx.x;
     const int64_t wave = tile_wave(p, blockIdx.x, chunk, waves);
@@ -648,7 +703,7 @@ k_tile_backward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int wav
     if (recorded != 0ULL) num_cells = __builtin_amdgcn_readlane(b.rc.end, __ffsll((long long)recorded) - 1);
     const u32x4* cells = RM == 2 ? reinterpret_cast<const u32x4*>(rec_region(p, wave)) : nullptr;
     backward_tile<SPB, RNG>(sc, p, b.active && !(leave && rest), b.ray, b.seed, b.view, b.Cf, b.dL, cells, num_cells,
-                            b.tile, rest || b.trunc, W, G, lane, gr, ctr, st.c + C_DROP);
+                            b.tile, rest || b.trunc, S, G, lane, gr, ctr, st.c + C_DROP);
     if (count_stats) flush_counters(ctr, st);
 }
 

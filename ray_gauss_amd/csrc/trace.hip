@@ -18,8 +18,8 @@
 // (t_c = b l, P = O' + b D^, D' = M' d, h = ln|sigma/thr|),
 //     0.5 |M (o + t d - mu)|^2 = h |P|^2 + h |D'|^2 (t - t_c)^2,
 // so each (sample, hit) costs one FMA pair and one exp.  The backward accumulates, per
-// (slab, hit), four scalars (sum w phi, sum w phi tau, sum w phi tau^2, sum w B) and expands
-// them into the 14 parameter gradients of backward/gaussians_aabb.cu:700-763.
+// (slab, hit), four scalars (sum m phi, sum m phi tau, sum m phi tau^2, sum m B; m = sigma w) and
+// expands them into the 14 parameter gradients of backward/gaussians_aabb.cu:700-763.
 //
 // Gradient scatter is wave-cooperative: every lane's list is sorted by slot, so after each
 // lane has prepared one slab, the 64 lanes (an 8x8 pixel tile) walk the union of their hit sets in
@@ -527,7 +527,11 @@ __device__ void direct_scatter_wave(const DevScene& sc, const DevParams& p, bool
             Isect I;
             if (intersect(g0, g1, g2, g3, ray, I) && overlaps(cur_tmin, cur_tmax, I.r1, I.r2)) {
                 refine_sampling(g0, g1, g2, g3, ray, I);
-                grad_moments<SPB, RNG>(I, g0.w, rgbv[leaf], cur_tb, cur_seed, p, Gq, Bq, dL, v);
+                float md[SPB];
+                sample_densities<SPB, RNG>(I, g0.w, cur_tb, cur_seed, p, md);
+                const float P[3] = {I.Px, I.Py, I.Pz}, D[3] = {I.Dx, I.Dy, I.Dz};
+                grad_moments<SPB, RNG>(P, D, g0.w, md, I.tc, project_color(dL, rgbv[leaf]), cur_tb, cur_seed, p, Gq, Bq,
+                                       dL, v);
                 c = true;
             }
         }
@@ -579,9 +583,9 @@ __device__ void backward_wave(const DevScene& sc, const DevParams& p, bool activ
         bool cur_dlist = false;  // the entries are a direct slab's recorded hits (all in the slab)
         int cur_dpos = 0;
         unsigned int cur_m = 0u;  // list mode: the entries in the slab (slab_mask), not yet scattered
-        // the prepared slab's sample buffers; after slab_coeffs sig and cr hold the per-sample
+        // the prepared slab's density and projected colour sums; after slab_coeffs the per-sample
         // backward coefficients G_i, Bq_i read by the scatter below
-        float sig[SPB], cr[SPB], cg[SPB], cb[SPB];
+        float sig[SPB], ep[SPB];
         if (alive && !pend) {
             if (!(T > p.t_eps)) {
                 alive = false;
@@ -600,8 +604,14 @@ __device__ void backward_wave(const DevScene& sc, const DevParams& p, bool activ
             {
                 const float tb = s.tb;
 #pragma unroll
-                for (int i = 0; i < SPB; ++i) sig[i] = cr[i] = cg[i] = cb[i] = 0.0f;
+                for (int i = 0; i < SPB; ++i) sig[i] = ep[i] = 0.0f;
                 int nh = 0;
+                auto add_hit = [&](const Isect& I, float sigma, int slot) {
+                    float md[SPB];
+                    sample_densities<SPB, RNG>(I, sigma, tb, seed, p, md);
+                    accum_densities<SPB>(md, project_color(dL, rgbv[slot]), p, sig, ep);
+                    ++nh;
+                };
                 auto direct_hit = [&](int slot) -> bool {
                     float4 g0, g1, g2, g3;
                     load_rec(sc.geo, slot, g0, g1, g2, g3);
@@ -609,8 +619,7 @@ __device__ void backward_wave(const DevScene& sc, const DevParams& p, bool activ
                     if (!intersect(g0, g1, g2, g3, ray, I)) return true;
                     if (!overlaps(tmin, tmax, I.r1, I.r2)) return true;
                     refine_sampling(g0, g1, g2, g3, ray, I);
-                    accum_hit<SPB, RNG>(I, g0.w, rgbv[slot], tb, seed, p, sig, cr, cg, cb);
-                    ++nh;
+                    add_hit(I, g0.w, slot);
                     return true;
                 };
                 if (s.direct && RM == 2 && s.dcnt >= 0) {
@@ -622,8 +631,7 @@ __device__ void backward_wave(const DevScene& sc, const DevParams& p, bool activ
                         if ((unsigned)slot < (unsigned)sc.n) {
                             float sigma;
                             const Isect I = entry_hit(sc, ray, slot, 0.0f, 0.0f, sigma);
-                            accum_hit<SPB, RNG>(I, sigma, rgbv[slot], tb, seed, p, sig, cr, cg, cb);
-                            ++nh;
+                            add_hit(I, sigma, slot);
                         } else {
                             count_drop(drops);
                         }
@@ -641,12 +649,11 @@ __device__ void backward_wave(const DevScene& sc, const DevParams& p, bool activ
                         const int slot = L.g[e][lane];
                         float sigma;
                         const Isect I = entry_hit(sc, ray, slot, L.r1[e][lane], L.r2[e][lane], sigma);
-                        accum_hit<SPB, RNG>(I, sigma, rgbv[slot], tb, seed, p, sig, cr, cg, cb);
-                        ++nh;
+                        add_hit(I, sigma, slot);
                     }
                 }
                 if (nh > 0) {
-                    slab_coeffs<SPB>(sig, cr, cg, cb, p, dL, T, Dr);
+                    slab_coeffs<SPB>(sig, ep, p, T, Dr);
                     cur_tb = tb;
                     cur_seed = seed;
                     cur_tmin = tmin;
@@ -670,7 +677,7 @@ __device__ void backward_wave(const DevScene& sc, const DevParams& p, bool activ
         jump = __ballot(prepped) != 0ULL && __ballot(has || dsc) == 0ULL;
         // converged: slabs whose hit set overflowed the list scatter from a packet traversal
         if (__ballot(dsc) != 0ULL)
-            direct_scatter_wave<SPB, RNG>(sc, p, dsc, ray, rgbv, cur_tb, cur_seed, cur_tmin, cur_tmax, sig, cr, dL, G,
+            direct_scatter_wave<SPB, RNG>(sc, p, dsc, ray, rgbv, cur_tb, cur_seed, cur_tmin, cur_tmax, sig, ep, dL, G,
                                      nst, lane, gr, view, drops);
         // wave-merged scatter over the prepared slabs' list hits.  A lane's key (view * n + slot of
         // its next hit; INT_MAX when it has none) changes only when its hit is scattered, and the
@@ -713,7 +720,11 @@ __device__ void backward_wave(const DevScene& sc, const DevParams& p, bool activ
                     float b, c;
                     isect_terms(g0, g1, g2, g3, ray, I, b, c);
                     refine_sampling(g0, g1, g2, g3, ray, I);
-                    grad_moments<SPB, RNG>(I, g0.w, rgbv[slot], cur_tb, cur_seed, p, sig, cr, dL, v);
+                    float md[SPB];
+                    sample_densities<SPB, RNG>(I, g0.w, cur_tb, cur_seed, p, md);
+                    const float P[3] = {I.Px, I.Py, I.Pz}, D[3] = {I.Dx, I.Dy, I.Dz};
+                    grad_moments<SPB, RNG>(P, D, g0.w, md, I.tc, project_color(dL, rgbv[slot]), cur_tb, cur_seed, p, sig,
+                                           ep, dL, v);
                 }
                 if (cur_dlist) {
                     ++e;
