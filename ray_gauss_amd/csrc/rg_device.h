@@ -12,6 +12,8 @@
 
 namespace rg {
 
+constexpr int kWave = 64;
+
 struct Ray {
     float ox, oy, oz;
     float dx, dy, dz;
@@ -117,6 +119,25 @@ struct Isect {
     float l;              // 1 / |D'|
 };
 
+// 1 / sqrt(x) with both operations correctly rounded, in 9 instructions instead of the 27 of the
+// general square root and division.  For x in [2^-60, 2^62) one Newton step from the native
+// reciprocal root gives the correctly rounded root and one more the correctly rounded reciprocal
+// (compared with the general operations for every mantissa and both parities of the exponent), but
+// for the roots whose mantissa is all ones.  Those and, unless the caller knows the range, other x
+// take the general operations.  In the backward at 1M Gaussians 145.9 -> 138.0 ms.
+template <bool RANGE = true>
+__device__ __forceinline__ float inv_sqrt_exact(float x) {
+#pragma clang fp contract(off)
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y;
+    const float s = __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
+    float l = __builtin_fmaf(__builtin_fmaf(-s, y, 1.0f), y, y);
+    bool general = (__float_as_uint(s) | 0xff800000u) == 0xffffffffu;
+    if (RANGE) general |= __float_as_uint(x) - 0x21800000u >= 0x5e800000u - 0x21800000u;
+    if (general) l = 1.0f / __builtin_sqrtf(x);
+    return l;
+}
+
 // Sampling terms of the bounding-ellipsoid test (everything but the roots), exact FP32 with the
 // operation order of the host FP32 checker.  Returns disc = 1 - |P|^2.
 __device__ __forceinline__ float isect_terms(const float4 g0, const float4 g1, const float4 g2, const float4 g3,
@@ -130,7 +151,7 @@ __device__ __forceinline__ float isect_terms(const float4 g0, const float4 g1, c
     const float Dp1 = (g2.x * r.dx + g2.y * r.dy) + g2.z * r.dz;
     const float Dp2 = (g3.x * r.dx + g3.y * r.dy) + g3.z * r.dz;
     const float ddp = (Dp0 * Dp0 + Dp1 * Dp1) + Dp2 * Dp2;
-    const float l = 1.0f / __builtin_sqrtf(ddp);
+    const float l = inv_sqrt_exact(ddp);
     const float Dh0 = Dp0 * l, Dh1 = Dp1 * l, Dh2 = Dp2 * l;
     b = -((Op0 * Dh0 + Op1 * Dh1) + Op2 * Dh2);
     c = ((Op0 * Op0 + Op1 * Op1) + Op2 * Op2) - 1.0f;

@@ -10,7 +10,6 @@
 
 namespace rg {
 
-constexpr int kWave = 64;
 constexpr int kGradVals = 14;
 
 enum CounterIdx { C_K = 0, C_P = 1, C_OVF = 2, C_FALLBACK = 3, C_GATHER = 4, C_LOSS = 6, C_REC_WORDS = 8,

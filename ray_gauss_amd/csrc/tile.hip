@@ -54,34 +54,18 @@ __device__ __forceinline__ bool tile_groups(const DevScene& sc, bool act, int vi
     return rem == 0ULL;
 }
 
-// The gathered depth range of a marching tile (wave-uniform).
-struct TileWalk {
-    float s1 = 0.0f;      // end of the range
-    int m = 1;            // its length in slabs
-    int cnt = 0;          // candidates in the list
-    bool valid = false;
-    bool direct = false;  // the round's candidates do not fit: it walks the tree itself
-};
-
-// Makes the list cover the round [tlag, whi].  The range's length doubles while the list is mostly
-// empty and halves while it is nearly full; a round whose own candidates do not fit is walked.
-__device__ __forceinline__ void tile_list(TileWalk& w, const DevScene& sc, const Beam& b, float tlag, float whi,
-                                          float slab, TileLds& W, int lane, bool alive, Counters& ctr) {
+// Makes the list cover the round [tlag, whi]: all of it, or with split at least its first leaves.  The
+// range's length doubles while the list is mostly empty and halves while it is nearly full.
+__device__ __forceinline__ void tile_list(TileWalk& w, const DevScene& sc, float tlag, float whi, float slab, bool split,
+                                          TileLds& W, int lane, bool alive, Counters& ctr) {
     if (w.valid && !(whi > w.s1)) return;
     if (w.valid && 4 * w.cnt < kTileCand) w.m = min(w.m * 2, kMaxSeg);
     else if (w.valid && 4 * w.cnt > 3 * kTileCand) w.m = max(w.m >> 1, 1);
     w.valid = true;
-    w.direct = false;
-    while (true) {
-        w.s1 = w.m > 1 ? fmaxf(tlag + (float)(w.m + 1) * slab, whi) : whi;
-        w.cnt = beam_gather(sc.nodes, sc.geo, sc.total_nodes, b, tlag, w.s1, W, lane);
-        if (alive) ctr.gathers++;
-        if (w.cnt >= 0) return;
-        if (w.m == 1) break;
-        w.m >>= 1;
-    }
-    w.cnt = 0;
-    w.direct = true;
+    w.s1 = range_end(w.m, tlag, whi, slab);
+    w.direct = !beam_gather(sc.nodes, sc.geo, sc.total_nodes, w, tlag, whi, slab, split, W, lane);
+    if (w.direct) w.cnt = 0;
+    if (alive) ctr.gathers++;
 }
 
 // The lanes of the next round: its depths [tlag, whi] and whether this lane takes part.
@@ -92,13 +76,13 @@ __device__ __forceinline__ bool tile_window(bool alive, float tb, float slab, fl
     return part;
 }
 
-// Chunk j of the list: this lane's candidate and the lanes whose candidate meets [wlo, whi].
+// Chunk j of the list: this lane's entry of W.slot and the lanes whose candidate meets [wlo, whi].
 __device__ __forceinline__ unsigned long long tile_chunk(const TileLds& W, int cnt, int j, int lane, float wlo, float whi,
                                                          int& slot) {
     const int i = 64 * j + lane;
     const bool in = i < cnt;
     slot = in ? W.slot[i] : 0;
-    return __ballot(in && !(W.z0[i] > whi) && !(W.z1[i] < wlo));
+    return __builtin_amdgcn_ballot_w64(in && !(W.z0[i] > whi) && !(W.z1[i] < wlo));
 }
 
 // After a round without candidates: every lane steps over the slabs that end before the next
@@ -146,30 +130,49 @@ __device__ __forceinline__ void tile_rec_round(TileRec& r, float tlag, int view,
 // Forward of the lanes with act, which share their view, as one beam.  Called by all 64 lanes.
 template <int SPB, bool RNG, int RM>
 __device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams& p, bool act, const Ray& ray,
-                                             unsigned int& seed, int view, int group, int hit_depth, TileLds& W, int lane,
+                                             unsigned int& seed, int view, const float* cam_u, int group, int hit_depth,
+                                             TileLds& W, int lane,
                                              Counters& ctr, RayOut& o, TileRec& rc) {
     const float slab = p.dt * (float)p.spb;
     const float4* __restrict__ rgbv = sc.rgb + (size_t)view * sc.n;
-    const Beam beam = make_beam(act, ray);
+    make_beam(act, ray, cam_u, W, lane);
     TileWalk w;
     w.m = p.seg_slabs;
     bool alive = act && o.T > p.t_eps;
     float tb = ray.tenter;
+    // sums of a round that goes on with another list, in memory: few do, and the registers are the gather's
+    volatile float held[4 * SPB];
+    int nh = 0;
+    bool any = false;  // the round has candidates
     while (__ballot(alive) != 0ULL) {
         float tlag, whi;
         const bool part = tile_window(alive, tb, slab, tlag, whi);
-        tile_list(w, sc, beam, tlag, whi, slab, W, lane, alive, ctr);
+        tile_list(w, sc, tlag, whi, slab, true, W, lane, alive, ctr);
         const float tmin = fmaxf(ray.tenter, tb), tmax = fminf(ray.texit, add_exact(tb, slab));
         float sig[SPB], cr[SPB], cg[SPB], cb[SPB];
 #pragma unroll
         for (int i = 0; i < SPB; ++i) sig[i] = cr[i] = cg[i] = cb[i] = 0.0f;
-        int nh = 0;
-        auto eval = [&](int slot, bool cond) {
+        if (w.first > 0) {
+#pragma unroll
+            for (int i = 0; i < SPB; ++i) {
+                sig[i] = held[4 * i];
+                cr[i] = held[4 * i + 1];
+                cg[i] = held[4 * i + 2];
+                cb[i] = held[4 * i + 3];
+            }
+        } else {
+            nh = 0;
+            any = false;
+        }
+        // at: the candidate's place in the list, or -1
+        auto eval = [&](int slot, int at, bool cond) {
             const float4 g0 = ld_uniform(sc.geo, 4 * (int64_t)slot), g1 = ld_uniform(sc.geo, 4 * (int64_t)slot + 1),
                          g2 = ld_uniform(sc.geo, 4 * (int64_t)slot + 2), g3 = ld_uniform(sc.geo, 4 * (int64_t)slot + 3);
             Isect I;
-            const bool hit = cond && intersect(g0, g1, g2, g3, ray, I) && overlaps(tmin, tmax, I.r1, I.r2);
-            const unsigned long long hits = __ballot(hit);
+            bool hit;
+            if (at >= 0) hit = listed_hit(W.oc[at], g1, g2, g3, ray, tmin, tmax, cond, I);
+            else hit = cond && intersect(g0, g1, g2, g3, ray, I) && overlaps(tmin, tmax, I.r1, I.r2);
+            const unsigned long long hits = __builtin_amdgcn_ballot_w64(hit);
             if (hits == 0ULL) return;
             if constexpr (RM == 1) {
                 if (!rc.full) tile_rec_event(rc, slot, hits, lane);
@@ -181,29 +184,45 @@ __device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams
                 ++nh;
             }
         };
-        bool any = w.direct;
+        any |= w.direct;
         for (int j = 0; kWave * j < w.cnt; ++j) {
             int sl;
             unsigned long long m = tile_chunk(W, w.cnt, j, lane, tlag, whi, sl);
             any |= m != 0ULL;
             while (m != 0ULL) {
-                const int slot = __builtin_amdgcn_readlane(sl, __builtin_ctzll(m));
+                const int i = __builtin_ctzll(m);
+                const int code = __builtin_amdgcn_readlane(sl, i);
                 m &= m - 1ULL;
-                eval(slot, part);
+                eval(code >> 1, (code & 1) ? -1 : kWave * j + i, part);
             }
         }
         if (w.direct) {
             const float ix = 1.0f / ray.dx, iy = 1.0f / ray.dy, iz = 1.0f / ray.dz;
-            for (int idx = 0; idx < sc.total_nodes;) {
+            for (int idx = w.first; idx < sc.total_nodes;) {
                 idx = __builtin_amdgcn_readfirstlane(idx);
                 const float4 lo = ld_node(sc.nodes, 2 * idx), hi = ld_node(sc.nodes, 2 * idx + 1);
                 const int miss = __float_as_int(lo.w), leaf = __float_as_int(hi.w);
                 if (miss <= idx || leaf >= sc.n) break;  // malformed link: never loop
                 const bool h = part && box_hit(lo, hi, ray, ix, iy, iz, tmin, tmax);
                 const bool met = __ballot(h) != 0ULL;
-                if (met && leaf >= 0) eval(leaf, h);
+                if (met && leaf >= 0) eval(leaf, -1, h);
                 idx = met && leaf < 0 ? idx + 1 : miss;
             }
+            w.valid = false;
+        } else if (w.limit < sc.total_nodes) {  // the round goes on with its other leaves
+#pragma unroll
+            for (int i = 0; i < SPB; ++i) {
+                held[4 * i] = sig[i];
+                held[4 * i + 1] = cr[i];
+                held[4 * i + 2] = cg[i];
+                held[4 * i + 3] = cb[i];
+            }
+            w.first = w.limit;
+            w.valid = false;
+            continue;
+        }
+        if (w.first > 0) {
+            w.first = 0;
             w.valid = false;
         }
         if constexpr (RM == 1) {
@@ -254,7 +273,7 @@ union BwdLds {
 // record of the tile (cells; lanes take part with their beam in it, tile, -1: none), and for the lanes with walk, once it ends, from the
 // tile's own gathers.
 template <int SPB, bool RNG>
-__device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParams& p, bool act, const Ray& ray,
+__device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParams& p, const rg_camera* cams, bool act, const Ray& ray,
                                               unsigned int seed, int view, const float* Cfwd, const float* dL,
                                               const u32x4* __restrict__ cells, int num_cells, int tile, bool walk,
                                               BwdLds& S, GradStage& G, int lane, const DevGrad& gr, Counters& ctr,
@@ -282,7 +301,6 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
     int pos = 0;
     unsigned long long todo = 0ULL;  // lanes of the beam being walked
     int gview = 0, group = -1;
-    Beam beam = {};
     TileWalk w;
     while (true) {
         const bool replay = pos < num_cells;
@@ -323,13 +341,13 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
                 const int f = __ffsll((long long)rem) - 1;
                 gview = __builtin_amdgcn_readlane(view, f);
                 todo = __ballot(alive && walk && group == __builtin_amdgcn_readlane(group, f));
-                beam = make_beam(((todo >> lane) & 1ULL) != 0ULL, ray);
+                make_beam(((todo >> lane) & 1ULL) != 0ULL, ray, cams[gview].u, W, lane);
                 w = TileWalk();
                 w.m = p.seg_slabs;
             }
             const bool mine = alive && ((todo >> lane) & 1ULL) != 0ULL;
             part = tile_window(mine, tb, slab, tlag, whi);
-            tile_list(w, sc, beam, tlag, whi, slab, W, lane, mine, ctr);
+            tile_list(w, sc, tlag, whi, slab, false, W, lane, mine, ctr);
         }
         const float4* __restrict__ rgbv = sc.rgb + (size_t)gview * sc.n;
         const int key_base = gview * sc.n;
@@ -392,7 +410,7 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
                                 any |= m != 0ULL;
                                 continue;
                             }
-                            slot = __builtin_amdgcn_readlane(sl, __builtin_ctzll(m));
+                            slot = __builtin_amdgcn_readlane(sl, __builtin_ctzll(m)) >> 1;
                             m &= m - 1ULL;
                         }
                         const float4 g0 = ld_uniform(sc.geo, 4 * (int64_t)slot), g1 = ld_uniform(sc.geo, 4 * (int64_t)slot + 1),
@@ -659,7 +677,7 @@ k_tile_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int wave
         const unsigned long long m = __ballot(mine);
         if (m == 0ULL) break;
         const int view = __builtin_amdgcn_readlane(q.view, __ffsll((long long)m) - 1);
-        forward_tile<SPB, RNG, RM>(sc, p, mine, ray, seed, view, g, hit_depth, W, lane, ctr, o, tr);
+        forward_tile<SPB, RNG, RM>(sc, p, mine, ray, seed, view, job.cams[view].u, g, hit_depth, W, lane, ctr, o, tr);
         if (mine) rc.full = tr.full;
     }
     if constexpr (RM == 1) {
@@ -702,7 +720,7 @@ k_tile_backward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int wav
     int num_cells = 0;
     if (recorded != 0ULL) num_cells = __builtin_amdgcn_readlane(b.rc.end, __ffsll((long long)recorded) - 1);
     const u32x4* cells = RM == 2 ? reinterpret_cast<const u32x4*>(rec_region(p, wave)) : nullptr;
-    backward_tile<SPB, RNG>(sc, p, b.active && !(leave && rest), b.ray, b.seed, b.view, b.Cf, b.dL, cells, num_cells,
+    backward_tile<SPB, RNG>(sc, p, job.cams, b.active && !(leave && rest), b.ray, b.seed, b.view, b.Cf, b.dL, cells, num_cells,
                             b.tile, rest || b.trunc, S, G, lane, gr, ctr, st.c + C_DROP);
     if (count_stats) flush_counters(ctr, st);
 }

@@ -82,7 +82,8 @@ def test_wavefronts_across_rows_of_tiles(gpu_device, words):
 @pytest.mark.parametrize("words", [0, 64, 4096])
 def test_rounds_with_more_candidates_than_the_list(gpu_device, words):
     """Large overlapping Gaussians: single slabs hold more candidates than a tile's list, so their
-    rounds walk the tree and have more events than one batch."""
+    rounds go on with further lists (in a backward without records, walk the tree) and have more
+    events than one batch."""
     sc = scenes.scene_uniform(1200, seed=5, log_scale_mean=-1.2)
     sc.densities[:] = 0.11 + 0.002 * np.arange(1200, dtype=np.float32) / 1200
     sc.scales[:] *= 4.0
@@ -98,4 +99,31 @@ def test_camera_inside_the_scene(gpu_device, t_near):
     sc = scenes.scene_uniform(3000, seed=11, log_scale_mean=-2.5)
     prm = scenes.RenderParams(dt=0.01, t_eps=1e-4, t_near=t_near, t_far=2.5)
     st = _compare(sc, prm, [_view(24, 16, radius=0.3)], gpu_device, np.zeros(384), np.arange(384), 512)
+    assert st["slab_hits"] > 0
+
+
+@pytest.mark.parametrize("n", [255, 256, 257, 511, 513])
+def test_lists_around_their_capacity(gpu_device, n):
+    """Every Gaussian is a candidate of the rounds at the centre: lists of all, or split between leaves."""
+    sc = scenes.scene_uniform(n, seed=n)
+    sc.positions[:] *= 0.01
+    sc.scales[:] = 0.3
+    sc.densities[:] = 0.11 + 0.002 * np.arange(n, dtype=np.float32) / n
+    prm = scenes.RenderParams(dt=0.02, t_eps=1e-4)
+    st = _compare(sc, prm, [_view(16, 8)], gpu_device, np.zeros(128), np.arange(128), 4096)
+    assert st["slab_hits"] >= n
+
+
+@pytest.mark.parametrize("power", [-34, -29, 0, 29, 34])
+def test_scales_beyond_the_range_of_the_fast_terms(gpu_device, power):
+    """A scene scaled by powers of two: squared lengths in ellipsoid space from 2^-70 to 2^80, inside and
+    outside the range in which the predicate's terms take the short square root."""
+    f = 2.0 ** power
+    sc = scenes.scene_uniform(600, seed=2)
+    sc.positions[:] *= f
+    sc.scales[:] *= f
+    prm = scenes.RenderParams(dt=0.01 * f, t_eps=1e-4, t_far=10.0 * f)
+    cam = look_at_camera(orbit_eye(3.0, 30.0, 20.0) * f, target=(0.0, 0.0, 0.0), width=24, height=16,
+                         fovx_deg=40.0).launch_record()
+    st = _compare(sc, prm, [cam], gpu_device, np.zeros(384), np.arange(384), 512)
     assert st["slab_hits"] > 0
