@@ -450,7 +450,7 @@ static int plan_waves(rg_handle* h, const rg::RayJob& j, rg::DevParams& p, hipSt
     if (waves >= rg::kOrderMin && views <= 4096) {
         if (waves > h->order_cap) {
             h->order_cap = 0;
-            if ((rc = dalloc(h, &h->order, waves)) || (rc = dalloc(h, &h->order_bucket, waves))) return rc;
+            if ((rc = dalloc(h, &h->order, rg::order_entries(waves))) || (rc = dalloc(h, &h->order_bucket, waves))) return rc;
             h->order_cap = waves;
         }
         if (views > h->order_views) {

@@ -246,6 +246,8 @@ bool stepper_only(const DevParams& p);
 int rays_per_wave(int64_t num_items);
 // Jobs of fewer wavefronts than this keep their own order (all of them start at once).
 constexpr int64_t kOrderMin = 2048;
+// Entries of DevParams::order for jobs of that many wavefronts, some of them split.
+int64_t order_entries(int64_t waves);
 // Cells of DevParams::order_grid for jobs over `views` views.
 int64_t order_grid_cells(int views);
 // Whether every 8x8 pixel block of the view (jittered or not) is a beam that the tile kernels take.

@@ -447,8 +447,9 @@ __device__ __forceinline__ int64_t wave_item(const DevParams& p, int64_t wave, i
     return (i & ~(int64_t)63) + 8 * y + x;
 }
 
-// rec_len of a ray in a wavefront's tile record: its 16-byte cells, the ray's beam in it, kTileRecord.
-constexpr int kTileRecord = 0x40000000, kTileGroupShift = 28;
+// rec_len of a ray in a wavefront's tile record: its 16-byte cells (at most 2^24), whether it is that of
+// a split wavefront, the ray's beam in it, kTileRecord.
+constexpr int kTileRecord = 0x40000000, kTileGroupShift = 28, kTileSplit = 1 << 27, kTileCells = kTileSplit - 1;
 
 // Starts a ray: clears its output; false when the ray has no slab to process (it misses the scene
 // box, or its first slab is below half an ulp of t).
@@ -557,7 +558,7 @@ template <bool RNG, int RM>
 __device__ __forceinline__ void backward_setup(const DevScene& sc, const DevParams& p, const RayJob& job, int64_t wave,
                                                int lane, int64_t item, const float* __restrict__ ray_colors,
                                                const float* __restrict__ dLdC, const float* __restrict__ target,
-                                               int loss_kind, DevStats st, BwdRay& b, float& loss) {
+                                               int loss_kind, DevStats st, BwdRay& b, float& loss, bool split = false) {
     RayRef q;
     const int rs = resolve(job, item, q);
     if (rs == RAY_BAD) atomicAdd(&st.c[C_BAD], 1ull);
@@ -592,9 +593,10 @@ __device__ __forceinline__ void backward_setup(const DevScene& sc, const DevPara
         if (id.x == q.view && id.y == q.pixel) {
             const int len = p.rec_len[item];
             if (len & kTileRecord) {
-                b.tile = (len >> kTileGroupShift) & 3;
+                // the record of the whole wavefront is no use to a part of it, nor the other way round
+                if (((len & kTileSplit) != 0) == split) b.tile = (len >> kTileGroupShift) & 3;
                 b.trunc = len < 0;
-                b.rc.end = min(len & ((1 << kTileGroupShift) - 1), (p.rays_per_wave * p.rec_words) >> 2);
+                b.rc.end = min(len & kTileCells, (p.rays_per_wave * p.rec_words) >> 2);
             } else {
                 b.rc.w = rec_region(p, wave) + 8 * lane;
                 b.rc.stride = 8 * p.rays_per_wave;

@@ -535,6 +535,15 @@ constexpr int kGrid = 128;              // cells of a view along each axis
 constexpr int kSplats = 1 << 20;        // Gaussians counted at most (every k-th of more)
 constexpr int kOrderBuckets = 32;       // half octaves of the weight
 constexpr int kOrderBlock = 1024;
+// A wavefront that costs more than an even share of the launch ends after the others however early it
+// starts, so it is split into quarters of its rays (narrower beams: each takes about half its time).  A
+// backward takes the forward's parts with its records.  The weights exaggerate: with shares 0.5 / 1 / 2 / 4 / none
+// (times an even one) a forward of one view of 100k Gaussians in blobs took 0.99 / 1.02 / 0.99 / 1.30 /
+// 1.55 ms, its backward 1.18 / 1.19 / 1.10 / 1.28 / 1.54, one at four times the slabs 1.61 / 1.72 / 1.83 / 2.72 / 3.26,
+// and an unbounded view of 1M, whose wavefronts are even, 12.5 / 10.7 / 9.98 / 10.0 / 10.0.  Ray lists, which
+// may have wavefronts that are no beams, are not split.
+constexpr float kSplitShare = 2.0f;
+constexpr int kSplitPart = 8;
 
 __global__ void __launch_bounds__(256) k_tile_splat(int n, int stride, const float4* __restrict__ geo,
                                                     const rg_camera* __restrict__ cams, int first_view,
@@ -562,6 +571,7 @@ __global__ void __launch_bounds__(256) k_tile_weight(DevParams p, RayJob job, in
     if (threadIdx.x < kOrderBuckets) cnt[threadIdx.x] = 0;
     __syncthreads();
     unsigned int w = 0u;
+    bool cut = false;
     RayRef q;
     const int64_t item = i < waves ? wave_item(p, i, 0) : num_items;
     if (item < num_items && resolve(job, item, q) == RAY_OK) {
@@ -574,11 +584,16 @@ __global__ void __launch_bounds__(256) k_tile_weight(DevParams p, RayJob job, in
                 for (int x = max(cx - 1, 0); x <= min(cx + 1, kGrid - 1); ++x) w += g[y * kGrid + x];
         } else {
             const int len = p.rec_len[item];
-            if (len & kTileRecord) w = (unsigned int)len & ((1u << kTileGroupShift) - 1u);
+            if (len & kTileRecord) {
+                w = (unsigned int)len & kTileCells;
+                cut = (len & kTileSplit) != 0;
+            }
         }
     }
-    // twice the exponent plus the leading bit of the mantissa; bucket 0 the heaviest
-    const int b = kOrderBuckets - 1 - min((__float_as_int((float)(w + 1u)) >> 22) - 2 * 127, kOrderBuckets - 1);
+    // twice the exponent plus the leading bit of the mantissa; bucket 0 the heaviest, and of records those
+    // of split wavefronts
+    const int b = cut ? 0 : max(kOrderBuckets - 1 - min((__float_as_int((float)(w + 1u)) >> 22) - 2 * 127, kOrderBuckets - 1),
+                                grid ? 0 : 1);
     if (i < waves) {
         bucket[i] = (unsigned char)b;
         atomicAdd(&cnt[b], 1);
@@ -587,12 +602,28 @@ __global__ void __launch_bounds__(256) k_tile_weight(DevParams p, RayJob job, in
     if (threadIdx.x < kOrderBuckets && cnt[threadIdx.x] > 0) atomicAdd(&hist[threadIdx.x], cnt[threadIdx.x]);
 }
 
+// The heaviest buckets whose wavefronts are split in four: those with more than kSplitShare of an even share of
+// the whole weight, as long as they are at most 1 / kSplitPart of the wavefronts.
+__device__ __forceinline__ int split_buckets(const int* hist, int waves, int slots) {
+    float total = 0.0f;
+    for (int k = 0; k < kOrderBuckets; ++k) total += (float)hist[k] * __builtin_amdgcn_exp2f(-0.5f * (float)k);
+    int n = 0, tiles = 0;
+    for (; n < kOrderBuckets; ++n) {
+        tiles += hist[n];
+        if (tiles > waves / kSplitPart) break;
+        if (!(__builtin_amdgcn_exp2f(-0.5f * (float)n) * (float)slots > kSplitShare * total)) break;
+    }
+    return n;
+}
+
 // The wavefronts by falling weight, near their own order within a bucket (hist: the buckets' sizes, then
-// their cursors); clears the grid for the next job.
+// their cursors), as 8 wave, or for each quarter k of a split one 8 wave + 2 k + 1, and -1 in the rest of
+// the list; clears the grid for the next job.  split: the number of heaviest buckets that are split, -1: by
+// their weight.
 __global__ void __launch_bounds__(kOrderBlock) k_tile_order(int waves, const unsigned char* __restrict__ bucket,
-                                                            int* __restrict__ hist, int* __restrict__ order,
-                                                            unsigned int* grid, int cells) {
-    __shared__ int cnt[kOrderBuckets], at[kOrderBuckets];
+                                                            int* __restrict__ hist, int* __restrict__ order, int entries,
+                                                            int split, int slots, unsigned int* grid, int cells) {
+    __shared__ int cnt[kOrderBuckets], at[kOrderBuckets], num_split, end;
     const int t = threadIdx.x, i = blockIdx.x * kOrderBlock + t;
     if (t < kOrderBuckets) cnt[t] = 0;
     for (int k = i; k < cells; k += gridDim.x * kOrderBlock) grid[k] = 0u;
@@ -609,25 +640,40 @@ __global__ void __launch_bounds__(kOrderBlock) k_tile_order(int waves, const uns
         rem &= ~m;
     }
     __syncthreads();
-    if (t < kOrderBuckets && cnt[t] > 0) {
+    if (t < kOrderBuckets) {
+        int n = split >= 0 ? split : split_buckets(hist, waves, slots);
+        if (split == 1 && hist[0] > waves / kSplitPart) n = 0;  // never expected: not this job's records
         int start = 0;
-        for (int k = 0; k < t; ++k) start += hist[k];
-        at[t] = start + atomicAdd(&hist[kOrderBuckets + t], cnt[t]);
+        for (int k = 0; k < t; ++k) start += hist[k] * (k < n ? 4 : 1);
+        if (cnt[t] > 0) at[t] = start + atomicAdd(&hist[kOrderBuckets + t], cnt[t]) * (t < n ? 4 : 1);
+        if (t == 0) num_split = n;
+        if (t == kOrderBuckets - 1) end = start + hist[t] * (t < n ? 4 : 1);
     }
     __syncthreads();
-    if (b >= 0) order[at[b] + rank] = i;
+    if (b >= num_split) order[at[b] + rank] = 8 * i;
+    else if (b >= 0)
+        for (int k = 0; k < 4; ++k) order[at[b] + 4 * rank + k] = 8 * i + 2 * k + 1;
+    for (int k = end + i; k < entries; k += gridDim.x * kOrderBlock) order[k] = -1;
 }
 
 // ------------------------------------------------------------------ kernels ------------------
 
 // Wavefront of a block, -1 past the last: runs of `chunk` go to one XCD (blocks are dispatched
 // round-robin over the eight), so that its L2 serves a compact part of the scene, and the runs in
-// turn to all of them, so that no XCD is left with the cheaper ones.
-__device__ __forceinline__ int64_t tile_wave(const DevParams& p, int64_t b, int chunk, int waves) {
+// turn to all of them, so that no XCD is left with the cheaper ones.  A part of a split wavefront is a
+// wavefront of a quarter of the rays (split).
+__device__ __forceinline__ int64_t tile_wave(DevParams& p, int64_t b, int chunk, int waves, bool& split) {
     const int64_t k = b >> 3;
     const int64_t i = ((k / chunk) * 8 + (b & 7)) * chunk + k % chunk;
+    split = false;
     if (i >= waves) return -1;
-    return p.order ? p.order[i] : i;
+    if (!p.order) return i;
+    const int code = p.order[i];
+    if (code < 0) return -1;
+    split = (code & 1) != 0;
+    if (!split) return code >> 3;
+    p.rays_per_wave >>= 2;
+    return 4 * (int64_t)(code >> 3) + ((code >> 1) & 3);
 }
 
 // Leaves the lanes with mine to the slab stepper.
@@ -643,7 +689,8 @@ k_tile_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int wave
                float* __restrict__ out_rgb, float* __restrict__ out_depth, float* __restrict__ out_opac, DevStats st) {
     __shared__ TileLds W;
     const int lane = threadIdx.x;
-    const int64_t wave = tile_wave(p, blockIdx.x, chunk, waves);
+    bool split;
+    const int64_t wave = tile_wave(p, blockIdx.x, chunk, waves, split);
     if (wave < 0) return;
     const int64_t item = wave_item(p, wave, lane);
     const bool in = item >= 0 && item < num_items;
@@ -681,7 +728,7 @@ k_tile_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int wave
         if (mine) rc.full = tr.full;
     }
     if constexpr (RM == 1) {
-        rc.pos = tr.pos | (max(group, 0) << kTileGroupShift) | kTileRecord;
+        rc.pos = tr.pos | (max(group, 0) << kTileGroupShift) | kTileRecord | (split ? kTileSplit : 0);
         if (lane == 0) ctr.rec_words += 4 * tr.pos;
         if (rs == RAY_NONE && in) {  // padding: no records
             p.rec_len[item] = 0;
@@ -701,14 +748,15 @@ k_tile_backward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int wav
     __shared__ BwdLds S;
     __shared__ GradStage G;
     const int lane = threadIdx.x;
-    const int64_t wave = tile_wave(p, blockIdx.x, chunk, waves);
+    bool split;
+    const int64_t wave = tile_wave(p, blockIdx.x, chunk, waves, split);
     if (wave < 0) return;
     const int64_t item = wave_item(p, wave, lane);
     const bool in = item >= 0 && item < num_items;
     Counters ctr;
     float loss = 0.0f;
     BwdRay b;
-    if (in) backward_setup<RNG, RM>(sc, p, job, wave, lane, item, ray_colors, dLdC, target, loss_kind, st, b, loss);
+    if (in) backward_setup<RNG, RM>(sc, p, job, wave, lane, item, ray_colors, dLdC, target, loss_kind, st, b, loss, split);
     if (target) add_loss(p, loss, lane, st);
     // the rays whose tile the forward recorded, and the others if they can go as a tile too
     const unsigned long long recorded = RM == 2 ? __ballot(b.active && b.tile >= 0) : 0ULL;
@@ -728,7 +776,7 @@ k_tile_backward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int wav
 // Launch of a tile kernel over all wavefronts of a job.
 template <typename K, typename... A>
 void launch_tiles(K kernel, const DevScene& sc, const DevParams& p, const RayJob& job, hipStream_t s, A... args) {
-    const int64_t waves = num_waves(p, job.num_rays);
+    const int64_t waves = p.order && !p.wide ? order_entries(num_waves(p, job.num_rays)) : num_waves(p, job.num_rays);
     // 64 wavefronts of the image's own order, at least 8 runs for each XCD; 8 of the ordered ones
     const int chunk = p.order ? 8 : (int)(waves < 8 * 8 * 64 ? (waves + 63) / 64 : 64);
     const int64_t nb = (waves + 8 * chunk - 1) / (8 * chunk) * (8 * chunk);
@@ -736,8 +784,8 @@ void launch_tiles(K kernel, const DevScene& sc, const DevParams& p, const RayJob
 }
 
 // Fills p.order (dear wavefronts first): from the Gaussians' means (forward), or the records.
-void launch_order(const DevScene& sc, const DevParams& p, const RayJob& job, bool records, unsigned long long* counters,
-                  hipStream_t s) {
+void launch_order(const DevScene& sc, const DevParams& p, const RayJob& job, bool records, int slots,
+                  unsigned long long* counters, hipStream_t s) {
     int* hist = reinterpret_cast<int*>(counters);
     const int waves = (int)num_waves(p, job.num_rays);
     const int first = job.ray_view ? 0 : job.view, views = job.ray_view ? job.num_views : 1;
@@ -749,7 +797,8 @@ void launch_order(const DevScene& sc, const DevParams& p, const RayJob& job, boo
     hipLaunchKernelGGL(k_tile_weight, dim3((waves + 255) / 256), dim3(256), 0, s, p, job, job.num_rays, first, waves,
                        records ? nullptr : p.order_grid, p.order_bucket, hist);
     hipLaunchKernelGGL(k_tile_order, dim3((waves + kOrderBlock - 1) / kOrderBlock), dim3(kOrderBlock), 0, s, waves,
-                       p.order_bucket, hist, p.order, p.order_grid, records ? 0 : views * kGrid * kGrid);
+                       p.order_bucket, hist, p.order, (int)(p.wide ? waves : order_entries(waves)),
+                       p.wide ? 0 : records ? 1 : -1, slots, p.order_grid, records ? 0 : views * kGrid * kGrid);
 }
 
 // Specialised on SPB (8 or 16 samples per slab), on whether the random generator is used and on the
@@ -784,6 +833,8 @@ int rays_per_wave(int64_t num_items) {
     return tiles <= 256 ? 4 : tiles <= 512 ? 8 : tiles <= 1024 ? 16 : tiles <= 3072 ? 32 : 64;
 }
 
+int64_t order_entries(int64_t waves) { return waves + 3 * (waves / kSplitPart); }
+
 int64_t order_grid_cells(int views) { return (int64_t)views * kGrid * kGrid; }
 
 // A block's rays differ by at most eight pixel steps of the image plane along each axis; their unit
@@ -804,7 +855,7 @@ hipError_t launch_forward(const DevScene& sc, const DevParams& p0, const RayJob&
     DevParams p = p0;
     p.wide_count = st.c + 12;
     if (!stepper_only(p)) {
-        if (p.order) launch_order(sc, p, job, false, st.c + 16, s);
+        if (p.order) launch_order(sc, p, job, false, 4096, st.c + 16, s);
         RG_TILE_DISPATCH(p.rec_mode == 1, 1, k_tile_forward, sc, p, job, s, hit_depth, out_rgb, out_depth, out_opacity, st);
         if (!p.wide) return hipGetLastError();
     } else {
@@ -820,7 +871,7 @@ hipError_t launch_backward(const DevScene& sc, const DevParams& p0, const RayJob
     DevParams p = p0;
     p.wide_count = st.c + 13;
     if (!stepper_only(p)) {
-        if (p.order) launch_order(sc, p, job, p.rec_mode == 2, st.c + 48, s);
+        if (p.order) launch_order(sc, p, job, p.rec_mode == 2, 3072, st.c + 48, s);
         RG_TILE_DISPATCH(p.rec_mode == 2, 2, k_tile_backward, sc, p, job, s, ray_colors, dLdC, target, loss_kind, count_stats,
                          gr, st);
         if (!p.wide) return hipGetLastError();

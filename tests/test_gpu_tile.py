@@ -127,3 +127,35 @@ def test_scales_beyond_the_range_of_the_fast_terms(gpu_device, power):
                          fovx_deg=40.0).launch_record()
     st = _compare(sc, prm, [cam], gpu_device, np.zeros(384), np.arange(384), 512)
     assert st["slab_hits"] > 0
+
+
+@pytest.mark.parametrize("words", [0, 64, 2048])
+@pytest.mark.parametrize("w,h", [(264, 520), (447, 455)])
+def test_split_wavefronts(gpu_device, w, h, words):
+    """Whole views with a dense spot: the dear wavefronts (of 32 rays and of 64, with ragged edges) march
+    in quarters, forward and backward; a backward of another view does not take their records."""
+    sc = scenes.scene_uniform(6000, seed=7)
+    sc.positions[:5000] = 0.08 * sc.positions[:5000] + 0.3
+    sc.scales[:5000] *= 0.2
+    prm = scenes.RenderParams(dt=0.01, t_eps=1e-4, white_background=True)
+    cams = [_view(w, h), _view(w, h, az=75.0)]
+    gen = torch.Generator(device=gpu_device).manual_seed(3)
+    dL = torch.randn((w * h, 3), generator=gen, device=gpu_device)
+    out = {}
+    for packet in (False, True):
+        rc, _ = prepared_caster(sc, prm, cams, gpu_device, TuneConfig(packet=packet, replay_words=words))
+        img = [rc.forward(v, None, depth=True, opacity=True) for v in (1, 0)]
+        st = rc.stats()
+        grads = []
+        for v in (0, 1):
+            rc.backward(v, None, img[1 - v][0], dL, rc.last_token)
+            assert rc.stats()["dropped"] == 0
+            grads.append({k: t.cpu().numpy() for k, t in rc.finish_grads().items() if t is not None})
+        out[packet] = (img, st, grads)
+    a, b = out[False], out[True]
+    for v in range(2):
+        for i in range(3):
+            assert torch.equal(a[0][v][i], b[0][v][i]), (v, i)
+        for k, t in a[2][v].items():
+            assert max_rel(b[2][v][k], t) <= 1e-5, (v, k)
+    assert a[1]["slab_hits"] == b[1]["slab_hits"] > 0 and a[1]["pairs"] == b[1]["pairs"]
