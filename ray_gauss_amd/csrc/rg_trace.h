@@ -96,25 +96,32 @@ __device__ __forceinline__ float sample_alpha(float s, float dt) {
     return 1.0f - __builtin_amdgcn_exp2f(s * (dt * kNegLog2e));
 }
 
-// colorBlending (forward/gaussians_aabb.cu:500-519) + depth (cuda_gui/gaussians_aabb.cu:415).
+// colorBlending (forward/gaussians_aabb.cu:500-519) + depth (cuda_gui/gaussians_aabb.cu:415) where it is
+// asked for.
 template <int SPB, bool RNG>
 __device__ __forceinline__ void composite(const float* sig, const float* cr, const float* cg, const float* cb, float tb,
-                                          unsigned int seed, const DevParams& p, RayOut& o) {
+                                          unsigned int seed, const DevParams& p, bool depth, RayOut& o) {
     unsigned int st = seed;
+    float ta[SPB];
 #pragma unroll
     for (int i = 0; i < SPB; ++i) {
         if (SPB > 8 && i >= p.spb) break;
         const float s = sig[i];
         const float alpha = sample_alpha(s, p.dt);
         // colour = sums / sigma: one reciprocal per sample (a sample without hits has zero sums)
-        const float inv = s > 0.0f ? __builtin_amdgcn_rcpf(s) : 0.0f;
+        const float inv = __builtin_amdgcn_rcpf(fmaxf(s, 0x1p-126f));
         const float r = cr[i] * inv, g = cg[i] * inv, b = cb[i] * inv;
-        const float ta = o.T * alpha;
-        o.C[0] += ta * r;
-        o.C[1] += ta * g;
-        o.C[2] += ta * b;
-        o.depth += ta * sample_t(tb, i, p.dt, RNG ? p.rnd_sample : 0, st);
+        ta[i] = o.T * alpha;
+        o.C[0] += ta[i] * r;
+        o.C[1] += ta[i] * g;
+        o.C[2] += ta[i] * b;
         o.T *= 1.0f - alpha;
+    }
+    if (!depth) return;
+#pragma unroll
+    for (int i = 0; i < SPB; ++i) {
+        if (SPB > 8 && i >= p.spb) break;
+        o.depth += ta[i] * sample_t(tb, i, p.dt, RNG ? p.rnd_sample : 0, st);
     }
 }
 

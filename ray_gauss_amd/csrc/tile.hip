@@ -70,9 +70,11 @@ __device__ __forceinline__ void tile_list(TileWalk& w, const DevScene& sc, float
 
 // The lanes of the next round: its depths [tlag, whi] and whether this lane takes part.
 __device__ __forceinline__ bool tile_window(bool alive, float tb, float slab, float& tlag, float& whi) {
-    tlag = uniform_f(wave_min64f(alive ? tb : INFINITY));
+    // depths are not negative: their order is that of their bits
+    const int bits = __float_as_int(tb);
+    tlag = __int_as_float(__builtin_amdgcn_readfirstlane(wave_min64(alive ? bits : 0x7f800000)));
     const bool part = alive && tb < tlag + kTileSync * slab;
-    whi = add_exact(uniform_f(wave_max64f(part ? tb : -INFINITY)), slab);
+    whi = add_exact(__int_as_float(__builtin_amdgcn_readfirstlane(~wave_min64(part ? ~bits : INT_MAX))), slab);
     return part;
 }
 
@@ -131,7 +133,7 @@ __device__ __forceinline__ void tile_rec_round(TileRec& r, float tlag, int view,
 template <int SPB, bool RNG, int RM>
 __device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams& p, bool act, const Ray& ray,
                                              unsigned int& seed, int view, const float* cam_u, int group, int hit_depth,
-                                             TileLds& W, int lane,
+                                             bool want_depth, TileLds& W, int lane,
                                              Counters& ctr, RayOut& o, TileRec& rc) {
     const float slab = p.dt * (float)p.spb;
     const float4* __restrict__ rgbv = sc.rgb + (size_t)view * sc.n;
@@ -141,7 +143,8 @@ __device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams
     bool alive = act && o.T > p.t_eps;
     float tb = ray.tenter;
     // sums of a round that goes on with another list, in memory: few do, and the registers are the gather's
-    volatile float held[4 * SPB];
+    float held_sums[4 * SPB];
+    __attribute__((address_space(5))) volatile float* held = (__attribute__((address_space(5))) volatile float*)held_sums;
     int nh = 0;
     bool any = false;  // the round has candidates
     while (__ballot(alive) != 0ULL) {
@@ -233,7 +236,7 @@ __device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams
                 ctr.K += nh;
                 if (p.max_hits > 0 && nh > p.max_hits) ctr.ovf++;
                 if (nh > hit_depth) ctr.fallback++;
-                composite<SPB, RNG>(sig, cr, cg, cb, tb, seed, p, o);
+                composite<SPB, RNG>(sig, cr, cg, cb, tb, seed, p, want_depth, o);
                 if (RNG && p.rnd_sample == 1) seed = skip_draws(seed, p.spb);  // the slab's draws are spent
             }
             const float nt = add_exact(tb, slab);
@@ -724,7 +727,7 @@ k_tile_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int wave
         const unsigned long long m = __ballot(mine);
         if (m == 0ULL) break;
         const int view = __builtin_amdgcn_readlane(q.view, __ffsll((long long)m) - 1);
-        forward_tile<SPB, RNG, RM>(sc, p, mine, ray, seed, view, job.cams[view].u, g, hit_depth, W, lane, ctr, o, tr);
+        forward_tile<SPB, RNG, RM>(sc, p, mine, ray, seed, view, job.cams[view].u, g, hit_depth, out_depth != nullptr, W, lane, ctr, o, tr);
         if (mine) rc.full = tr.full;
     }
     if constexpr (RM == 1) {

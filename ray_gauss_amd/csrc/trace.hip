@@ -464,7 +464,7 @@ __device__ __forceinline__ bool forward_step(const DevScene& sc, const DevParams
     if (hit) *hit = nh > 0;
     if (p.max_hits > 0 && nh > p.max_hits) ctr.ovf++;
     if (nh > 0) {
-        composite<SPB, RNG>(sig, cr, cg, cb, tb, seed, p, o);
+        composite<SPB, RNG>(sig, cr, cg, cb, tb, seed, p, true, o);
         if (RNG && p.rnd_sample == 1) seed = skip_draws(seed, p.spb);  // the slab's draws are spent
     }
     return advance_slab(s, p);
