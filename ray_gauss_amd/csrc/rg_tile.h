@@ -34,8 +34,17 @@ struct Beam {
     float rmin[3], rmax[3];  // 1 / dmin, 1 / dmax
 };
 
+// A slab's samples in wavefronts that hold one in each lane (spread), exchanged between a ray's eight lanes.
+struct SpreadLds {
+    float alpha[kWave], rest[kWave];
+    float v[4][kWave];
+};
+
 struct TileLds {
-    int stack[kTileStack];
+    union {
+        int stack[kTileStack];  // during a gather
+        SpreadLds spread;       // after the round's hits
+    };
     int slot[kTileCand];                 // 2 slot + 1 where the terms are out of inv_sqrt_exact's range
     float4 oc[kTileCand];                // the predicate's O' = M' (o - mu) and c = |O'|^2 - 1
     float z0[kTileCand], z1[kTileCand];  // depth range in which the beam can meet the candidate

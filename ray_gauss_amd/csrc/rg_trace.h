@@ -205,6 +205,25 @@ __device__ __forceinline__ void ray_in_ellipsoid(const float4 g1, const float4 g
 // lanes and expand the sum once per Gaussian (expand_grad) instead of once per lane.
 constexpr int kMoments = 13;
 
+// The moments of a ray from its four sums.
+__device__ __forceinline__ void ray_moments(const float* P, const float* D, float sigma, float S0, float T1, float T2,
+                                            float Sc, const float* dL, float* v) {
+    float W[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        v[a] = P[a] * S0 + D[a] * T1;
+        W[a] = P[a] * T1 + D[a] * T2;
+    }
+    // with U = Gy' and W = P T1 + D T2: Y'_ab = P_a U_b + D_a W_b; (0,0) (1,1) (2,2) (0,1) (0,2) (1,2)
+    const int ya[6] = {0, 1, 2, 0, 0, 1}, yb[6] = {0, 1, 2, 1, 2, 2};
+#pragma unroll
+    for (int k = 0; k < 6; ++k) v[3 + k] = P[ya[k]] * v[yb[k]] + D[ya[k]] * W[yb[k]];
+    v[9] = S0 * __builtin_amdgcn_rcpf(sigma);
+    v[10] = dL[0] * Sc;
+    v[11] = dL[1] * Sc;
+    v[12] = dL[2] * Sc;
+}
+
 template <int SPB, bool RNG>
 __device__ __forceinline__ void grad_moments(const float* P, const float* D, float sigma, const float* m, float tc, float F,
                                              float tb, unsigned int seed, const DevParams& p, const float* Gq,
@@ -221,20 +240,7 @@ __device__ __forceinline__ void grad_moments(const float* P, const float* D, flo
         T2 += wp * (tau * tau);
         Sc += m[i] * Bq[i];
     }
-    float W[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        v[a] = P[a] * S0 + D[a] * T1;
-        W[a] = P[a] * T1 + D[a] * T2;
-    }
-    // with U = Gy' and W = P T1 + D T2: Y'_ab = P_a U_b + D_a W_b; (0,0) (1,1) (2,2) (0,1) (0,2) (1,2)
-    const int ya[6] = {0, 1, 2, 0, 0, 1}, yb[6] = {0, 1, 2, 1, 2, 2};
-#pragma unroll
-    for (int k = 0; k < 6; ++k) v[3 + k] = P[ya[k]] * v[yb[k]] + D[ya[k]] * W[yb[k]];
-    v[9] = S0 * __builtin_amdgcn_rcpf(sigma);
-    v[10] = dL[0] * Sc;
-    v[11] = dL[1] * Sc;
-    v[12] = dL[2] * Sc;
+    ray_moments(P, D, sigma, S0, T1, T2, Sc, dL, v);
 }
 
 // The 14 gradient values of one Gaussian from its summed moments m (grad_moments):
@@ -565,10 +571,11 @@ template <bool RNG, int RM>
 __device__ __forceinline__ void backward_setup(const DevScene& sc, const DevParams& p, const RayJob& job, int64_t wave,
                                                int lane, int64_t item, const float* __restrict__ ray_colors,
                                                const float* __restrict__ dLdC, const float* __restrict__ target,
-                                               int loss_kind, DevStats st, BwdRay& b, float& loss, bool split = false) {
+                                               int loss_kind, DevStats st, BwdRay& b, float& loss, bool split = false,
+                                               bool lead = true) {
     RayRef q;
     const int rs = resolve(job, item, q);
-    if (rs == RAY_BAD) atomicAdd(&st.c[C_BAD], 1ull);
+    if (rs == RAY_BAD && lead) atomicAdd(&st.c[C_BAD], 1ull);
     if (rs != RAY_OK) return;
     b.Cf[0] = ray_colors[3 * q.out];
     b.Cf[1] = ray_colors[3 * q.out + 1];

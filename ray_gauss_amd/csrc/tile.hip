@@ -129,8 +129,83 @@ __device__ __forceinline__ void tile_rec_round(TileRec& r, float tlag, int view,
     r.n = 0;
 }
 
+// Spread wavefronts: at most eight rays, each in eight lanes, one sample of the slab per lane (lane = 8 ray +
+// sample).  An event then takes the arithmetic of one sample instead of eight, and a lane sums its sample over
+// the events in their order, as elsewhere.  They are the wavefronts of small jobs and the parts of split
+// ones: fewer than the GPU holds, and each nearly alone on its SIMD, where the length of its chain of
+// instructions is its time.  One 64x64 view of 4096 Gaussians: forward 158 -> 137 us, backward 185 -> 150;
+// 30k Gaussians with random samples (parts of 32-ray wavefronts) 384 -> 362 and 465 -> 399.
+
+// Depth of the lane's sample.
+template <bool RNG>
+__device__ __forceinline__ float spread_t(float tb, int i, unsigned int seed, const DevParams& p) {
+    unsigned int st = seed;
+    if (!RNG || p.rnd_sample != 1) return sample_t(tb, i, p.dt, RNG ? p.rnd_sample : 0, st);
+    float t = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const float tk = sample_t(tb, k, p.dt, p.rnd_sample, st);
+        t = k == i ? tk : t;
+    }
+    return t;
+}
+
+// Density of a hit at the lane's sample, zero at or below thr.
+__device__ __forceinline__ float spread_density(const Isect& I, float sigma, float t, float thr) {
+    const float sw = sigma * weight(wexp(I), t - I.tc);
+    return sw > thr ? sw : 0.0f;
+}
+
+// composite over the eight lanes of a ray: T, which all have, and in each lane one of the colours' or the
+// depth's sums (lane & 3), in the order of the samples.
+__device__ __forceinline__ void spread_composite(float sig, float cr, float cg, float cb, float t, const DevParams& p,
+                                                 SpreadLds& X, int lane, float& T, float& sum) {
+    const float alpha = sample_alpha(sig, p.dt);
+    const float inv = __builtin_amdgcn_rcpf(fmaxf(sig, 0x1p-126f));
+    X.alpha[lane] = alpha;
+    X.rest[lane] = 1.0f - alpha;
+    X.v[0][lane] = cr * inv;
+    X.v[1][lane] = cg * inv;
+    X.v[2][lane] = cb * inv;
+    X.v[3][lane] = t;
+    __builtin_amdgcn_wave_barrier();
+    const int first = lane & 56, c = lane & 3;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float ta = T * X.alpha[first + j];
+        sum += ta * X.v[c][first + j];
+        T *= X.rest[first + j];
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+
+// slab_coeffs for the lane's sample: overwrites (sig, ep) with its (G, Bq).
+__device__ __forceinline__ void spread_coeffs(float& sig, float& ep, const DevParams& p, SpreadLds& X, int lane, float& T,
+                                              float& Dr) {
+    const float alpha = sample_alpha(sig, p.dt);
+    const float inv = sig > 0.0f ? __builtin_amdgcn_rcpf(sig) : 0.0f;
+    const float E = ep * inv;
+    X.alpha[lane] = alpha;
+    X.rest[lane] = 1.0f - alpha;
+    X.v[0][lane] = E;
+    __builtin_amdgcn_wave_barrier();
+    const int first = lane & 56;
+    float Ti = T, Di = Dr;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        Ti = (lane & 7) == j ? T : Ti;
+        Di = (lane & 7) == j ? Dr : Di;
+        Dr -= T * X.alpha[first + j] * X.v[0][first + j];
+        T *= X.rest[first + j];
+    }
+    __builtin_amdgcn_wave_barrier();
+    const float Bq = Ti * alpha * inv;
+    sig = p.dt * (Ti * E - Di) - Bq * E;
+    ep = Bq;
+}
+
 // Forward of the lanes with act, which share their view, as one beam.  Called by all 64 lanes.
-template <int SPB, bool RNG, int RM>
+template <int SPB, bool RNG, int RM, bool SPREAD>
 __device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams& p, bool act, const Ray& ray,
                                              unsigned int& seed, int view, const float* cam_u, int group, int hit_depth,
                                              bool want_depth, TileLds& W, int lane,
@@ -143,7 +218,8 @@ __device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams
     bool alive = act && o.T > p.t_eps;
     float tb = ray.tenter;
     // sums of a round that goes on with another list, in memory: few do, and the registers are the gather's
-    float held_sums[4 * SPB];
+    constexpr int NS = SPREAD ? 1 : SPB;  // samples of a lane
+    float held_sums[4 * NS];
     __attribute__((address_space(5))) volatile float* held = (__attribute__((address_space(5))) volatile float*)held_sums;
     int nh = 0;
     bool any = false;  // the round has candidates
@@ -152,12 +228,12 @@ __device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams
         const bool part = tile_window(alive, tb, slab, tlag, whi);
         tile_list(w, sc, tlag, whi, slab, true, W, lane, alive, ctr);
         const float tmin = fmaxf(ray.tenter, tb), tmax = fminf(ray.texit, add_exact(tb, slab));
-        float sig[SPB], cr[SPB], cg[SPB], cb[SPB];
+        float sig[NS], cr[NS], cg[NS], cb[NS];
 #pragma unroll
-        for (int i = 0; i < SPB; ++i) sig[i] = cr[i] = cg[i] = cb[i] = 0.0f;
+        for (int i = 0; i < NS; ++i) sig[i] = cr[i] = cg[i] = cb[i] = 0.0f;
         if (w.first > 0) {
 #pragma unroll
-            for (int i = 0; i < SPB; ++i) {
+            for (int i = 0; i < NS; ++i) {
                 sig[i] = held[4 * i];
                 cr[i] = held[4 * i + 1];
                 cg[i] = held[4 * i + 2];
@@ -167,6 +243,7 @@ __device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams
             nh = 0;
             any = false;
         }
+        const float ts = SPREAD ? spread_t<RNG>(tb, lane & 7, seed, p) : 0.0f;
         // at: the candidate's place in the list, or -1
         auto eval = [&](int slot, int at, bool cond) {
             const float4 g0 = ld_uniform(sc.geo, 4 * (int64_t)slot), g1 = ld_uniform(sc.geo, 4 * (int64_t)slot + 1),
@@ -182,7 +259,16 @@ __device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams
             }
             if (hit) {
                 refine_sampling(g0, g1, g2, g3, ray, I);
-                accum_hit<SPB, RNG>(I, g0.w, ld_uniform(rgbv, slot), tb, seed, p, sig, cr, cg, cb);
+                if constexpr (SPREAD) {
+                    const float4 col = ld_uniform(rgbv, slot);
+                    const float m = spread_density(I, g0.w, ts, p.sigma_thr);
+                    sig[0] += m;
+                    cr[0] += m * col.x;
+                    cg[0] += m * col.y;
+                    cb[0] += m * col.z;
+                } else {
+                    accum_hit<SPB, RNG>(I, g0.w, ld_uniform(rgbv, slot), tb, seed, p, sig, cr, cg, cb);
+                }
                 if (tb == ray.tenter || I.r1 > tmin) ctr.P++;
                 ++nh;
             }
@@ -214,7 +300,7 @@ __device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams
             w.valid = false;
         } else if (w.limit < sc.total_nodes) {  // the round goes on with its other leaves
 #pragma unroll
-            for (int i = 0; i < SPB; ++i) {
+            for (int i = 0; i < NS; ++i) {
                 held[4 * i] = sig[i];
                 held[4 * i + 1] = cr[i];
                 held[4 * i + 2] = cg[i];
@@ -236,7 +322,8 @@ __device__ __forceinline__ void forward_tile(const DevScene& sc, const DevParams
                 ctr.K += nh;
                 if (p.max_hits > 0 && nh > p.max_hits) ctr.ovf++;
                 if (nh > hit_depth) ctr.fallback++;
-                composite<SPB, RNG>(sig, cr, cg, cb, tb, seed, p, want_depth, o);
+                if constexpr (SPREAD) spread_composite(sig[0], cr[0], cg[0], cb[0], ts, p, W.spread, lane, o.T, o.C[0]);
+                else composite<SPB, RNG>(sig, cr, cg, cb, tb, seed, p, want_depth, o);
                 if (RNG && p.rnd_sample == 1) seed = skip_draws(seed, p.spb);  // the slab's draws are spent
             }
             const float nt = add_exact(tb, slab);
@@ -263,11 +350,21 @@ struct KeptEvents {
     float4 ptc[kKept][kWave];   // the offset P and t_c
 };
 
+// The same of a spread wavefront, behind the exchange area, which lies where a walked tile's does.
+constexpr int kKeptSpread = 8;
+struct KeptSpread {
+    SpreadLds X;
+    float m[kKeptSpread][kWave];
+    float4 ptc[kKeptSpread][kWave];
+};
+
 // A walked tile holds its candidates, a replayed one its round's kept events.
 union BwdLds {
     TileLds W;
     KeptEvents K;
+    KeptSpread S;
 };
+static_assert(sizeof(KeptSpread) <= sizeof(KeptEvents) && sizeof(TileLds) <= sizeof(KeptEvents), "LDS of a backward");
 
 // Backward of the lanes with act, called by all 64 lanes.  In each round the wavefront has a list
 // of events -- a Gaussian and the lanes that hit it in their slab of the round -- which it goes
@@ -275,7 +372,7 @@ union BwdLds {
 // and to sum each Gaussian's gradient moments over its lanes.  The events come from the forward's
 // record of the tile (cells; lanes take part with their beam in it, tile, -1: none), and for the lanes with walk, once it ends, from the
 // tile's own gathers.
-template <int SPB, bool RNG>
+template <int SPB, bool RNG, bool SPREAD>
 __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParams& p, const rg_camera* cams, bool act, const Ray& ray,
                                               unsigned int seed, int view, const float* Cfwd, const float* dL,
                                               const u32x4* __restrict__ cells, int num_cells, int tile, bool walk,
@@ -357,9 +454,11 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
         const float tmin = fmaxf(ray.tenter, tb), tmax = fminf(ray.texit, add_exact(tb, slab));
         const unsigned int cur_seed = seed;
         // the density sums and the projected colour sums, then the coefficients G_i, Bq_i
-        float sig[SPB], ep[SPB];
+        constexpr int NS = SPREAD ? 1 : SPB;  // samples of a lane
+        float sig[NS], ep[NS];
 #pragma unroll
-        for (int i = 0; i < SPB; ++i) sig[i] = ep[i] = 0.0f;
+        for (int i = 0; i < NS; ++i) sig[i] = ep[i] = 0.0f;
+        const float ts = SPREAD ? spread_t<RNG>(tb, lane & 7, seed, p) : 0.0f;
         int nh = 0;
         bool any = false, one = false;  // the round has candidates; its events fit one batch
         int ne = 0;
@@ -455,7 +554,8 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
             float bq, cq;
             isect_terms(g0, g1, g2, g3, ray, I, bq, cq);
             refine_sampling(g0, g1, g2, g3, ray, I);
-            sample_densities<SPB, RNG>(I, g0.w, tb, cur_seed, p, md);
+            if constexpr (SPREAD) md[0] = spread_density(I, g0.w, ts, p.sigma_thr);
+            else sample_densities<SPB, RNG>(I, g0.w, tb, cur_seed, p, md);
             return make_float4(I.Px, I.Py, I.Pz, I.tc);
         };
         each_event(false, [&](int number, int slot, bool in) {
@@ -463,10 +563,19 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
                          g2 = ld_uniform(sc.geo, 4 * (int64_t)slot + 2), g3 = ld_uniform(sc.geo, 4 * (int64_t)slot + 3);
             const float4 col = ld_uniform(rgbv, slot);
             if (!in) return;
-            float md[SPB];
+            float md[NS];
             const float4 ptc = densities(g0, g1, g2, g3, md);
-            accum_densities<SPB>(md, project_color(dL, col), p, sig, ep);
-            if constexpr (SPB == 8) {
+            if constexpr (SPREAD) {
+                sig[0] += md[0];
+                ep[0] += md[0] * project_color(dL, col);
+                if (replay && number < kKeptSpread) {
+                    S.S.m[number][lane] = md[0];
+                    S.S.ptc[number][lane] = ptc;
+                }
+            } else {
+                accum_densities<SPB>(md, project_color(dL, col), p, sig, ep);
+            }
+            if constexpr (SPB == 8 && !SPREAD) {
                 if (replay && number < kKept) {
                     S.K.m[number][0][lane] = make_float4(md[0], md[1], md[2], md[3]);
                     S.K.m[number][1][lane] = make_float4(md[4], md[5], md[6], md[7]);
@@ -476,7 +585,8 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
             ++nh;
         });
         if (nh > 0) {
-            slab_coeffs<SPB>(sig, ep, p, T, Dr);
+            if constexpr (SPREAD) spread_coeffs(sig[0], ep[0], p, W.spread, lane, T, Dr);
+            else slab_coeffs<SPB>(sig, ep, p, T, Dr);
             if (RNG && p.rnd_sample == 1) seed = skip_draws(seed, p.spb);  // the slab's draws are spent
         }
         if (__builtin_amdgcn_ballot_w64(nh > 0) != 0ULL) {
@@ -488,10 +598,13 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
 #pragma unroll
                 for (int k = 0; k < kMoments; ++k) v[k] = 0.0f;
                 if (in) {
-                    float md[SPB];
+                    float md[NS];
                     float4 ptc;
-                    if (SPB == 8 && replay && number < kKept) {
-                        if constexpr (SPB == 8) {
+                    if (SPB == 8 && replay && number < (SPREAD ? kKeptSpread : kKept)) {
+                        if constexpr (SPREAD) {
+                            md[0] = S.S.m[number][lane];
+                            ptc = S.S.ptc[number][lane];
+                        } else if constexpr (SPB == 8) {
                             const float4 a = S.K.m[number][0][lane], b = S.K.m[number][1][lane];
                             md[0] = a.x, md[1] = a.y, md[2] = a.z, md[3] = a.w;
                             md[4] = b.x, md[5] = b.y, md[6] = b.z, md[7] = b.w;
@@ -503,7 +616,13 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
                     const float P[3] = {ptc.x, ptc.y, ptc.z};
                     float D[3];
                     ray_in_ellipsoid(g1, g2, g3, ray, D);
-                    grad_moments<SPB, RNG>(P, D, g0.w, md, ptc.w, project_color(dL, col), tb, cur_seed, p, sig, ep, dL, v);
+                    if constexpr (SPREAD) {
+                        const float tau = ts - ptc.w;
+                        const float wp = md[0] * (sig[0] + ep[0] * project_color(dL, col));
+                        ray_moments(P, D, g0.w, wp, wp * tau, wp * (tau * tau), md[0] * ep[0], dL, v);
+                    } else {
+                        grad_moments<SPB, RNG>(P, D, g0.w, md, ptc.w, project_color(dL, col), tb, cur_seed, p, sig, ep, dL, v);
+                    }
                 }
                 grad_scatter_wave(v, key_base + slot, sc, gr, lane, G, nst, drops);
             });
@@ -539,7 +658,8 @@ constexpr int kSplats = 1 << 20;        // Gaussians counted at most (every k-th
 constexpr int kOrderBuckets = 32;       // half octaves of the weight
 constexpr int kOrderBlock = 1024;
 // A wavefront that costs more than an even share of the launch ends after the others however early it
-// starts, so it is split into quarters of its rays (narrower beams: each takes about half its time).  A
+// starts, so it is split into quarters of its rays (narrower beams: each takes about half its time; in
+// eighths, spread ones, the parts of 64 rays cost more together than they shorten: 1.10 ms instead of 0.99).  A
 // backward takes the forward's parts with its records.  The weights exaggerate: with shares 0.5 / 1 / 2 / 4 / none
 // (times an even one) a forward of one view of 100k Gaussians in blobs took 0.99 / 1.02 / 0.99 / 1.30 /
 // 1.55 ms, its backward 1.18 / 1.19 / 1.10 / 1.28 / 1.54, one at four times the slabs 1.61 / 1.72 / 1.83 / 2.72 / 3.26,
@@ -547,6 +667,9 @@ constexpr int kOrderBlock = 1024;
 // may have wavefronts that are no beams, are not split.
 constexpr float kSplitShare = 2.0f;
 constexpr int kSplitPart = 8;
+// Rays of a part of a split wavefront: a quarter, but no fewer than a spread one holds.
+__host__ __device__ inline int split_rays(const DevParams& p) { return max(p.rays_per_wave / 4, min(p.rays_per_wave, 8)); }
+
 
 __global__ void __launch_bounds__(256) k_tile_splat(int n, int stride, const float4* __restrict__ geo,
                                                     const rg_camera* __restrict__ cams, int first_view,
@@ -605,7 +728,7 @@ __global__ void __launch_bounds__(256) k_tile_weight(DevParams p, RayJob job, in
     if (threadIdx.x < kOrderBuckets && cnt[threadIdx.x] > 0) atomicAdd(&hist[threadIdx.x], cnt[threadIdx.x]);
 }
 
-// The heaviest buckets whose wavefronts are split in four: those with more than kSplitShare of an even share of
+// The heaviest buckets whose wavefronts are split: those with more than kSplitShare of an even share of
 // the whole weight, as long as they are at most 1 / kSplitPart of the wavefronts.
 __device__ __forceinline__ int split_buckets(const int* hist, int waves, int slots) {
     float total = 0.0f;
@@ -620,12 +743,13 @@ __device__ __forceinline__ int split_buckets(const int* hist, int waves, int slo
 }
 
 // The wavefronts by falling weight, near their own order within a bucket (hist: the buckets' sizes, then
-// their cursors), as 8 wave, or for each quarter k of a split one 8 wave + 2 k + 1, and -1 in the rest of
+// their cursors), as 16 wave, or for each part k of a split one 16 wave + 2 k + 1, and -1 in the rest of
 // the list; clears the grid for the next job.  split: the number of heaviest buckets that are split, -1: by
 // their weight.
 __global__ void __launch_bounds__(kOrderBlock) k_tile_order(int waves, const unsigned char* __restrict__ bucket,
                                                             int* __restrict__ hist, int* __restrict__ order, int entries,
-                                                            int split, int slots, unsigned int* grid, int cells) {
+                                                            int split, int parts, int slots, unsigned int* grid,
+                                                            int cells) {
     __shared__ int cnt[kOrderBuckets], at[kOrderBuckets], num_split, end;
     const int t = threadIdx.x, i = blockIdx.x * kOrderBlock + t;
     if (t < kOrderBuckets) cnt[t] = 0;
@@ -647,15 +771,15 @@ __global__ void __launch_bounds__(kOrderBlock) k_tile_order(int waves, const uns
         int n = split >= 0 ? split : split_buckets(hist, waves, slots);
         if (split == 1 && hist[0] > waves / kSplitPart) n = 0;  // never expected: not this job's records
         int start = 0;
-        for (int k = 0; k < t; ++k) start += hist[k] * (k < n ? 4 : 1);
-        if (cnt[t] > 0) at[t] = start + atomicAdd(&hist[kOrderBuckets + t], cnt[t]) * (t < n ? 4 : 1);
+        for (int k = 0; k < t; ++k) start += hist[k] * (k < n ? parts : 1);
+        if (cnt[t] > 0) at[t] = start + atomicAdd(&hist[kOrderBuckets + t], cnt[t]) * (t < n ? parts : 1);
         if (t == 0) num_split = n;
-        if (t == kOrderBuckets - 1) end = start + hist[t] * (t < n ? 4 : 1);
+        if (t == kOrderBuckets - 1) end = start + hist[t] * (t < n ? parts : 1);
     }
     __syncthreads();
-    if (b >= num_split) order[at[b] + rank] = 8 * i;
+    if (b >= num_split) order[at[b] + rank] = 16 * i;
     else if (b >= 0)
-        for (int k = 0; k < 4; ++k) order[at[b] + 4 * rank + k] = 8 * i + 2 * k + 1;
+        for (int k = 0; k < parts; ++k) order[at[b] + parts * rank + k] = 16 * i + 2 * k + 1;
     for (int k = end + i; k < entries; k += gridDim.x * kOrderBlock) order[k] = -1;
 }
 
@@ -664,7 +788,7 @@ __global__ void __launch_bounds__(kOrderBlock) k_tile_order(int waves, const uns
 // Wavefront of a block, -1 past the last: runs of `chunk` go to one XCD (blocks are dispatched
 // round-robin over the eight), so that its L2 serves a compact part of the scene, and the runs in
 // turn to all of them, so that no XCD is left with the cheaper ones.  A part of a split wavefront is a
-// wavefront of a quarter of the rays (split).
+// wavefront of split_rays rays (split).
 __device__ __forceinline__ int64_t tile_wave(DevParams& p, int64_t b, int chunk, int waves, bool& split) {
     const int64_t k = b >> 3;
     const int64_t i = ((k / chunk) * 8 + (b & 7)) * chunk + k % chunk;
@@ -674,28 +798,32 @@ __device__ __forceinline__ int64_t tile_wave(DevParams& p, int64_t b, int chunk,
     const int code = p.order[i];
     if (code < 0) return -1;
     split = (code & 1) != 0;
-    if (!split) return code >> 3;
-    p.rays_per_wave >>= 2;
-    return 4 * (int64_t)(code >> 3) + ((code >> 1) & 3);
+    if (!split) return code >> 4;
+    const int parts = p.rays_per_wave / split_rays(p);
+    p.rays_per_wave = split_rays(p);
+    return (int64_t)(code >> 4) * parts + ((code >> 1) & 7);
 }
 
 // Leaves the lanes with mine to the slab stepper.
+template <bool SPREAD>
 __device__ __forceinline__ void tile_leave(const DevParams& p, int64_t wave, bool mine, int lane) {
-    const unsigned long long m = __ballot(mine);
+    unsigned long long m = __ballot(mine);
+    if (SPREAD) {  // in the stepper a lane has a ray
+        unsigned long long rays = 0ULL;
+        for (int r = 0; r < 8; ++r) rays |= ((m >> (8 * r)) & 1ULL) << r;
+        m = rays;
+    }
     if (lane == 0)
         p.wide[atomicAdd(p.wide_count, 1ull)] = make_int4((int)wave, (int)(unsigned int)m, (int)(unsigned int)(m >> 32), 0);
 }
 
-template <int SPB, bool RNG, int RM>
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(SPB == 8 ? 4 : 3)))
-k_tile_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int waves, int chunk, int hit_depth,
-               float* __restrict__ out_rgb, float* __restrict__ out_depth, float* __restrict__ out_opac, DevStats st) {
-    __shared__ TileLds W;
-    const int lane = threadIdx.x;
-    bool split;
-    const int64_t wave = tile_wave(p, blockIdx.x, chunk, waves, split);
-    if (wave < 0) return;
-    const int64_t item = wave_item(p, wave, lane);
+template <int SPB, bool RNG, int RM, bool SPREAD>
+__device__ __forceinline__ void forward_wave(const DevScene& sc, const DevParams& p, const RayJob& job, int64_t num_items,
+                                             int64_t wave, bool split, int hit_depth, float* __restrict__ out_rgb,
+                                             float* __restrict__ out_depth, float* __restrict__ out_opac, DevStats st,
+                                             TileLds& W, int lane) {
+    const bool lead = !SPREAD || (lane & 7) == 0;  // of the ray's lanes
+    const int64_t item = wave_item(p, wave, SPREAD ? lane >> 3 : lane);
     const bool in = item >= 0 && item < num_items;
     Counters ctr;
     RayRef q;
@@ -713,7 +841,7 @@ k_tile_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int wave
     }
     int group = 0;  // one view, all of it narrow
     if (p.wide && !tile_groups(sc, alive, q.view, ray, group)) {
-        tile_leave(p, wave, in, lane);
+        tile_leave<SPREAD>(p, wave, in, lane);
         return;
     }
     Rec rc;
@@ -727,20 +855,76 @@ k_tile_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int wave
         const unsigned long long m = __ballot(mine);
         if (m == 0ULL) break;
         const int view = __builtin_amdgcn_readlane(q.view, __ffsll((long long)m) - 1);
-        forward_tile<SPB, RNG, RM>(sc, p, mine, ray, seed, view, job.cams[view].u, g, hit_depth, out_depth != nullptr, W, lane, ctr, o, tr);
+        forward_tile<SPB, RNG, RM, SPREAD>(sc, p, mine, ray, seed, view, job.cams[view].u, g, hit_depth,
+                                           out_depth != nullptr, W, lane, ctr, o, tr);
         if (mine) rc.full = tr.full;
+    }
+    if constexpr (SPREAD) {  // the sums of the ray's lanes
+        const float sum = o.C[0];
+        for (int c = 0; c < 3; ++c) o.C[c] = __shfl(sum, (lane & 56) + c);
+        o.depth = __shfl(sum, (lane & 56) + 3);
     }
     if constexpr (RM == 1) {
         rc.pos = tr.pos | (max(group, 0) << kTileGroupShift) | kTileRecord | (split ? kTileSplit : 0);
         if (lane == 0) ctr.rec_words += 4 * tr.pos;
-        if (rs == RAY_NONE && in) {  // padding: no records
+        if (rs == RAY_NONE && in && lead) {  // padding: no records
             p.rec_len[item] = 0;
             p.rec_id[item] = make_int2(-1, -1);
         }
     }
-    if (rs == RAY_OK) forward_finish<RM>(p, q, item, o, rc, ctr, out_rgb, out_depth, out_opac);
-    if (rs == RAY_BAD) forward_bad<RM>(p, q, item, st, out_rgb, out_depth, out_opac);
+    if (rs == RAY_OK && lead) forward_finish<RM>(p, q, item, o, rc, ctr, out_rgb, out_depth, out_opac);
+    if (rs == RAY_BAD && lead) forward_bad<RM>(p, q, item, st, out_rgb, out_depth, out_opac);
+    if (!lead) ctr = Counters();
     flush_counters(ctr, st);
+}
+
+template <int SPB, bool RNG, int RM>
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(SPB == 8 ? 4 : 3)))
+k_tile_forward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int waves, int chunk, int hit_depth,
+               float* __restrict__ out_rgb, float* __restrict__ out_depth, float* __restrict__ out_opac, DevStats st) {
+    __shared__ TileLds W;
+    bool split;
+    const int64_t wave = tile_wave(p, blockIdx.x, chunk, waves, split);
+    if (wave < 0) return;
+    if constexpr (SPB == 8) {
+        if (p.rays_per_wave <= 8) {
+            forward_wave<SPB, RNG, RM, true>(sc, p, job, num_items, wave, split, hit_depth, out_rgb, out_depth, out_opac, st,
+                                             W, threadIdx.x);
+            return;
+        }
+    }
+    forward_wave<SPB, RNG, RM, false>(sc, p, job, num_items, wave, split, hit_depth, out_rgb, out_depth, out_opac, st, W,
+                                      threadIdx.x);
+}
+
+template <int SPB, bool RNG, int RM, bool SPREAD>
+__device__ __forceinline__ void backward_wave(const DevScene& sc, const DevParams& p, const RayJob& job, int64_t num_items,
+                                              int64_t wave, bool split, const float* __restrict__ ray_colors,
+                                              const float* __restrict__ dLdC, const float* __restrict__ target,
+                                              int loss_kind, int count_stats, const DevGrad& gr, DevStats st, BwdLds& S,
+                                              GradStage& G, int lane) {
+    const bool lead = !SPREAD || (lane & 7) == 0;  // of the ray's lanes
+    const int64_t item = wave_item(p, wave, SPREAD ? lane >> 3 : lane);
+    const bool in = item >= 0 && item < num_items;
+    Counters ctr;
+    float loss = 0.0f;
+    BwdRay b;
+    if (in) backward_setup<RNG, RM>(sc, p, job, wave, lane, item, ray_colors, dLdC, target, loss_kind, st, b, loss, split, lead);
+    if (target) add_loss(p, lead ? loss : 0.0f, lane, st);
+    // the rays whose tile the forward recorded, and the others if they can go as a tile too
+    const unsigned long long recorded = RM == 2 ? __ballot(b.active && b.tile >= 0) : 0ULL;
+    const bool rest = b.active && b.tile < 0;
+    int group;
+    const bool leave = p.wide && __ballot(rest) != 0ULL &&
+                       (__ballot(rest && b.rc.w) != 0ULL || !tile_groups(sc, rest, b.view, b.ray, group));
+    if (leave) tile_leave<SPREAD>(p, wave, rest, lane);
+    int num_cells = 0;
+    if (recorded != 0ULL) num_cells = __builtin_amdgcn_readlane(b.rc.end, __ffsll((long long)recorded) - 1);
+    const u32x4* cells = RM == 2 ? reinterpret_cast<const u32x4*>(rec_region(p, wave)) : nullptr;
+    backward_tile<SPB, RNG, SPREAD>(sc, p, job.cams, b.active && !(leave && rest), b.ray, b.seed, b.view, b.Cf, b.dL, cells,
+                                    num_cells, b.tile, rest || b.trunc, S, G, lane, gr, ctr, st.c + C_DROP);
+    if (!lead) ctr = Counters();
+    if (count_stats) flush_counters(ctr, st);
 }
 
 template <int SPB, bool RNG, int RM>
@@ -750,30 +934,18 @@ k_tile_backward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int wav
                 DevGrad gr, DevStats st) {
     __shared__ BwdLds S;
     __shared__ GradStage G;
-    const int lane = threadIdx.x;
     bool split;
     const int64_t wave = tile_wave(p, blockIdx.x, chunk, waves, split);
     if (wave < 0) return;
-    const int64_t item = wave_item(p, wave, lane);
-    const bool in = item >= 0 && item < num_items;
-    Counters ctr;
-    float loss = 0.0f;
-    BwdRay b;
-    if (in) backward_setup<RNG, RM>(sc, p, job, wave, lane, item, ray_colors, dLdC, target, loss_kind, st, b, loss, split);
-    if (target) add_loss(p, loss, lane, st);
-    // the rays whose tile the forward recorded, and the others if they can go as a tile too
-    const unsigned long long recorded = RM == 2 ? __ballot(b.active && b.tile >= 0) : 0ULL;
-    const bool rest = b.active && b.tile < 0;
-    int group;
-    const bool leave = p.wide && __ballot(rest) != 0ULL &&
-                       (__ballot(rest && b.rc.w) != 0ULL || !tile_groups(sc, rest, b.view, b.ray, group));
-    if (leave) tile_leave(p, wave, rest, lane);
-    int num_cells = 0;
-    if (recorded != 0ULL) num_cells = __builtin_amdgcn_readlane(b.rc.end, __ffsll((long long)recorded) - 1);
-    const u32x4* cells = RM == 2 ? reinterpret_cast<const u32x4*>(rec_region(p, wave)) : nullptr;
-    backward_tile<SPB, RNG>(sc, p, job.cams, b.active && !(leave && rest), b.ray, b.seed, b.view, b.Cf, b.dL, cells, num_cells,
-                            b.tile, rest || b.trunc, S, G, lane, gr, ctr, st.c + C_DROP);
-    if (count_stats) flush_counters(ctr, st);
+    if constexpr (SPB == 8) {
+        if (p.rays_per_wave <= 8) {
+            backward_wave<SPB, RNG, RM, true>(sc, p, job, num_items, wave, split, ray_colors, dLdC, target, loss_kind,
+                                              count_stats, gr, st, S, G, threadIdx.x);
+            return;
+        }
+    }
+    backward_wave<SPB, RNG, RM, false>(sc, p, job, num_items, wave, split, ray_colors, dLdC, target, loss_kind, count_stats,
+                                       gr, st, S, G, threadIdx.x);
 }
 
 // Launch of a tile kernel over all wavefronts of a job.
@@ -801,7 +973,8 @@ void launch_order(const DevScene& sc, const DevParams& p, const RayJob& job, boo
                        records ? nullptr : p.order_grid, p.order_bucket, hist);
     hipLaunchKernelGGL(k_tile_order, dim3((waves + kOrderBlock - 1) / kOrderBlock), dim3(kOrderBlock), 0, s, waves,
                        p.order_bucket, hist, p.order, (int)(p.wide ? waves : order_entries(waves)),
-                       p.wide ? 0 : records ? 1 : -1, slots, p.order_grid, records ? 0 : views * kGrid * kGrid);
+                       p.wide || p.rays_per_wave <= split_rays(p) ? 0 : records ? 1 : -1,
+                       p.rays_per_wave / split_rays(p), slots, p.order_grid, records ? 0 : views * kGrid * kGrid);
 }
 
 // Specialised on SPB (8 or 16 samples per slab), on whether the random generator is used and on the
@@ -828,12 +1001,15 @@ bool stepper_only(const DevParams& p) {
 
 // Small jobs spread their rays over more wavefronts: with fewer than the GPU holds (4 on each of its
 // 1024 SIMDs) the slowest wavefront is the launch, and a narrower beam has fewer candidates.  Beyond
-// that narrow wavefronts only repeat work.  Drop-in training step with 64 / 32 / 16 / 8 / 4 rays (ms):
-// 64 tiles 2.57 / 1.95 / 1.24 / 0.92 / 0.75, 475 tiles 4.17 / 2.72 / 1.67 / 1.31 / 1.20, 2555 tiles
-// 3.32 / 2.25 / 2.13 / 2.34 / 3.37, 3750 tiles 9.9 / 11.3 / 13.2 / 18.8 / 29.3.
+// that narrow wavefronts only repeat work.  Drop-in training step with 4 / 8 / 16 / 32 / 64 rays (us; - : not
+// measured): 64 tiles of 4k Gaussians 490 / 583 / - / - / -, 256 of 20k 750 / 968 / 1550 / - / -, 529 of 20k
+// 796 / 855 / 938 / - / -, 1024 of 30k in blobs 1115 / 1061 / 956 / - / -, unbounded 1934 / 1333 / 1261 / - / -,
+// 2025 - / 1178 / 1016 / 958 / - and - / 1950 / 1490 / 1327 / -, 3025 of 50k - / 1646 / 1337 / 1257 / - and - / 3154 /
+// 2196 / 1720 / -; before the spread wavefronts, 2555 tiles 3370 / 2340 / 2130 / 2250 / 3320, 3750 tiles 29.3 / 18.8 /
+// 13.2 / 11.3 / 9.9 ms.
 int rays_per_wave(int64_t num_items) {
     const int64_t tiles = (num_items + kWave - 1) / kWave;
-    return tiles <= 256 ? 4 : tiles <= 512 ? 8 : tiles <= 1024 ? 16 : tiles <= 3072 ? 32 : 64;
+    return tiles <= 576 ? 4 : tiles <= 1024 ? 16 : tiles <= 3072 ? 32 : 64;
 }
 
 int64_t order_entries(int64_t waves) { return waves + 3 * (waves / kSplitPart); }

@@ -159,3 +159,15 @@ def test_split_wavefronts(gpu_device, w, h, words):
         for k, t in a[2][v].items():
             assert max_rel(b[2][v][k], t) <= 1e-5, (v, k)
     assert a[1]["slab_hits"] == b[1]["slab_hits"] > 0 and a[1]["pairs"] == b[1]["pairs"]
+
+
+@pytest.mark.parametrize("rnd", [0, 1, 2])
+@pytest.mark.parametrize("spb", [3, 8, 11])
+def test_samples_across_lanes(gpu_device, spb, rnd):
+    """Small jobs hold a ray in eight lanes, one sample each (with more than eight per slab they take the
+    other form), with every placement of the samples."""
+    sc = scenes.scene_uniform(2000, seed=spb)
+    prm = scenes.RenderParams(dt=0.02, samples_per_slab=spb, t_eps=1e-3, jitter=rnd & 1, rnd_sample=rnd, iteration=7,
+                              white_background=True)
+    st = _compare(sc, prm, [_view(29, 19)], gpu_device, np.zeros(551), np.arange(551), 512)
+    assert st["slab_hits"] > 0
