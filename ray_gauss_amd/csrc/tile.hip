@@ -380,7 +380,7 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
                                               unsigned long long* drops) {
     const float slab = p.dt * (float)p.spb;
     TileLds& W = S.W;
-    int nst = 0;
+    Staged staged;
     bool alive = act && (ray.tenter < ray.texit) && (add_exact(ray.tenter, slab) > ray.tenter) && 1.0f > p.t_eps;
     float T = 1.0f;
     float Dr = dL[0] * Cfwd[0] + dL[1] * Cfwd[1] + dL[2] * Cfwd[2];  // dLdC . (colour not yet composited)
@@ -624,7 +624,7 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
                         grad_moments<SPB, RNG>(P, D, g0.w, md, ptc.w, project_color(dL, col), tb, cur_seed, p, sig, ep, dL, v);
                     }
                 }
-                grad_scatter_wave(v, key_base + slot, sc, gr, lane, G, nst, drops);
+                grad_scatter_wave(v, key_base + slot, sc, gr, lane, G, staged, drops);
             });
         }
         if (replay) pos += 1 + total;
@@ -642,7 +642,7 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
             }
         }
     }
-    stage_flush(G, nst, sc, gr, lane, drops);
+    stage_flush(G, staged, sc, gr, lane, drops);
 }
 
 // ------------------------------------------------------------------ order --------------------

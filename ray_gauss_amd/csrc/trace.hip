@@ -495,7 +495,7 @@ __device__ void direct_scatter_wave(const DevScene& sc, const DevParams& p, bool
                                     const float4* __restrict__ rgbv, float cur_tb, unsigned int cur_seed,
                                     float cur_tmin, float cur_tmax,
                                     const float* Gq, const float* Bq, const float* dL, GradStage& G,
-                                    int& nst, int lane, const DevGrad& gr, int view, unsigned long long* drops) {
+                                    Staged& st, int lane, const DevGrad& gr, int view, unsigned long long* drops) {
     const float ix = 1.0f / ray.dx, iy = 1.0f / ray.dy, iz = 1.0f / ray.dz;
     const int total = sc.total_nodes;
     bool live = dsc;
@@ -542,7 +542,7 @@ __device__ void direct_scatter_wave(const DevScene& sc, const DevParams& p, bool
             float w[kMoments];
 #pragma unroll
             for (int k = 0; k < kMoments; ++k) w[k] = mine ? v[k] : 0.0f;
-            grad_scatter_wave(w, vw * sc.n + leaf, sc, gr, lane, G, nst, drops);
+            grad_scatter_wave(w, vw * sc.n + leaf, sc, gr, lane, G, st, drops);
             rem &= ~__ballot(mine);
         }
         idx = miss;
@@ -559,7 +559,7 @@ __device__ void backward_wave(const DevScene& sc, const DevParams& p, bool activ
                               const float4* __restrict__ rgbv, const float* Cfwd, const float* dL, IList<CAP>& L,
                               GradStage& G, int lane, const DevGrad& gr, int view, Counters& ctr, Rec& rc,
                               unsigned long long* drops) {
-    int nst = 0;  // records in the staging area
+    Staged st;  // records in the staging area
     bool alive = active && (ray.tenter < ray.texit) && (add_exact(ray.tenter, p.dt * (float)p.spb) > ray.tenter);
     float T = 1.0f;
     float Dr = dL[0] * Cfwd[0] + dL[1] * Cfwd[1] + dL[2] * Cfwd[2];  // dLdC . (colour not yet composited)
@@ -678,7 +678,7 @@ __device__ void backward_wave(const DevScene& sc, const DevParams& p, bool activ
         // converged: slabs whose hit set overflowed the list scatter from a packet traversal
         if (__ballot(dsc) != 0ULL)
             direct_scatter_wave<SPB, RNG>(sc, p, dsc, ray, rgbv, cur_tb, cur_seed, cur_tmin, cur_tmax, sig, ep, dL, G,
-                                     nst, lane, gr, view, drops);
+                                     st, lane, gr, view, drops);
         // wave-merged scatter over the prepared slabs' list hits.  A lane's key (view * n + slot of
         // its next hit; INT_MAX when it has none) changes only when its hit is scattered, and the
         // following hit's slot is loaded ahead of that hit's arithmetic.
@@ -733,10 +733,10 @@ __device__ void backward_wave(const DevScene& sc, const DevParams& p, bool activ
                     my = cur_m != 0u ? key_base + nxt : INT_MAX;
                 }
             }
-            grad_scatter_wave(v, mn, sc, gr, lane, G, nst, drops);
+            grad_scatter_wave(v, mn, sc, gr, lane, G, st, drops);
         }
     }
-    stage_flush(G, nst, sc, gr, lane, drops);
+    stage_flush(G, st, sc, gr, lane, drops);
 }
 
 // Renders the work items below `end` of wavefront `wave`, one per lane.
