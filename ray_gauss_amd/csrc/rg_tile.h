@@ -32,6 +32,7 @@ struct Beam {
     float u[3], v[3];
     float eps;
     float rmin[3], rmax[3];  // 1 / dmin, 1 / dmax
+    int cuts;                // halvings of the leaves that a gather may make
 };
 
 // A slab's samples in wavefronts that hold one in each lane (spread), exchanged between a ray's eight lanes.
@@ -113,6 +114,11 @@ __device__ __forceinline__ void make_beam(bool act, const Ray& r, const float* a
         b.v[a] = v[a] * hv;
     }
     b.eps = wave_max64f(__builtin_sqrtf(dev)) * 1.0001f + 1e-6f;
+    // A round whose candidates take several lists evaluates all of them; one that walks the tree, those in
+    // the boxes that its rays meet, which are fewer where 64 rays are scattered over a wide beam.  Forward of
+    // random rays in blocks of 8 / 32 / 64 / 128 of 1024 pixels (widths 0.006, 0.023, 0.045, 0.09) at 1M Gaussians,
+    // several lists: 4.86 / 27.2 / 103 / 498 ms, at most two: 6.55 / 26.2 / 56 / 77.
+    b.cuts = fmaxf(hu, hv) < 0.0125f ? 0x7fffffff : 1;
     __syncthreads();
     if (lane == 0) W.beam = b;
     __syncthreads();
@@ -262,8 +268,8 @@ __device__ __forceinline__ int drop_candidates(TileLds& W, int cnt, float s1, un
 
 // Gathers the candidates of W's beam within [tlag, w.s1] (a range of w.m slabs) and the leaves
 // from w.first on into W, sorted by slot, and sets w.cnt.  When they do not fit, the range is halved, down to the round
-// [tlag, whi], and then with split the leaves to the lower half of those found (w.limit); what was found
-// stays where it still belongs.  Returns false when they do not fit all the same.  64 nodes are taken
+// [tlag, whi], and then with split, as often as the beam allows, the leaves to the lower half of those found
+// (w.limit); what was found stays where it still belongs.  Returns false when they do not fit all the same.  64 nodes are taken
 // at a time from the top of a stack, and the leaves among them are tested 64 at a time too: the test is
 // most of a gather's arithmetic (230 of 300 instructions), and few of the 64 nodes are leaves.  Testing
 // them as they came, starting again with half the range and walking the tree for each round whose
@@ -281,6 +287,7 @@ __device__ __forceinline__ bool beam_gather(const float4* __restrict__ nodes, co
     if (lane == 0) W.stack[0] = 0;
     int sp = 1, queue = 0;
     __syncthreads();
+    int cuts = split ? b.cuts : 0;
     while (sp > 0 || queue > 0) {
         // the next nodes and, once there are 64, leaves; each of the p nodes puts at most two in its
         // place, and a nearly full stack is walked in depth
@@ -339,7 +346,8 @@ __device__ __forceinline__ bool beam_gather(const float4* __restrict__ nodes, co
                 if (w.m > 1) {
                     w.m >>= 1;
                     w.s1 = range_end(w.m, tlag, whi, slab);
-                } else if (split) {
+                } else if (cuts > 0) {
+                    --cuts;
                     unsigned int key[kCandLane];
                     int rank[kCandLane];
                     rank_keys(W, w.cnt, lane, key, rank);

@@ -26,12 +26,13 @@ constexpr float kTileSync = 0.75f;  // lanes within this many slabs of the lagga
 // (per direction component, from its first ray; 8x8 pixels of a 1000-pixel, 40-degree view are 0.006)
 // kTileSpread and sqrt(kTileDensity / n); other wavefronts go to the slab stepper.  A beam's
 // candidates grow with the Gaussians and with the square of its width, its rays' own hits do not.
-// Measured on 64 random rays of a block of S pixels out of 1024 (stepper / tile, train step): 1M
-// Gaussians S = 32 103 / 54 ms, 64 175 / 152, 128 (spread 0.09) 274 / 377; 300k Gaussians S = 128
-// 109 / 88, 256 125 / 97; 20k 256 10.1 / 8.9.  Several beams: a list of 8x8 tiles with ragged edges
-// has wavefronts that hold the end of one row of tiles and the start of the next (one beam each; in
+// Measured on 64 random rays of a block of S pixels out of 1024 (train step, every wavefront's rays in the
+// stepper / as tiles with bounds 0.2 and 3000): 1M Gaussians S = 32 102 / 45 ms, 64 177 / 151, 128 (spread 0.09)
+// 283 / 242, 256 (up to four beams) 323 / 380; 300k S = 128 115 / 43, 256 130 / 51; 20k 256 10.4 / 7.6, 1024
+// 7.0 / 19.6; with the bounds below 45, 151, 246, 361; 43, 82; 10.9, 4.1.  Several beams: a list of 8x8 tiles
+// with ragged edges has wavefronts that hold the end of one row of tiles and the start of the next (one beam each; in
 // the stepper the 1 % of such wavefronts took 10 of 290 ms at 1M Gaussians).
-constexpr float kTileSpread = 0.2f, kTileDensity = 3000.0f;
+constexpr float kTileSpread = 0.1f, kTileDensity = 2000.0f;
 constexpr int kTileGroups = 4;
 
 // Assigns the lanes with act to beams (group 0 .. kTileGroups - 1); false when they make up more.
