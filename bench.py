@@ -55,11 +55,11 @@ def backward_bytes(R, P):
     return 24.0 * R + 112.0 * P
 
 
-def measured_traffic(workload, kernel="k_backward"):
+def measured_traffic(workload, kernel="k_tile_backward"):
     """HBM-side bytes per launch of `kernel` from the rocprofv3 summary committed for this workload
     (FETCH_SIZE + WRITE_SIZE, each scaled by its reading for a device copy of known size); None
     when no summary exists.  The summary names the commands it was made with."""
-    path = os.path.join(ROOT, "profiles", f"k_backward_{workload}.md")
+    path = os.path.join(ROOT, "profiles", f"{kernel}_{workload}.md")
     try:
         with open(path) as f:
             for line in f:
@@ -433,10 +433,10 @@ def main():
         "counters": {"K_slab_hits": K, "P_pairs": P, "fallback_slabs": st["fallback_slabs"],
                      "gathers": st["gathers"], "replay_words": st["replay_words"],
                      "replay_truncated_rays": st["replay_truncated"]},
-        "roofline": {"bound": "hbm", "kernel": "k_backward", "kernel_ms": bk_ms, "achieved": achieved,
+        "roofline": {"bound": "hbm", "kernel": "k_tile_backward", "kernel_ms": bk_ms, "achieved": achieved,
                      "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBPS, "traffic": traffic,
                      "traffic_source": traffic_src, "algorithmic_bytes": B_bwd},
-        "forward_kernel": {"kernel": "k_forward", "kernel_ms": fk_ms,
+        "forward_kernel": {"kernel": "k_tile_forward", "kernel_ms": fk_ms,
                            "achieved_GBps": forward_bytes(R, P) / (fk_ms * 1e-3) / 1e9},
         "step_hbm_GBps": B_step / dt_b / 1e9,
         "step_bytes": {"total": B_step, "records": B_rec},

@@ -47,8 +47,11 @@ typedef struct rg_config {
     int32_t hit_depth;         /* per-ray interval list capacity: 8, 16 or 32                    */
     int32_t seg_slabs;         /* initial slabs per interval gather: 1..4096                     */
     int32_t max_hits_per_slab; /* >0: count slabs whose hit set exceeds it (max_prim_slice)      */
-    int32_t packet_traversal;  /* 1: the lanes of a wavefront walk the LBVH together (one node
-                                  sequence, per-lane box tests); 0: per-lane walks                */
+    int32_t packet_traversal;  /* 1: wavefronts of narrow beams march as one (tiles), in others the
+                                  lanes walk the LBVH together (one node sequence, per-lane box
+                                  tests); 0: per-lane walks.  hit_depth, fwd_hit_depth, ray_chunk,
+                                  refill_lanes, bwd_ray_chunk and bwd_window are settings of the
+                                  wavefronts that are not tiles                                   */
     int32_t jitter;            /* RenderOptixSettings.jitter: sub-pixel jitter (gaussians_aabb.cu:409) */
     int32_t rnd_sample;        /* RenderOptixSettings.rnd_sample: 0 grid, 1 random, 2 mid-sample     */
     uint32_t iteration;        /* RenderOptixSettings.iteration: seeds tea<4>(iteration, pixel)       */
@@ -140,8 +143,8 @@ typedef struct rg_stats {
     int64_t slab_hits;        /* K: sum over processed slabs of |hit set|                     */
     int64_t pairs;            /* P: distinct (ray, Gaussian) pairs                            */
     int64_t overflow_slabs;   /* slabs with more hits than max_hits_per_slab (optix_utils:205) */
-    int64_t fallback_slabs;   /* slabs whose hit set exceeded hit_depth (per-slab traversal)   */
-    int64_t gathers;          /* interval-list gathers (BVH traversals)                       */
+    int64_t fallback_slabs;   /* slabs whose hit set exceeded hit_depth                        */
+    int64_t gathers;          /* gathers, counted for each ray they were made for             */
     int64_t replay_words;     /* words of hit-list records written by the forward (rg_train_batch) */
     int64_t replay_truncated; /* rays whose records did not fit replay_words                    */
     int64_t dropped;          /* gradient records or replayed hits skipped by a bounds check:

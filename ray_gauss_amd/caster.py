@@ -20,11 +20,15 @@ from .cameras import launch_record_from
 
 @dataclass
 class TuneConfig:
-    """Launch tuning: interval-list depth per ray, initial slabs per gather, whether a wavefront's
+    """Launch tuning.  Wavefronts whose rays form narrow beams (tiles of a view) march as one and use
+    seg_slabs (their first gathered range), replay_words, tree_builder and fwd_jump; the other fields are
+    settings of the per-ray slab stepper, which takes all other rays (all of them with packet off, or with
+    ray_chunk and refill_lanes set), and the figures below are its.  Interval-list depth per ray, initial slabs per gather, whether a wavefront's
     lanes walk the LBVH as one packet, the forward kernel's own (smaller) list depth, and the
     words per ray in which a forward records its hit lists for the backward over the same rays
-    (0: the backward walks the tree again; 1536 words = 6 KB of device memory per ray), and the
-    tree built at a rebuild: 0, the LBVH in Morton order (about 9 ms at 1M Gaussians with the
+    (0: the backward walks the tree again; 1536 words = 6 KB of device memory per ray, of which a tile
+    uses its share for its rays' common events), and the
+    tree built at a rebuild: 0, the LBVH in Morton order (about 1 ms at 1M Gaussians with the
     preprocessing, cheap enough to rebuild on every call as the reference does); 1, a binned-SAH
     tree (about 70 ms, 11 % faster forward at 1M Gaussians), for loops that build once and then
     refit every step.  ray_chunk: 0 launches the forward as one wavefront per 8x8 tile; a multiple
