@@ -252,6 +252,7 @@ rg::DevParams dev_params(const rg_handle* h) {
     p.queue = h->queue;
     p.bwd_window = h->cfg.bwd_window > 0.0f ? h->cfg.bwd_window : 0.5f;
     p.fwd_jump = h->cfg.fwd_round_per_slab ? 0 : 1;
+    p.tiles = 0;
     p.rays_per_wave = 64;
     p.wide = nullptr;
     p.wide_count = nullptr;
@@ -438,11 +439,12 @@ int rg_set_view_colors(rg_handle* h, int32_t view, const float* rgb, void* strea
     return RG_OK;
 }
 
-// Wavefronts of the job: how many rays each holds, the order they are taken in, and room for those
-// that the tile kernels leave to the slab stepper.  A whole view whose 8x8 blocks are all narrow
-// beams leaves none.
+// Wavefronts of the job (p: dev_params, of a forward or a backward): whether they go through the tile
+// kernels, how many rays each holds, the order they are taken in, and room for those that the tile
+// kernels leave to the slab stepper.  A whole view whose 8x8 blocks are all narrow beams leaves none.
 static int plan_waves(rg_handle* h, const rg::RayJob& j, rg::DevParams& p, hipStream_t s) {
-    if (rg::stepper_only(p)) return RG_OK;
+    p.tiles = rg::takes_tiles(p) ? 1 : 0;
+    if (!p.tiles) return RG_OK;
     p.rays_per_wave = rg::rays_per_wave(j.num_rays);
     const int64_t waves = (j.num_rays + 63) / 64 * (64 / p.rays_per_wave);
     const int views = j.ray_view ? j.num_views : 1;
@@ -518,7 +520,7 @@ static void rec_backward(const rg_handle* h, const rg::RayJob& j, uint64_t token
     p.rec_id = h->rec_id;
     p.rec_words = r.words;
     p.rec_mode = 2;
-    p.rays_per_wave = r.rays_per_wave;  // the records' layout (never fewer wavefronts than planned)
+    p.rays_per_wave = r.rays_per_wave;  // the records' layout (of as many rays or more: never more wavefronts than planned)
 }
 
 int rg_forward(rg_handle* h, int32_t view, int64_t num_rays, const int32_t* pixels, float* out_rgb, float* out_depth,

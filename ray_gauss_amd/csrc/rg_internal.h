@@ -72,7 +72,10 @@ struct DevParams {
     float bwd_window;
     // forward: step over slabs empty for every lane of a wavefront together (jump_empty)
     int fwd_jump;
-    // rays a wavefront holds (64, 32, 16, 8 or 4; fewer than 64 only in grid launches)
+    // the job goes through the tile kernels (narrow beams) first: decided once, with the handle's own
+    // settings, for the forward and the backward of a job, whose records are of one form
+    int tiles;
+    // rays a wavefront holds (64, 32, 16, 8 or 4; fewer than 64 only with tiles)
     int rays_per_wave;
     // wavefronts whose rays do not make up narrow beams, left by the tile kernel to the slab stepper:
     // (wavefront, lanes: low, high word, 0), and their number (nullptr: none)
@@ -240,8 +243,9 @@ hipError_t launch_debug_hits(const DevScene& sc, const DevParams& p, const RayJo
                              hipStream_t s);
 
 // ---- launchers (tile.hip) ---------------------------------------------------------------------
-// Whether these settings leave every ray to the slab stepper (in wavefronts of 64).
-bool stepper_only(const DevParams& p);
+// Whether jobs with the handle's settings go through the tile kernels; if not, every ray goes to the slab
+// stepper (in wavefronts of 64).  ray_chunk is the forward's, in a backward too.
+bool takes_tiles(const DevParams& p);
 // Rays per wavefront for a job of num_items work items.
 int rays_per_wave(int64_t num_items);
 // Jobs of fewer wavefronts than this keep their own order (all of them start at once).

@@ -996,8 +996,8 @@ void launch_order(const DevScene& sc, const DevParams& p, const RayJob& job, boo
 
 // The stepper takes all rays where its own options are asked for (per-lane walks, refilled lanes) and
 // below depth zero, where a beam's bounds do not hold.
-bool stepper_only(const DevParams& p) {
-    return !p.packet || !(p.t_near >= 0.0f) || (p.ray_chunk > 0 && p.refill_lanes > 0);
+bool takes_tiles(const DevParams& p) {
+    return p.packet && p.t_near >= 0.0f && !(p.ray_chunk > 0 && p.refill_lanes > 0);
 }
 
 // Small jobs spread their rays over more wavefronts: with fewer than the GPU holds (4 on each of its
@@ -1034,12 +1034,10 @@ hipError_t launch_forward(const DevScene& sc, const DevParams& p0, const RayJob&
     if (job.num_rays <= 0) return hipSuccess;
     DevParams p = p0;
     p.wide_count = st.c + 12;
-    if (!stepper_only(p)) {
+    if (p.tiles) {
         if (p.order) launch_order(sc, p, job, false, 4096, st.c + 16, s);
         RG_TILE_DISPATCH(p.rec_mode == 1, 1, k_tile_forward, sc, p, job, s, hit_depth, out_rgb, out_depth, out_opacity, st);
         if (!p.wide) return hipGetLastError();
-    } else {
-        p.wide = nullptr;
     }
     return launch_forward_steps(sc, p, job, hit_depth, out_rgb, out_depth, out_opacity, st, s);
 }
@@ -1050,13 +1048,11 @@ hipError_t launch_backward(const DevScene& sc, const DevParams& p0, const RayJob
     if (job.num_rays <= 0) return hipSuccess;
     DevParams p = p0;
     p.wide_count = st.c + 13;
-    if (!stepper_only(p)) {
+    if (p.tiles) {
         if (p.order) launch_order(sc, p, job, p.rec_mode == 2, 3072, st.c + 48, s);
         RG_TILE_DISPATCH(p.rec_mode == 2, 2, k_tile_backward, sc, p, job, s, ray_colors, dLdC, target, loss_kind, count_stats,
                          gr, st);
         if (!p.wide) return hipGetLastError();
-    } else {
-        p.wide = nullptr;
     }
     return launch_backward_steps(sc, p, job, hit_depth, ray_colors, dLdC, target, loss_kind, count_stats, gr, st, s);
 }

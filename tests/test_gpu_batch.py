@@ -362,3 +362,37 @@ def test_persistent_full_view_and_pixel_lists(gpu_device):
                                 TuneConfig(ray_chunk=ch, refill_lanes=16 if ch else 0, bwd_ray_chunk=ch))
         out[ch] = (rc.forward(0)[0], rc.forward(0, px)[0])
     assert torch.equal(out[0][0], out[128][0]) and torch.equal(out[0][1], out[128][1])
+
+
+@pytest.mark.parametrize("w,h", [(64, 64), (320, 200), (512, 500)])
+def test_forward_and_backward_agree_on_tiles(gpu_device, w, h):
+    """Every mix of the forward's and the backward's chunks with refilled lanes, at jobs of 64, 1000 and
+    4032 tiles (4, 16 and 64 rays in a wavefront of the tile kernels): both passes process every ray
+    and the backward replays what the forward recorded, without a gather of its own."""
+    sc = scenes.scene_uniform(3000, seed=w)
+    prm = scenes.RenderParams(dt=0.02, t_eps=1e-4, white_background=True)
+    cam = look_at_camera(orbit_eye(3.0, 30.0, 20.0), width=w, height=h, fovx_deg=40.0).launch_record()
+    rv, rp, _ = make_ray_batch([cam], None, gpu_device)
+    gen = torch.Generator(device=gpu_device).manual_seed(3)
+    target = torch.rand((rv.shape[0], 3), generator=gen, device=gpu_device)
+    ref = None
+    for chunk in (0, 64):
+        for refill in (0, 16):
+            for bchunk in (0, 64):
+                rc, _ = prepared_caster(sc, prm, [cam], gpu_device,
+                                        TuneConfig(ray_chunk=chunk, refill_lanes=refill, bwd_ray_chunk=bchunk))
+                rgb, _, _ = rc.forward_batch(rv, rp)
+                rc.backward_batch(rv, rp, rgb, 2.0 * (rgb - target), rc.last_token)
+                st = rc.stats()
+                assert st["dropped"] == 0 and st["gathers"] == 0, (chunk, refill, bchunk, st)
+                g = {k: v.cpu().numpy() for k, v in rc.finish_grads().items() if v is not None}
+                loss = torch.zeros(1, device=gpu_device)
+                rc.train_batch(rv, rp, target, 0, None, loss)
+                gt = {k: v.cpu().numpy() for k, v in rc.finish_grads().items() if v is not None}
+                if ref is None:
+                    ref = (rgb, g, float(loss))
+                    assert abs(ref[2] - float(((rgb - target) ** 2).double().sum())) <= 1e-5 * ref[2]
+                assert torch.equal(rgb, ref[0])
+                assert abs(float(loss) - ref[2]) <= 1e-5 * ref[2], (chunk, refill, bchunk)
+                for k, v in ref[1].items():
+                    assert max_rel(g[k], v) <= 1e-5 and max_rel(gt[k], v) <= 1e-5, (chunk, refill, bchunk, k)
