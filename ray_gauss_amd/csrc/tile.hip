@@ -69,12 +69,16 @@ __device__ __forceinline__ void tile_list(TileWalk& w, const DevScene& sc, float
     if (alive) ctr.gathers++;
 }
 
+// Whether a lane at depth tb takes part in the round whose laggard is at tlag <= tb; the laggard always does
+// (at depths where a slab is less than an ulp of t, tlag + kTileSync * slab may round to tlag).
+__device__ __forceinline__ bool in_round(float tb, float tlag, float slab) { return tb - tlag < kTileSync * slab; }
+
 // The lanes of the next round: its depths [tlag, whi] and whether this lane takes part.
 __device__ __forceinline__ bool tile_window(bool alive, float tb, float slab, float& tlag, float& whi) {
     // depths are not negative: their order is that of their bits
     const int bits = __float_as_int(tb);
     tlag = __int_as_float(__builtin_amdgcn_readfirstlane(wave_min64(alive ? bits : 0x7f800000)));
-    const bool part = alive && tb < tlag + kTileSync * slab;
+    const bool part = alive && in_round(tb, tlag, slab);
     whi = add_exact(__int_as_float(__builtin_amdgcn_readfirstlane(~wave_min64(part ? ~bits : INT_MAX))), slab);
     return part;
 }
@@ -429,7 +433,7 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
                 if (!(nt > tb) || !(nt < ray.texit)) alive = false;
                 else tb = nt;
             }
-            part = alive && mine && tb < tlag + kTileSync * slab;
+            part = alive && mine && in_round(tb, tlag, slab);
         } else {
             if ((__ballot(alive && walk) & todo) == 0ULL) {  // the next beam
                 if (group < 0) {
