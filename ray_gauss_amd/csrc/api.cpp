@@ -256,6 +256,8 @@ rg::DevParams dev_params(const rg_handle* h) {
     p.rays_per_wave = 64;
     p.wide = nullptr;
     p.wide_count = nullptr;
+    p.sample_wide = nullptr;
+    p.sample_limit = 0;
     p.order = nullptr;
     p.order_bucket = nullptr;
     p.order_grid = nullptr;

@@ -78,9 +78,12 @@ struct DevParams {
     // rays a wavefront holds (64, 32, 16, 8 or 4; fewer than 64 only with tiles)
     int rays_per_wave;
     // wavefronts whose rays do not make up narrow beams, left by the tile kernel to the slab stepper:
-    // (wavefront, lanes: low, high word, 0), and their number (nullptr: none)
+    // (wavefront, lanes: low, high word, 0), their number and that of the parts of them taken (nullptr: none)
     int4* wide;
     unsigned long long* wide_count;
+    // number of such wavefronts among those looked at, and the number past which the widths allowed are halved
+    const unsigned long long* sample_wide;
+    int sample_limit;
     // order in which the tile kernels' blocks take the wavefronts (nullptr: their own), with the weight
     // bucket of each and the grid of counts they come from (zero between jobs)
     int* order;
@@ -97,10 +100,10 @@ struct DevGrad {
 
 // Counters (device, kCounters): 0 K, 1 P, 2 overflow slabs, 3 fallback slabs, 4 gathers, 6 loss (float),
 // 7 debug scratch, 8 record words, 9 truncated records, 10 dropped by bounds checks, 11 rays with
-// an out-of-range view or pixel, 12 / 13 wavefronts left to the stepper by the forward / backward,
-// 14 loss of narrow wavefronts (double), 15 unused, 16..47 / 48..79 sizes and cursors of the order's
-// buckets in the forward / backward
-constexpr int kCounters = 80;
+// an out-of-range view or pixel, 12 / 13 unused, 14 loss of narrow wavefronts (double), 15 unused, 16..47 /
+// 48..79 sizes and cursors of the order's buckets in the forward / backward, 80, 81 / 82, 83 wavefronts left to
+// the stepper by the forward / backward and the parts of them it took, 84 / 85 wide ones of those looked at
+constexpr int kCounters = 86;
 struct DevStats {
     unsigned long long* c;
 };

@@ -33,7 +33,7 @@ struct Beam {
     float u[3], v[3];
     float eps;
     float rmin[3], rmax[3];  // 1 / dmin, 1 / dmax
-    int cuts;                // halvings of the leaves that a gather may make
+    int cuts;                // halvings of the leaves that a round's gathers may make
 };
 
 // A slab's samples in wavefronts that hold one in each lane (spread), exchanged between a ray's eight lanes.
@@ -215,6 +215,8 @@ struct TileWalk {
     int m = 1;             // its length in slabs
     int cnt = 0;           // candidates in the list
     int first = 0, limit = 0;  // nodes whose leaves it covers
+    int cuts = 0;            // halvings of the leaves that the round may still make
+    int skip = 0, back = 0;  // rounds to walk before the next gather, and after the last one that failed
     bool valid = false;
     bool direct = false;   // the round's candidates do not fit: it walks the tree itself
 };
@@ -288,7 +290,7 @@ __device__ __forceinline__ bool beam_gather(const float4* __restrict__ nodes, co
     if (lane == 0) W.stack[0] = 0;
     int sp = 1, queue = 0;
     __syncthreads();
-    int cuts = split ? b.cuts : 0;
+    if (w.first == 0) w.cuts = split ? b.cuts : 0;
     while (sp > 0 || queue > 0) {
         // the next nodes and, once there are 64, leaves; each of the p nodes puts at most two in its
         // place, and a nearly full stack is walked in depth
@@ -347,8 +349,8 @@ __device__ __forceinline__ bool beam_gather(const float4* __restrict__ nodes, co
                 if (w.m > 1) {
                     w.m >>= 1;
                     w.s1 = range_end(w.m, tlag, whi, slab);
-                } else if (cuts > 0) {
-                    --cuts;
+                } else if (w.cuts > 0) {
+                    --w.cuts;
                     unsigned int key[kCandLane];
                     int rank[kCandLane];
                     rank_keys(W, w.cnt, lane, key, rank);

@@ -34,19 +34,36 @@ constexpr float kTileSync = 0.75f;  // lanes within this many slabs of the lagga
 // the stepper the 1 % of such wavefronts took 10 of 290 ms at 1M Gaussians).
 constexpr float kTileSpread = 0.1f, kTileDensity = 2000.0f;
 constexpr int kTileGroups = 4;
+// Where more than one in kHalfShare of a job's wavefronts (of kSampled looked at) are no beams, only those of
+// half these widths march as tiles: the others are beams by chance, each as dear as the widest allowed, and
+// the launch lasts as long as they do before the stepper begins.  Rays as above, up to four beams a wavefront,
+// train step of 4096 wavefronts (all in the stepper / all beams as tiles / this rule): 300k S = 256 154 / 205 /
+// 125 ms, 100k 256 62.9 / 39.0 / 38.4, 100k 512 45.1 / 69.4 / 44.2, 20k larger Gaussians 256 32.9 / 35.9 / 35.5,
+// 512 43.7 / 76.0 / 41.5; of 1024 wavefronts 1M 256 321 / 350 / 135.
+constexpr int kSampled = 1024, kHalfShare = 8;
+// Rounds that are walked after gathers that failed, before the next gather, at most (1, 3, 7, ...): in a dense
+// stretch the next round's candidates do not fit either.  300k S = 128, 4096 wavefronts 92.7 -> 86.5 ms, 100k S = 256
+// 45.9 -> 39.0.
+constexpr int kMaxSkip = 15;
+
+// Whether the job's wavefronts are held to beams of half the widths (k_tile_sample).
+__device__ __forceinline__ bool half_beams(const DevParams& p) {
+    return p.sample_wide && *p.sample_wide > (unsigned long long)p.sample_limit;
+}
 
 // Assigns the lanes with act to beams (group 0 .. kTileGroups - 1); false when they make up more.
-__device__ __forceinline__ bool tile_groups(const DevScene& sc, bool act, int view, const Ray& r, int& group) {
-    const float limit = fminf(kTileSpread, __builtin_sqrtf(kTileDensity / (float)sc.n));
+__device__ __forceinline__ bool tile_groups(const DevScene& sc, bool half, bool act, int view, const Ray& r, int& group) {
+    float limit = fminf(kTileSpread, __builtin_sqrtf(kTileDensity / (float)sc.n));
+    if (half) limit *= 0.5f;
     group = -1;
     unsigned long long rem = __ballot(act);
     for (int k = 0; k < kTileGroups && rem != 0ULL; ++k) {
         const int f = __ffsll((long long)rem) - 1;
-        const float x = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(r.dx), f));
-        const float y = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(r.dy), f));
-        const float z = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(r.dz), f));
-        const bool near = fabsf(r.dx - x) <= limit && fabsf(r.dy - y) <= limit && fabsf(r.dz - z) <= limit;
-        const bool mine = ((rem >> threadIdx.x) & 1ULL) != 0ULL && view == __builtin_amdgcn_readlane(view, f) && near;
+        const float x = fabsf(r.dx - __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(r.dx), f)));
+        const float y = fabsf(r.dy - __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(r.dy), f)));
+        const float z = fabsf(r.dz - __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(r.dz), f)));
+        const bool in = ((rem >> threadIdx.x) & 1ULL) != 0ULL && view == __builtin_amdgcn_readlane(view, f);
+        const bool mine = in && x <= limit && y <= limit && z <= limit;
         if (mine) group = k;
         const unsigned long long m = __ballot(mine);
         if (m == 0ULL) return false;  // a NaN direction
@@ -63,9 +80,17 @@ __device__ __forceinline__ void tile_list(TileWalk& w, const DevScene& sc, float
     if (w.valid && 4 * w.cnt < kTileCand) w.m = min(w.m * 2, kMaxSeg);
     else if (w.valid && 4 * w.cnt > 3 * kTileCand) w.m = max(w.m >> 1, 1);
     w.valid = true;
+    if (w.skip > 0) {
+        --w.skip;
+        w.direct = true;
+        w.cnt = 0;
+        return;
+    }
     w.s1 = range_end(w.m, tlag, whi, slab);
     w.direct = !beam_gather(sc.nodes, sc.geo, sc.total_nodes, w, tlag, whi, slab, split, W, lane);
     if (w.direct) w.cnt = 0;
+    w.back = w.direct ? min(2 * w.back + 1, kMaxSkip) : 0;
+    w.skip = w.back;
     if (alive) ctr.gathers++;
 }
 
@@ -438,7 +463,7 @@ __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParam
             if ((__ballot(alive && walk) & todo) == 0ULL) {  // the next beam
                 if (group < 0) {
                     int g = 0;
-                    if (!tile_groups(sc, alive && walk, view, ray, g)) g = view;  // (left to this kernel: one view)
+                    if (!tile_groups(sc, half_beams(p), alive && walk, view, ray, g)) g = view;  // (left to this kernel: one view)
                     group = alive && walk ? g : INT_MAX;
                 }
                 const unsigned long long rem = __ballot(alive && walk);
@@ -845,7 +870,7 @@ __device__ __forceinline__ void forward_wave(const DevScene& sc, const DevParams
         alive = forward_begin(p, ray, o);
     }
     int group = 0;  // one view, all of it narrow
-    if (p.wide && !tile_groups(sc, alive, q.view, ray, group)) {
+    if (p.wide && !tile_groups(sc, half_beams(p), alive, q.view, ray, group)) {
         tile_leave<SPREAD>(p, wave, in, lane);
         return;
     }
@@ -921,7 +946,7 @@ __device__ __forceinline__ void backward_wave(const DevScene& sc, const DevParam
     const bool rest = b.active && b.tile < 0;
     int group;
     const bool leave = p.wide && __ballot(rest) != 0ULL &&
-                       (__ballot(rest && b.rc.w) != 0ULL || !tile_groups(sc, rest, b.view, b.ray, group));
+                       (__ballot(rest && b.rc.w) != 0ULL || !tile_groups(sc, half_beams(p), rest, b.view, b.ray, group));
     if (leave) tile_leave<SPREAD>(p, wave, rest, lane);
     int num_cells = 0;
     if (recorded != 0ULL) num_cells = __builtin_amdgcn_readlane(b.rc.end, __ffsll((long long)recorded) - 1);
@@ -951,6 +976,38 @@ k_tile_backward(DevScene sc, DevParams p, RayJob job, int64_t num_items, int wav
     }
     backward_wave<SPB, RNG, RM, false>(sc, p, job, num_items, wave, split, ray_colors, dLdC, target, loss_kind, count_stats,
                                        gr, st, S, G, threadIdx.x);
+}
+
+// Counts the wavefronts that are no beams, every stride-th of the job looked at.
+__global__ void __launch_bounds__(kWave) k_tile_sample(DevScene sc, DevParams p, RayJob job, int64_t num_items, int stride,
+                                                       unsigned long long* count) {
+    const int lane = threadIdx.x;
+    const int64_t item = wave_item(p, (int64_t)blockIdx.x * stride, lane);
+    RayRef q;
+    q.view = -1;
+    Ray ray = {};
+    bool alive = false;
+    if (item >= 0 && item < num_items && resolve(job, item, q) == RAY_OK) {
+        const rg_camera cam = job.cams[q.view];
+        unsigned int seed = p.jitter ? tea4(p.iteration, (unsigned int)q.pixel) : 0u;
+        ray = make_ray(cam, q.pixel, sc.box, p.t_near, p.t_far, p.jitter, &seed);
+        RayOut o;
+        alive = forward_begin(p, ray, o);
+    }
+    int group;
+    if (!tile_groups(sc, false, alive, q.view, ray, group) && lane == 0) atomicAdd(count, 1ull);
+}
+
+// Counts for half_beams.  Not in the smallest jobs (4 rays a wavefront), where each wavefront's march is short
+// either way and the launch would show, nor before a replay, which takes the forward's beams.
+void launch_sample(const DevScene& sc, DevParams& p, const RayJob& job, unsigned long long* count, hipStream_t s) {
+    if (!p.wide || p.rays_per_wave <= 4 || p.rec_mode == 2) return;
+    const int64_t waves = num_waves(p, job.num_rays);
+    const int64_t stride = (waves + kSampled - 1) / kSampled;
+    const int64_t samples = (waves + stride - 1) / stride;
+    hipLaunchKernelGGL(k_tile_sample, dim3((unsigned)samples), dim3(kWave), 0, s, sc, p, job, job.num_rays, (int)stride, count);
+    p.sample_wide = count;
+    p.sample_limit = (int)(samples / kHalfShare);
 }
 
 // Launch of a tile kernel over all wavefronts of a job.
@@ -1037,8 +1094,9 @@ hipError_t launch_forward(const DevScene& sc, const DevParams& p0, const RayJob&
                           float* out_depth, float* out_opacity, DevStats st, hipStream_t s) {
     if (job.num_rays <= 0) return hipSuccess;
     DevParams p = p0;
-    p.wide_count = st.c + 12;
+    p.wide_count = st.c + 80;
     if (p.tiles) {
+        launch_sample(sc, p, job, st.c + 84, s);
         if (p.order) launch_order(sc, p, job, false, 4096, st.c + 16, s);
         RG_TILE_DISPATCH(p.rec_mode == 1, 1, k_tile_forward, sc, p, job, s, hit_depth, out_rgb, out_depth, out_opacity, st);
         if (!p.wide) return hipGetLastError();
@@ -1051,8 +1109,9 @@ hipError_t launch_backward(const DevScene& sc, const DevParams& p0, const RayJob
                            int count_stats, DevGrad gr, DevStats st, hipStream_t s) {
     if (job.num_rays <= 0) return hipSuccess;
     DevParams p = p0;
-    p.wide_count = st.c + 13;
+    p.wide_count = st.c + 82;
     if (p.tiles) {
+        launch_sample(sc, p, job, st.c + 85, s);
         if (p.order) launch_order(sc, p, job, p.rec_mode == 2, 3072, st.c + 48, s);
         RG_TILE_DISPATCH(p.rec_mode == 2, 2, k_tile_backward, sc, p, job, s, ray_colors, dLdC, target, loss_kind, count_stats,
                          gr, st);

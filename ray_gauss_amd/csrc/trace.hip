@@ -739,14 +739,36 @@ __device__ void backward_wave(const DevScene& sc, const DevParams& p, bool activ
     stage_flush(G, st, sc, gr, lane, drops);
 }
 
-// Renders the work items below `end` of wavefront `wave`, one per lane.
+// Parts, of at least 4 rays, that each of the nw wavefronts left by the tile kernels is cut into: as many as
+// the GPU holds at once, since with fewer the slowest wavefront is the launch.  64 random rays of a block of
+// 128 of 1024 pixels, 4096 wavefronts of which every fifth or so is left, 300k Gaussians: train step 158 -> 104 ms.
+// More parts than that only repeat work: 64 rays of 512-pixel blocks at 20k 41.9 -> 54.6 ms with four times as many.
+__device__ __forceinline__ int wide_parts(const DevParams& p, int64_t nw) {
+    int parts = 1;
+    while (8 * parts <= p.rays_per_wave && 2 * parts * nw <= kWideBlocks) parts *= 2;
+    return parts;
+}
+
+// The wavefront whose part a block takes next, as its place in p.wide (-1: none is left), and this lane's
+// place among its rays (rays_per_wave: none).
+__device__ __forceinline__ int64_t next_wide(const DevParams& p, int64_t nw, int parts, int lane, int& ray) {
+    int i = 0;
+    if (lane == 0) i = (int)atomicAdd(p.wide_count + 1, 1ull);
+    i = __builtin_amdgcn_readfirstlane(i);
+    if (i >= nw * parts) return -1;
+    const int rays = p.rays_per_wave / parts;
+    ray = lane < rays ? (i % parts) * rays + lane : p.rays_per_wave;
+    return i / parts;
+}
+
+// Renders the work items below `end` of wavefront `wave`, one per lane (lane_ray: its place in the wavefront).
 template <int SPB, int CAP, bool RNG, int RM>
 __device__ __forceinline__ void forward_items(const DevScene& sc, const DevParams& p, const RayJob& job, int64_t wave,
-                                              int64_t end, IList<CAP>& L, int lane, float* __restrict__ out_rgb,
+                                              int64_t end, IList<CAP>& L, int lane, int lane_ray, float* __restrict__ out_rgb,
                                               float* __restrict__ out_depth, float* __restrict__ out_opac, DevStats st) {
     Counters ctr;
     RayRef q;
-    const int64_t item = wave_item(p, wave, lane);
+    const int64_t item = lane_ray < p.rays_per_wave ? wave_item(p, wave, lane_ray) : -1;
     const bool in = item >= 0 && item < end;
     const int rs = in ? resolve(job, item, q) : (int)RAY_NONE;
     if (rs == RAY_BAD) {
@@ -758,7 +780,7 @@ __device__ __forceinline__ void forward_items(const DevScene& sc, const DevParam
         RayOut o;
         Rec rc;
         if constexpr (RM == 1) {
-            rc.w = rec_region(p, wave) + 8 * lane;
+            rc.w = rec_region(p, wave) + 8 * lane_ray;
             rc.stride = 8 * p.rays_per_wave;
             rc.end = p.rec_words;
         }
@@ -778,26 +800,35 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(SPB 
                                                    float* __restrict__ out_opac, DevStats st) {
     __shared__ IList<CAP> L;
     const int lane = threadIdx.x;
-    const int64_t nb = p.wide ? (int64_t)*p.wide_count : 1;
-    for (int64_t i = p.wide ? blockIdx.x : 0; i < nb; i += gridDim.x)
-        forward_items<SPB, CAP, RNG, RM>(sc, p, job, p.wide ? p.wide[i].x : block_item(blockIdx.x, gridDim.x), num_items, L,
-                                         lane, out_rgb, out_depth, out_opac, st);
+    const int64_t nw = p.wide ? (int64_t)*p.wide_count : 1;
+    const int parts = p.wide ? wide_parts(p, nw) : 1;
+    while (nw > 0) {
+        int64_t wave = block_item(blockIdx.x, gridDim.x);
+        int ray = lane;
+        if (p.wide) {
+            const int64_t i = next_wide(p, nw, parts, lane, ray);
+            if (i < 0) return;
+            wave = p.wide[i].x;
+        }
+        forward_items<SPB, CAP, RNG, RM>(sc, p, job, wave, num_items, L, lane, ray, out_rgb, out_depth, out_opac, st);
+        if (!p.wide) return;
+    }
 }
 
-// Backward of the work items below `end` of wavefront `wave`, one per lane; lanes: those that take part
+// Backward of the work items below `end` of wavefront `wave`, one per lane (lane_ray); lanes: those that take part
 // (the rest were done by the tile kernel, with the loss and the bad rays of all of them).
 template <int SPB, int CAP, bool RNG, int RM>
 __device__ __forceinline__ void backward_items(const DevScene& sc, const DevParams& p, const RayJob& job, int64_t wave,
                                                int64_t end, unsigned long long lanes, IList<CAP>& L, GradStage& G, int lane,
-                                               const float* __restrict__ ray_colors, const float* __restrict__ dLdC,
+                                               int lane_ray, const float* __restrict__ ray_colors, const float* __restrict__ dLdC,
                                                const float* __restrict__ target, int loss_kind, int count_stats,
                                                const DevGrad& gr, DevStats st) {
     Counters ctr;
     float loss = 0.0f;
     BwdRay b;
-    const int64_t item = wave_item(p, wave, lane);
-    if (item >= 0 && item < end && ((lanes >> lane) & 1ULL))
-        backward_setup<RNG, RM>(sc, p, job, wave, lane, item, ray_colors, dLdC, target, loss_kind, st, b, loss);
+    const int64_t item = lane_ray < p.rays_per_wave ? wave_item(p, wave, lane_ray) : -1;
+    if (item >= 0 && item < end && ((lanes >> lane_ray) & 1ULL))
+        backward_setup<RNG, RM>(sc, p, job, wave, lane_ray, item, ray_colors, dLdC, target, loss_kind, st, b, loss);
     backward_wave<SPB, CAP, RNG, RM>(sc, p, b.active, b.ray, b.seed, sc.rgb + (size_t)b.view * sc.n, b.Cf, b.dL, L, G,
                                      lane, gr, b.view, ctr, b.rc, st.c + C_DROP);
     if (count_stats) flush_counters(ctr, st);
@@ -816,17 +847,22 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(3)))
     __shared__ IList<CAP> L;
     __shared__ GradStage G;
     const int lane = threadIdx.x;
-    const int64_t nb = p.wide ? (int64_t)*p.wide_count : 1;
-    for (int64_t i = p.wide ? blockIdx.x : 0; i < nb; i += gridDim.x) {
+    const int64_t nw = p.wide ? (int64_t)*p.wide_count : 1;
+    const int parts = p.wide ? wide_parts(p, nw) : 1;
+    while (nw > 0) {
         int64_t wave = block_item(blockIdx.x, gridDim.x);
+        int ray = lane;
         unsigned long long lanes = ~0ULL;
         if (p.wide) {
+            const int64_t i = next_wide(p, nw, parts, lane, ray);
+            if (i < 0) return;
             const int4 w = p.wide[i];
             wave = w.x;
             lanes = (unsigned long long)(unsigned int)w.y | (unsigned long long)(unsigned int)w.z << 32;
         }
-        backward_items<SPB, CAP, RNG, RM>(sc, p, job, wave, num_items, lanes, L, G, lane, ray_colors, dLdC, target,
+        backward_items<SPB, CAP, RNG, RM>(sc, p, job, wave, num_items, lanes, L, G, lane, ray, ray_colors, dLdC, target,
                                           loss_kind, count_stats, gr, st);
+        if (!p.wide) return;
     }
 }
 
@@ -842,7 +878,7 @@ k_forward_pq(DevScene sc, DevParams p, RayJob job, int64_t num_items, float* __r
     unsigned int spent = 0u;
     while (take_chunk(p, num_items, blockIdx.x & 7, lo, hi, spent))
         for (int64_t base = lo; base < hi; base += kWave)  // counters are flushed per tile
-            forward_items<SPB, CAP, RNG, RM>(sc, p, job, base / kWave, hi, L, lane, out_rgb, out_depth, out_opac, st);
+            forward_items<SPB, CAP, RNG, RM>(sc, p, job, base / kWave, hi, L, lane, lane, out_rgb, out_depth, out_opac, st);
 }
 
 // Persistent forward that refills idle lanes (refill_lanes = k, 0 < k < 64): as soon as k lanes
@@ -945,7 +981,7 @@ k_backward_pq(DevScene sc, DevParams p, RayJob job, int64_t num_items, const flo
     unsigned int spent = 0u;
     while (take_chunk(p, num_items, xcd, lo, hi, spent))
         for (int64_t base = lo; base < hi; base += kWave)  // counters are flushed per tile
-            backward_items<SPB, CAP, RNG, RM>(sc, p, job, base / kWave, hi, ~0ULL, L, G, lane, ray_colors, dLdC, target,
+            backward_items<SPB, CAP, RNG, RM>(sc, p, job, base / kWave, hi, ~0ULL, L, G, lane, lane, ray_colors, dLdC, target,
                                               loss_kind, count_stats, gr, st);
 }
 
@@ -1116,7 +1152,7 @@ static void launch_persistent(K kernel, int64_t items, const DevParams& p, hipSt
 // Blocks of a stepper launch: one per wavefront, or as many as take the tile kernel's leftovers in
 // turn (their number is known on the device alone; none is the common case).
 static unsigned int step_blocks(const DevParams& p, int64_t items) {
-    const int64_t nb = num_waves(p, items);
+    const int64_t nb = num_waves(p, items) * (p.wide ? (p.rays_per_wave + 3) / 4 : 1);
     return (unsigned int)(p.wide ? (nb < kWideBlocks ? nb : kWideBlocks) : ((nb + 7) / 8) * 8);
 }
 

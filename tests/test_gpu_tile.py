@@ -171,3 +171,35 @@ def test_samples_across_lanes(gpu_device, spb, rnd):
                               white_background=True)
     st = _compare(sc, prm, [_view(29, 19)], gpu_device, np.zeros(551), np.arange(551), 512)
     assert st["slab_hits"] > 0
+
+
+def _blocks(size, block, groups, seed):
+    """Rays in groups of 64, random pixels of a block each, of a view size x size."""
+    rng = np.random.default_rng(seed)
+    x, y = (rng.integers(0, size - block + 1, groups)[:, None] + rng.integers(0, block, (groups, 64)) for _ in range(2))
+    return (y * size + x).reshape(-1)
+
+
+@pytest.mark.parametrize("words", [0, 512])
+@pytest.mark.parametrize("block,groups", [(96, 600), (256, 600), (512, 600), (256, 3200), (512, 3200)])
+def test_random_rays_of_blocks(gpu_device, block, groups, words):
+    """Wavefronts of 16 and 64 random rays of wide blocks beside ordinary tiles: some are beams, the others
+    are left to the stepper in parts; where many are left, beams are held to half the width."""
+    sc = scenes.scene_uniform(3000, seed=block)
+    prm = scenes.RenderParams(dt=0.02, t_eps=1e-4, white_background=True)
+    px = np.concatenate([_blocks(1024, block, groups, 1), tile_order_pixels(1024, 1024)[: 64 * 100]])
+    st = _compare(sc, prm, [_view(1024, 1024)], gpu_device, np.zeros(len(px)), px, words)
+    assert st["slab_hits"] > 0
+
+
+@pytest.mark.parametrize("words", [0, 64, 4096])
+def test_wide_beams_in_dense_stretches(gpu_device, words):
+    """Wide beams whose rounds hold more candidates than the list: they are walked, and the rounds after
+    them too, a growing number before the next gather."""
+    sc = scenes.scene_uniform(1200, seed=5, log_scale_mean=-1.2)
+    sc.densities[:] = 0.11 + 0.002 * np.arange(1200, dtype=np.float32) / 1200
+    sc.scales[:] *= 3.0
+    prm = scenes.RenderParams(dt=0.02, t_eps=1e-4)
+    px = _blocks(128, 16, 4, 2)
+    st = _compare(sc, prm, [_view(128, 128)], gpu_device, np.zeros(len(px)), px, words)
+    assert st["fallback_slabs"] > 0 and st["slab_hits"] > 300 * 256
