@@ -1039,12 +1039,12 @@ void launch_order(const DevScene& sc, const DevParams& p, const RayJob& job, boo
                        p.rays_per_wave / split_rays(p), slots, p.order_grid, records ? 0 : views * kGrid * kGrid);
 }
 
-// Specialised on SPB (8 or 16 samples per slab), on whether the random generator is used and on the
+// Specialised on SPB (8 samples per slab, or any number up to 16), on whether the random generator is used and on the
 // record mode.
 #define RG_TILE_DISPATCH(RMV, RMON, KERNEL, ...)                                                       \
     do {                                                                                               \
         const bool rng = p.jitter || p.rnd_sample;                                                     \
-        if (p.spb <= 8) {                                                                              \
+        if (p.spb == 8) {                                                                              \
             if (rng) launch_tiles(RMV ? KERNEL<8, true, RMON> : KERNEL<8, true, 0>, __VA_ARGS__);      \
             else launch_tiles(RMV ? KERNEL<8, false, RMON> : KERNEL<8, false, 0>, __VA_ARGS__);        \
         } else {                                                                                       \

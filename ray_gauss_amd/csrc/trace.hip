@@ -1071,7 +1071,7 @@ __global__ void k_loss_out(const unsigned long long* c, float* out) {
         else if (CAPV <= 16) hipLaunchKernelGGL((KERNEL<SPBC, 16, RNGC, RMC>), __VA_ARGS__);                         \
         else hipLaunchKernelGGL((KERNEL<SPBC, 32, RNGC, RMC>), __VA_ARGS__);                                         \
     } while (0)
-// Kernels are specialised on SPB (8 or 16 samples per slab), the list capacity, on whether the
+// Kernels are specialised on SPB (8 samples per slab, or any number up to 16), the list capacity, on whether the
 // random generator is used at all (jitter or rnd_sample), which costs registers, and on the
 // hit-list record mode (RMV: 0 none, or the kernel's recording / replaying mode), so that kernels
 // without records carry none of their code.
@@ -1162,16 +1162,16 @@ hipError_t launch_forward_steps(const DevScene& sc, const DevParams& p, const Ra
     if (items <= 0) return hipSuccess;
     const bool rng = p.jitter || p.rnd_sample;
     if (p.ray_chunk > 0 && !p.wide && p.refill_lanes > 0 && p.refill_lanes < kWave) {
-        RG_DISPATCH_ANY(RG_PQ_CAP6, p.spb <= 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 1, 1, k_forward_refill, items, p,
+        RG_DISPATCH_ANY(RG_PQ_CAP6, p.spb == 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 1, 1, k_forward_refill, items, p,
                         s, sc, p, job, items, out_rgb, out_depth, out_opacity, st);
         return hipGetLastError();
     }
     if (p.ray_chunk > 0 && !p.wide) {
-        RG_DISPATCH_ANY(RG_PQ_CAP6, p.spb <= 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 1, 1, k_forward_pq, items, p, s,
+        RG_DISPATCH_ANY(RG_PQ_CAP6, p.spb == 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 1, 1, k_forward_pq, items, p, s,
                         sc, p, job, items, out_rgb, out_depth, out_opacity, st);
         return hipGetLastError();
     }
-    RG_DISPATCH_FWD(p.spb <= 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 1, k_forward, dim3(step_blocks(p, items)), dim3(kWave),
+    RG_DISPATCH_FWD(p.spb == 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 1, k_forward, dim3(step_blocks(p, items)), dim3(kWave),
                     0, s, sc, p, job, items, out_rgb, out_depth, out_opacity, st);
     return hipGetLastError();
 }
@@ -1183,11 +1183,11 @@ hipError_t launch_backward_steps(const DevScene& sc, const DevParams& p, const R
     if (items <= 0) return hipSuccess;
     const bool rng = p.jitter || p.rnd_sample;
     if (p.ray_chunk > 0 && !p.wide) {
-        RG_DISPATCH_ANY(RG_PQ_CAP, p.spb <= 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 2, 2, k_backward_pq, items, p, s,
+        RG_DISPATCH_ANY(RG_PQ_CAP, p.spb == 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 2, 2, k_backward_pq, items, p, s,
                         sc, p, job, items, ray_colors, dLdC, target, loss_kind, count_stats, gr, st);
         return hipGetLastError();
     }
-    RG_DISPATCH(p.spb <= 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 2, k_backward, dim3(step_blocks(p, items)), dim3(kWave), 0, s,
+    RG_DISPATCH(p.spb == 8 ? 8 : 16, hit_depth, rng, p.rec_mode == 2, k_backward, dim3(step_blocks(p, items)), dim3(kWave), 0, s,
                 sc, p, job, items, ray_colors, dLdC, target, loss_kind, count_stats, gr, st);
     return hipGetLastError();
 }

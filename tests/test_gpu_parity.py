@@ -196,3 +196,28 @@ def test_random_sampling_parity(gpu_device, jitter, rnd):
     for k in ("positions", "scales", "quats", "densities", "sh"):
         e = max_rel(g[k].cpu().numpy(), og[k])
         assert e <= GRAD_TOL, (k, e, rel_err(g[k].cpu().numpy(), og[k]))
+
+
+@pytest.mark.parametrize("rnd", [0, 1])
+@pytest.mark.parametrize("spb", [1, 3, 5, 7, 11, 16])
+@pytest.mark.parametrize("packet", [True, False])
+def test_samples_per_slab_parity(gpu_device, packet, spb, rnd):
+    """Slabs of other than eight samples: each slab composites its own samples and no more, in the tiles
+    and in the slab stepper, images and gradients against the oracle."""
+    sc = scenes.scene_uniform(1500, seed=spb)
+    prm = scenes.RenderParams(dt=0.02, samples_per_slab=spb, t_eps=1e-4, jitter=rnd, rnd_sample=rnd, iteration=5)
+    cam = scenes.workload("small4k").cameras[0].launch_record()
+    px = torch.arange(0, 4096, 7, dtype=torch.int32)
+    rc, _ = prepared_caster(sc, prm, [cam], gpu_device, TuneConfig(packet=packet))
+    rgb, _, _ = rc.forward(0, px)
+    tok = rc.last_token
+    ref, ok, rec = check_image(rc, sc, prm, cam, rgb, px.numpy())
+    target = np.random.default_rng(1).uniform(0, 1, rgb.shape)
+    dL = 2.0 * (rgb.cpu().numpy().astype(np.float64) - target) * ok[:, None]
+    rc.backward(0, px, rgb, torch.from_numpy(dL.astype(np.float32)).cuda(), tok)
+    g = rc.finish_grads()
+    box = gpu_box(rc)
+    og = O.full_backward(prm, sc, cam["eye"], box[0], box[1], cam, rgb.cpu().numpy().astype(np.float64), dL,
+                         pixels=px.numpy(), record=rec)
+    for k in ("positions", "scales", "quats", "densities", "sh"):
+        assert max_rel(g[k].cpu().numpy(), og[k]) <= GRAD_TOL, k
