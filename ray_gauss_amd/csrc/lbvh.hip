@@ -486,7 +486,7 @@ __global__ void k_check(int n, const float4* __restrict__ nodes, const int* __re
         }
     } else {
         const int a = p + 1, b = right[p];
-        if (a >= total || b <= a || b >= total) {
+        if (a >= total || b <= a || b >= total || leaf != ~b) {  // (gathers descend by the node's own link)
             e++;
         } else {
             const float4 alo = nodes[2 * a], ahi = nodes[2 * a + 1], blo = nodes[2 * b], bhi = nodes[2 * b + 1];
