@@ -177,7 +177,6 @@ int ensure_gaussian_capacity(rg_handle* h, int64_t n) {
     if ((rc = dalloc(h, &b.perm, cap))) return rc;
     if ((rc = dalloc(h, &b.iperm, cap))) return rc;
     if ((rc = dalloc(h, &b.nodes, 2 * total))) return rc;
-    if ((rc = dalloc(h, &b.parent, total))) return rc;
     if ((rc = dalloc(h, &b.right, total))) return rc;
     if ((rc = dalloc(h, &b.counter, total))) return rc;
     if ((rc = dalloc(h, &b.leaf_node, cap))) return rc;
@@ -338,7 +337,7 @@ int rg_destroy(rg_handle* h) {
     if (!h) return RG_OK;
     void* ptrs[] = {h->geo, h->brec, h->leafbox, h->acc, h->box, h->counters, h->queue, h->bvh.keys[0], h->bvh.keys[1],
                     h->bvh.vals[0], h->bvh.vals[1], h->bvh.hist, h->bvh.perm, h->bvh.iperm, h->bvh.nodes,
-                    h->bvh.parent, h->bvh.right, h->bvh.counter, h->bvh.leaf_node, h->bvh.k_parent,
+                    h->bvh.right, h->bvh.counter, h->bvh.leaf_node, h->bvh.k_parent,
                     h->bvh.k_left, h->bvh.k_right, h->bvh.k_first, h->bvh.k_last, h->cams, h->rgb, h->drgb,
                     h->train_rgb, h->rec, h->rec_len, h->rec_id, h->wide, h->order, h->order_bucket, h->order_grid, h->bvh.sah_prims[0], h->bvh.sah_prims[1],
                     h->bvh.sah_tasks[0], h->bvh.sah_tasks[1], h->bvh.sah_ctr, h->bvh.k_pre};

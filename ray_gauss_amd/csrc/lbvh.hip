@@ -250,7 +250,7 @@ __global__ void k_karras(int n, const unsigned long long* __restrict__ keys, int
 
 // DFS preorder renumbering + threaded links.
 __global__ void k_preorder(int n, const int* __restrict__ kl, const int* __restrict__ kf, const int* __restrict__ kla,
-                           const int* __restrict__ kpar, float4* nodes, int* parent, int* right, int* leaf_node,
+                           const int* __restrict__ kpar, float4* nodes, int* right, int* leaf_node,
                            int* kpre) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
     const int total = 2 * n - 1;
@@ -284,13 +284,8 @@ __global__ void k_preorder(int n, const int* __restrict__ kl, const int* __restr
     nodes[2 * pre].w = __int_as_float(miss);
     if (!internal) nodes[2 * pre + 1].w = __int_as_float(leafk);
     const int p = kpar[x];
-    if (p < 0) {
-        parent[pre] = -1;
-    } else if (x_is_left) {
-        parent[pre] = pre - 1;
-    } else {
+    if (p >= 0 && !x_is_left) {
         const int ppre = 2 * kf[p] + lt;  // right edge adds no left turn
-        parent[pre] = ppre;
         right[ppre] = pre;
         nodes[2 * ppre + 1].w = __int_as_float(~pre);
     }
@@ -559,7 +554,7 @@ hipError_t launch_lbvh_finish(int n, const int* sorted_vals, BvhBuffers& b, hipS
     const int total = 2 * n - 1;
     hipLaunchKernelGGL(k_set_perm, dim3(blocks(n, 256)), dim3(256), 0, s, n, sorted_vals, b.perm, b.iperm);
     hipLaunchKernelGGL(k_preorder, dim3(blocks(total, 256)), dim3(256), 0, s, n, b.k_left, b.k_first, b.k_last,
-                       b.k_parent, b.nodes, b.parent, b.right, b.leaf_node, b.k_pre);
+                       b.k_parent, b.nodes, b.right, b.leaf_node, b.k_pre);
     return hipGetLastError();
 }
 

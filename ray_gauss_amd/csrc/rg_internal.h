@@ -132,7 +132,6 @@ struct BvhBuffers {
     int* perm;
     int* iperm;
     float4* nodes;
-    int* parent;            // preorder
     int* right;             // preorder
     int* counter;           // refit flags
     int* leaf_node;         // slot -> preorder index of its leaf
