@@ -180,9 +180,11 @@ def autotune(caster: RayCaster, ray_view, ray_pixel, target, axes: dict | None =
     backward over the batch): starting from the caster's current TuneConfig, each axis in turn is
     swept with the others held at the best values so far, `passes` times over all axes; each
     configuration is run once untimed, then timed `reps` times with HIP events (the minimum
-    counts).  Returns (best TuneConfig, table of (config fields, ms)) and leaves the caster on the
+    counts).  Of the default axes the chunks of persistent launches are left out where the best
+    configuration so far goes through the tile kernels, which do not use them.  Returns (best TuneConfig, table of (config fields, ms)) and leaves the caster on the
     best configuration."""
-    axes = TUNE_AXES if axes is None else axes
+    default = axes is None
+    axes = TUNE_AXES if default else axes
     table, seen = [], {}
     loss = torch.zeros(1, dtype=torch.float32, device=ray_view.device)
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -210,6 +212,9 @@ def autotune(caster: RayCaster, ray_view, ray_pixel, target, axes: dict | None =
     best_ms = timed(best)
     for _ in range(passes):
         for field, values in axes.items():
+            tiles = best.packet and caster.params.t_near >= 0 and not (best.ray_chunk and best.refill_lanes)
+            if default and tiles and field in ("ray_chunk", "bwd_ray_chunk"):
+                continue
             for v in values:
                 cfg = dataclasses.replace(best, **{field: v})
                 ms = timed(cfg)

@@ -9,7 +9,7 @@ import torch
 
 from oracle import oracle as O
 from ray_gauss_amd import scenes
-from ray_gauss_amd.batch import BatchedTrainer, autotune, make_ray_batch
+from ray_gauss_amd.batch import TUNE_AXES, BatchedTrainer, autotune, make_ray_batch
 from ray_gauss_amd.cameras import look_at_camera, orbit_eye
 from ray_gauss_amd.caster import TuneConfig
 
@@ -396,3 +396,25 @@ def test_forward_and_backward_agree_on_tiles(gpu_device, w, h):
                 assert abs(float(loss) - ref[2]) <= 1e-5 * ref[2], (chunk, refill, bchunk)
                 for k, v in ref[1].items():
                     assert max_rel(g[k], v) <= 1e-5 and max_rel(gt[k], v) <= 1e-5, (chunk, refill, bchunk, k)
+
+
+@pytest.mark.parametrize("packet", [True, False])
+def test_autotune_sweeps_what_acts(blobs, packet):
+    """Of the default axes the persistent launches' chunks are swept where the slab stepper takes the
+    rays, and left as they are where tiles do."""
+    sc, prm, cams, pixels, rc, t, rv, rp, offs = blobs
+    target = torch.zeros((rv.shape[0], 3), device=rv.device)
+    axes = {k: v for k, v in TUNE_AXES.items() if k != "packet"}
+    rc.set_tune(TuneConfig(packet=packet))
+    try:
+        saved = dict(TUNE_AXES)
+        TUNE_AXES.clear()
+        TUNE_AXES.update(axes)
+        cfg, table = autotune(rc, rv, rp, target, reps=1, save=False)
+    finally:
+        TUNE_AXES.clear()
+        TUNE_AXES.update(saved)
+        rc.set_tune(TuneConfig())
+    chunks = {(c["ray_chunk"], c["bwd_ray_chunk"]) for c, _ in table}
+    assert chunks == {(64, 0)} if packet else len(chunks) == 4
+    assert {c["hit_depth"] for c, _ in table} == {8, 16, 32}
