@@ -418,3 +418,35 @@ def test_autotune_sweeps_what_acts(blobs, packet):
     chunks = {(c["ray_chunk"], c["bwd_ray_chunk"]) for c, _ in table}
     assert chunks == {(64, 0)} if packet else len(chunks) == 4
     assert {c["hit_depth"] for c, _ in table} == {8, 16, 32}
+
+
+@pytest.mark.parametrize("chunk", [64, 128, 256])
+@pytest.mark.parametrize("packet,t_near", [(False, 0.0), (True, -0.5)])
+def test_persistent_stepper_equals_grid_launch(blobs, gpu_device, packet, t_near, chunk):
+    """The slab stepper's persistent kernels without refilled lanes (per-lane walks, and packet walks of
+    rays that begin behind the eye, which no beam takes) against its grid launch: bit-identical images,
+    the same gathers and records, gradients equal up to the order of atomic sums."""
+    sc, prm, cams, pixels, rc0, t0, rv, rp, offs = blobs
+    prm = scenes.RenderParams(**{**prm.__dict__, "t_near": t_near})
+    gen = torch.Generator(device=gpu_device).manual_seed(7)
+    target = torch.rand((rv.shape[0], 3), generator=gen, device=gpu_device)
+    res = {}
+    for ch in (0, chunk):
+        rc, _ = prepared_caster(sc, prm, cams, gpu_device, TuneConfig(packet=packet, ray_chunk=ch, bwd_ray_chunk=ch))
+        rgb, depth, opac = rc.forward_batch(rv, rp, depth=True, opacity=True)
+        st = rc.stats()
+        rc.backward_batch(rv, rp, rgb, 2.0 * (rgb - target), rc.last_token)
+        assert rc.stats()["dropped"] == 0
+        g = {k: v.cpu().numpy() for k, v in rc.finish_grads().items() if v is not None}
+        loss = torch.zeros(1, device=gpu_device)
+        rc.train_batch(rv, rp, target, 0, None, loss)
+        gt = {k: v.cpu().numpy() for k, v in rc.finish_grads().items() if v is not None}
+        res[ch] = (rgb, depth, opac, st, g, gt, float(loss))
+    a, b = res[0], res[chunk]
+    for i in range(3):
+        assert torch.equal(a[i], b[i]), i
+    for k in ("slab_hits", "pairs", "gathers", "replay_words"):
+        assert a[3][k] == b[3][k], k
+    assert abs(a[6] - b[6]) <= 1e-6 * abs(a[6])
+    for k, v in a[4].items():
+        assert max_rel(b[4][k], v) <= 1e-5 and max_rel(b[5][k], a[5][k]) <= 1e-5, k
