@@ -49,9 +49,10 @@ typedef struct rg_config {
     int32_t max_hits_per_slab; /* >0: count slabs whose hit set exceeds it (max_prim_slice)      */
     int32_t packet_traversal;  /* 1: wavefronts of narrow beams march as one (tiles), in others the
                                   lanes walk the LBVH together (one node sequence, per-lane box
-                                  tests); 0: per-lane walks.  hit_depth, fwd_hit_depth, ray_chunk,
-                                  refill_lanes, bwd_ray_chunk and bwd_window are settings of the
-                                  wavefronts that are not tiles                                   */
+                                  tests); 0: per-lane walks.  hit_depth, fwd_hit_depth and bwd_window
+                                  are settings of the wavefronts that are not tiles, ray_chunk and
+                                  bwd_ray_chunk of jobs without any (packet_traversal 0, t_near < 0,
+                                  or ray_chunk and refill_lanes > 0)                               */
     int32_t jitter;            /* RenderOptixSettings.jitter: sub-pixel jitter (gaussians_aabb.cu:409) */
     int32_t rnd_sample;        /* RenderOptixSettings.rnd_sample: 0 grid, 1 random, 2 mid-sample     */
     uint32_t iteration;        /* RenderOptixSettings.iteration: seeds tea<4>(iteration, pixel)       */

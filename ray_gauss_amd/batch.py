@@ -181,8 +181,8 @@ def autotune(caster: RayCaster, ray_view, ray_pixel, target, axes: dict | None =
     swept with the others held at the best values so far, `passes` times over all axes; each
     configuration is run once untimed, then timed `reps` times with HIP events (the minimum
     counts).  Of the default axes the chunks of persistent launches are left out where the best
-    configuration so far goes through the tile kernels, which do not use them.  Returns (best TuneConfig, table of (config fields, ms)) and leaves the caster on the
-    best configuration."""
+    configuration so far goes through the tile kernels, which do not use them.  Returns (best
+    TuneConfig, table of (config fields, ms)) and leaves the caster on the best configuration."""
     default = axes is None
     axes = TUNE_AXES if default else axes
     table, seen = [], {}

@@ -23,9 +23,10 @@ class TuneConfig:
     """Launch tuning.  Wavefronts whose rays form narrow beams (tiles of a view) march as one and use
     seg_slabs (their first gathered range), replay_words, tree_builder and fwd_jump; the other fields are
     settings of the per-ray slab stepper, which takes all other rays (all of them with packet off, or with
-    ray_chunk and refill_lanes set), and the figures below are its.  Interval-list depth per ray, initial slabs per gather, whether a wavefront's
-    lanes walk the LBVH as one packet, the forward kernel's own (smaller) list depth, and the
-    words per ray in which a forward records its hit lists for the backward over the same rays
+    ray_chunk and refill_lanes set; ray_chunk, refill_lanes and bwd_ray_chunk act only there), and the
+    figures below are its.  Interval-list depth per ray, initial slabs per gather, whether a
+    wavefront's lanes walk the LBVH as one packet, the forward kernel's own (smaller) list depth, and
+    the words per ray in which a forward records its hit lists for the backward over the same rays
     (0: the backward walks the tree again; 1536 words = 6 KB of device memory per ray, of which a tile
     uses its share for its rays' common events), and the
     tree built at a rebuild: 0, the LBVH in Morton order (about 1 ms at 1M Gaussians with the

@@ -339,7 +339,8 @@ int rg_destroy(rg_handle* h) {
                     h->bvh.vals[0], h->bvh.vals[1], h->bvh.hist, h->bvh.perm, h->bvh.iperm, h->bvh.nodes,
                     h->bvh.right, h->bvh.counter, h->bvh.leaf_node, h->bvh.k_parent,
                     h->bvh.k_left, h->bvh.k_right, h->bvh.k_first, h->bvh.k_last, h->cams, h->rgb, h->drgb,
-                    h->train_rgb, h->rec, h->rec_len, h->rec_id, h->wide, h->order, h->order_bucket, h->order_grid, h->bvh.sah_prims[0], h->bvh.sah_prims[1],
+                    h->train_rgb, h->rec, h->rec_len, h->rec_id, h->wide, h->order, h->order_bucket,
+                    h->order_grid, h->bvh.sah_prims[0], h->bvh.sah_prims[1],
                     h->bvh.sah_tasks[0], h->bvh.sah_tasks[1], h->bvh.sah_ctr, h->bvh.k_pre};
     for (void* p : ptrs)
         if (p) hipFree(p);

@@ -13,8 +13,9 @@
 // times, and its time goes to the predicate of its candidates, the 8 samples of 1220 events (35 lanes
 // hit on average) and the gathers.  Forward 224 -> 119.7 ms, and backward 204 -> 167 ms from the events it
 // leaves; with the candidates' terms in the list, the shorter roots and the tighter beams 99.2 ms; with
-// leaves tested 64 at a time, ranges that shrink while they are gathered and rounds of several lists 87.9.  With cheaper rounds and merged
-// gradient records 83.7 and 134.7 ms: 477k and 660k vector instructions a tile, one every 3.4 and 3.9 cycles.
+// leaves tested 64 at a time, ranges that shrink while they are gathered and rounds of several lists 87.9.
+// With cheaper rounds and merged gradient records 83.7 and 134.7 ms: 477k and 660k vector instructions a
+// tile, one every 3.4 and 3.9 cycles.
 #pragma once
 
 #include "rg_device.h"

@@ -400,8 +400,8 @@ static_assert(sizeof(KeptSpread) <= sizeof(KeptEvents) && sizeof(TileLds) <= siz
 // of events -- a Gaussian and the lanes that hit it in their slab of the round -- which it goes
 // through twice: to recompute the slabs' sample buffers and from them the per-sample coefficients,
 // and to sum each Gaussian's gradient moments over its lanes.  The events come from the forward's
-// record of the tile (cells; lanes take part with their beam in it, tile, -1: none), and for the lanes with walk, once it ends, from the
-// tile's own gathers.
+// record of the tile (cells; lanes take part with their beam in it, tile, -1: none), and for the lanes with
+// walk, once it ends, from the tile's own gathers.
 template <int SPB, bool RNG, bool SPREAD>
 __device__ __forceinline__ void backward_tile(const DevScene& sc, const DevParams& p, const rg_camera* cams, bool act, const Ray& ray,
                                               unsigned int seed, int view, const float* Cfwd, const float* dL,
